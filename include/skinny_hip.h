@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define SKINNY_ABI_VERSION 19
+#define SKINNY_ABI_VERSION 20
 
 /* Error codes. */
 #define SKINNY_OK 0
@@ -103,6 +103,15 @@ typedef struct skinny_qmm_tile {
 int skinny_qmm_w4g64_bf16(const uint16_t* x, int M, int K, int ldx,
                           const uint32_t* w_frag, int N, uint16_t* y, int ldy,
                           const skinny_qmm_tile* tile, void* stream);
+
+/* The product for many rows (prompts; M >= 1, meant for more than 16), each weight read once per block
+ * of rows. K is cut as the 1..16-row entry points cut it: `splits` splits of `groups` groups (a WAVE_X
+ * tile's waves; 1 for SLAB_X), the group sums added in order within a split, the splits in order, so
+ * every row is bitwise what those entry points give for it with that tile. epilogue 0: y [M, N];
+ * 1: a gate|up weight (N = 2F), y [M, N] = [gate | up]; 2: the same weight, y [M, N/2] = silu(gate) * up.
+ * Needs K/128 >= splits * groups, ldx % 8 == 0, x and w_frag 16-byte aligned. */
+int skinny_qmm_w4g64_rows_bf16(const uint16_t* x, int M, int K, int ldx, const uint32_t* w_frag, int N,
+                               uint16_t* y, int ldy, int splits, int groups, int epilogue, void* stream);
 
 /* Tile the table picks for (K, N). Keyed by (K, N) only. */
 int skinny_qmm_pick_tile(int K, int N, skinny_qmm_tile* tile);

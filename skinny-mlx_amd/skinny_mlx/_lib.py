@@ -22,7 +22,7 @@ LIB_NAME = "libskinny_hip.so"
 # SKINNY_HIP_LIB names another build of the same library (the host-only sanitizer build the CPU
 # tests load); unset, the in-tree build next to this file.
 LIB_PATH = os.environ.get("SKINNY_HIP_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 _c_void_p = ctypes.c_void_p
 _c_int = ctypes.c_int
@@ -66,6 +66,9 @@ SIGNATURES: dict[str, tuple] = {
         _c_int,
         [_c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _tile_p, _c_void_p],
     ),
+    "skinny_qmm_w4g64_rows_bf16": (
+        _c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
+                 _c_void_p]),
     "skinny_qmm_pick_tile": (_c_int, [_c_int, _c_int, _tile_p]),
     "skinny_qmm_w4g64_glu_bf16": (
         _c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _tile_p, _c_void_p]),

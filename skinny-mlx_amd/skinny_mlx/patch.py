@@ -8,7 +8,7 @@ Call surface kept from the reference module (skinny_mlx/patch.py:22-115): `SKINN
 How it works here:
 
 * Routing by token count. A call with M tokens in SKINNY_RANGE runs the skinny kernel on the
-  weights packed at patch time; M > 16 runs as 16-row pieces when 16 is in the range; anything
+  weights packed at patch time; M > 16 runs with the bits of 16-row pieces when 16 is in the range; anything
   else keeps the unpatched semantics (fp32 dequantise + GEMM, what mx.quantized_matmul computes
   for the reference outside its range, patch.py:30-35). The default range is 1..16 rather than
   the reference's 6..16: the skinny kernel is the only path whose output for a token does not
@@ -56,7 +56,7 @@ _GATE_UP = ("gate_proj", "up_proj")
 
 
 def _skinny_ok(m: int) -> bool:
-    """Whether an M-token call takes the skinny kernel (M > 16 runs as 16-row pieces)."""
+    """Whether an M-token call takes the skinny kernel (M > 16 runs with the bits of 16-row pieces)."""
     lo, hi = SKINNY_RANGE
     return lo <= m <= hi or (m > MAX_M and lo <= MAX_M <= hi)
 

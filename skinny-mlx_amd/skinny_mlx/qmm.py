@@ -24,7 +24,8 @@ Differences from the reference, by design:
   * bf16 activations go straight into the MFMA (the reference casts to fp16, qmm.py:136);
   * the tile depends on (K, N) only, never on M (the reference's RF/SK change with M,
     qmm.py:123), so each token's output is bitwise identical for every M = 1..16;
-  * M > 16 runs in 16-row chunks (the reference hands M outside 6..16 to mx.quantized_matmul).
+  * M > 16 runs in 16-row chunks, or from a few chunks on in one launch with the same bits
+    (skinny_qmm_w4g64_rows_bf16; the reference hands M outside 6..16 to mx.quantized_matmul).
 """
 
 from __future__ import annotations
@@ -265,6 +266,9 @@ def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = N
     L = _lib.lib()
     stream = _lib.stream_of(x2)
     splits, tile = _plain_config(k, n)
+    if m >= rows_from(n, splits) and not CONFIG_OVERRIDE and not SPLITK_OVERRIDE:
+        _rows(x2, w, y, splits, tile, EPI_PLAIN, "skinny_qmm")
+        return y.reshape(*lead, n)
     if splits > 1:
         ws = splitk_workspace(x2.device, n, splits, stream)
         for m0 in range(0, m, MAX_M):
@@ -281,6 +285,39 @@ def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = N
         _lib.check(L.skinny_qmm_w4g64_bf16(xc.data_ptr(), mc, k, x2.stride(0), w.data_ptr(), n, yc.data_ptr(),
                                            y.stride(0), ctypes.byref(tile), stream), "skinny_qmm")
     return y.reshape(*lead, n)
+
+
+# The many-row kernel (skinny_qmm_w4g64_rows_bf16): epilogues, and the rows one launch takes.
+EPI_PLAIN, EPI_GLU_SPLIT, EPI_SWIGLU = 0, 1, 2
+_ROWS_MAX = 16384
+_ROWS_WIDE_N = 8192
+_ROWS_MAX_N = 1 << 20  # one launch's grid
+
+
+def rows_from(n: int, splits: int) -> int:
+    """Rows from which one launch of the many-row kernel replaces the 16-row pieces (same bits).
+    Measured on MI355X in us, pieces against one launch: a weight of many row tiles from two pieces
+    on (2560 x 19456 gate|up, 20 rows: 24 / 15), others from three (4096 x 2560, 33 rows: 18 / 16; 32
+    rows: 12 / 15), a split-K shape, whose pieces spread K over the whole GPU, from five (9728 x
+    2560, 64 rows: 33 / 34; 77 rows: 41 / 36)."""
+    if n > _ROWS_MAX_N:
+        return 1 << 62
+    if splits > 1:
+        return 4 * MAX_M + 1
+    return MAX_M + 1 if n >= _ROWS_WIDE_N else 2 * MAX_M + 1
+
+
+def _rows(x2: torch.Tensor, w: torch.Tensor, y: torch.Tensor, splits: int, tile, epilogue: int, what: str) -> None:
+    """The many-row kernel over the rows of x2 with the cut of K of (splits, tile): bitwise the
+    16-row pieces."""
+    m, k = x2.shape
+    groups = tile.waves if tile.kind == _WAVE_X else 1
+    L = _lib.lib()
+    stream = _lib.stream_of(x2)
+    for m0 in range(0, m, _ROWS_MAX):
+        _lib.check(L.skinny_qmm_w4g64_rows_bf16(x2[m0:].data_ptr(), min(_ROWS_MAX, m - m0), k, x2.stride(0), w.data_ptr(),
+                                                w.shape[0], y[m0:].data_ptr(), y.stride(0), splits, groups, epilogue,
+                                                stream), what)
 
 
 _SPLITK: dict[tuple[int, int], tuple] = {}
@@ -425,7 +462,7 @@ def skinny_qmm_partial_gated(y: torch.Tensor, z: torch.Tensor, norm_w: torch.Ten
     return PartialSum(parts)
 
 
-def _rows(x: torch.Tensor, k: int) -> torch.Tensor:
+def _step_rows(x: torch.Tensor, k: int) -> torch.Tensor:
     if x.shape[-1] != k:
         raise ValueError(f"x has K={x.shape[-1]}, weights have K={k}")
     x2 = x.reshape(-1, k)
@@ -542,7 +579,7 @@ def skinny_qmm_conv(x: torch.Tensor, w: torch.Tensor, c: int, conv_state: torch.
     overrides the library's choice."""
     k = packed_k(w)
     n = w.shape[0]
-    x2 = _rows(x, k)
+    x2 = _step_rows(x, k)
     m = x2.shape[0]
     kw = _check_conv(c, conv_state, conv_w, window, m)
     y = torch.empty((m, n), dtype=torch.bfloat16, device=x2.device)
@@ -588,7 +625,7 @@ def skinny_mlp_fused_partial(x: torch.Tensor, w_gate_up: torch.Tensor, w_down: t
     k = packed_k(w_gate_up)
     f = w_gate_up.shape[0] // 2
     n = w_down.shape[0]
-    x2 = _rows(x, k)
+    x2 = _step_rows(x, k)
     m = x2.shape[0]
     if act.dtype != torch.bfloat16 or act.shape[0] < m or act.shape[1] != f or not act.is_contiguous():
         raise ValueError(f"act must be contiguous bf16 [>= {m}, {f}]")
@@ -658,6 +695,9 @@ def skinny_glu(x: torch.Tensor, w: torch.Tensor, swiglu: bool, out: torch.Tensor
             raise ValueError(f"out must be bf16 [M, {width}] with unit inner stride")
         y = out
     tile = glu_tile(k, f)
+    if m >= rows_from(2 * f, 1):
+        _rows(x2, w, y, 1, tile, EPI_SWIGLU if swiglu else EPI_GLU_SPLIT, "skinny_glu")
+        return y.reshape(*lead, width)
     L = _lib.lib()
     stream = _lib.stream_of(x2)
     for m0 in range(0, m, MAX_M):

@@ -346,3 +346,24 @@ def test_fused_mlp_entry_point_validates_on_host():
     _expect_einval(call(f=9680), "bad shape")
     _expect_einval(call(ldx=2552), "ldx=2552")
     _expect_einval(call(sync_bytes=need - 4), "sync of")
+
+
+def test_qmm_rows_argument_validation_on_host():
+    L = _lib.lib()
+    d = ctypes.c_void_p(4096)
+
+    def call(x=d, m=64, k=2560, ldx=2560, w=d, n=2560, y=d, ldy=2560, splits=1, groups=4, epi=0):
+        return L.skinny_qmm_w4g64_rows_bf16(x, m, k, ldx, w, n, y, ldy, splits, groups, epi, None)
+
+    _expect_einval(call(x=None), "null")
+    _expect_einval(call(m=0), "M=0")
+    _expect_einval(call(k=2500), "K=2500")
+    _expect_einval(call(n=2568), "N=2568")
+    _expect_einval(call(n=2576, ldy=2576, epi=2), "multiple of 32")
+    _expect_einval(call(ldx=2552), "ldx")
+    _expect_einval(call(ldy=2544), "ldy")
+    _expect_einval(call(epi=2, ldy=1264), "ldy")
+    _expect_einval(call(epi=3), "epilogue")
+    _expect_einval(call(splits=3, groups=8), "a pair of 128 each")
+    _expect_einval(call(x=ctypes.c_void_p(4104)), "misaligned")
+    _expect_einval(call(m=1 << 24, n=1 << 20, ldy=1 << 20), "too large")
