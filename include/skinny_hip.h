@@ -338,6 +338,18 @@ int skinny_qkv_attention_fused_bf16(const uint16_t* x, int M, int K, int ldx, co
 /* 1 when skinny_qkv_attention_fused_bf16 runs for (K, N, Hkv, maxlen) on the current device, 0
  * when it does not, a negative code when the device cannot be queried. */
 int skinny_qkv_attention_supported(int K, int N, int Hkv, int maxlen);
+/* The fused attention for a prompt of M tokens (more than one step holds) after the pos0 cached ones:
+ * rows, cache entries and outputs bitwise those of skinny_attention_fused_bf16 over consecutive 16-token
+ * steps. keys = the cache length after the call (pos0[0] + M, known to the host; at most maxlen), Hq/Hkv
+ * <= 4. Needs a workspace of skinny_attn_prompt_workspace_bytes(M, Hq, Hkv, keys) bytes, 16-byte aligned (no
+ * initialisation; less makes more launches, down to four 16-token pieces' partials). */
+size_t skinny_attn_prompt_workspace_bytes(int M, int Hq, int Hkv, int keys);
+int skinny_attention_prompt_bf16(const uint16_t* qkv, int ldq, int M, int Hq, int Hkv, int D,
+                                 const uint16_t* q_norm, const uint16_t* k_norm, float eps, const float* rope_table,
+                                 int rope_positions, const int32_t* pos0, int keys, uint16_t* k_cache,
+                                 uint16_t* vt_cache, int maxlen, float scale, void* workspace,
+                                 size_t workspace_bytes, uint16_t* out, void* stream);
+
 /* skinny_attention_fused_bf16 without the workspace argument, for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc). No
  * counterpart in the reference. The chunk partials live in a file-scope device array of this
@@ -383,6 +395,15 @@ int skinny_attention_general_bf16(const uint16_t* qkv, int ldq, int M, int Hq, i
                                   int rope_positions, const int32_t* pos0, const int32_t* tree,
                                   uint16_t* k_cache, uint16_t* vt_cache, int maxlen, float scale, void* workspace,
                                   size_t workspace_bytes, uint16_t* out, void* stream);
+/* The same for a prompt of M tokens, as skinny_attention_prompt_bf16: bitwise the 16-token steps. */
+size_t skinny_attn_general_prompt_workspace_bytes(int M, int Hq, int Hkv, int D, int keys);
+int skinny_attention_general_prompt_bf16(const uint16_t* qkv, int ldq, int M, int Hq, int Hkv, int D, int q_stride,
+                                         int k_offset, int v_offset, int gate_offset, const uint16_t* q_norm,
+                                         const uint16_t* k_norm, float eps, int rotary_dim, const float* rope_table,
+                                         int rope_positions, const int32_t* pos0, int keys, uint16_t* k_cache,
+                                         uint16_t* vt_cache, int maxlen, float scale, void* workspace,
+                                         size_t workspace_bytes, uint16_t* out, void* stream);
+
 size_t skinny_attn_general_workspace_bytes(int Hq, int Hkv, int D, int maxlen);
 /* Accepted draft-tree path into the attention caches of `layers` layers (K and V^T of layer l
  * at l * layer_stride elements): with p0 = *pos - pos_back the tree's first slot, the node at

@@ -92,20 +92,19 @@ __global__ __launch_bounds__(64 * kWaves) void attn_chunk_kernel(const int32_t* 
 constexpr int kCombineBlock = 32;
 constexpr int kCombineWaves = 4;  // waves of the merge for caches of more than kCombineBlock chunks
 
-template <int W>
-__global__ __launch_bounds__(64 * W) void attn_combine_kernel(const float* __restrict__ part_o,
-                                                              const float* __restrict__ part_ml, int M, int Hq, int Hkv,
-                                                              const int32_t* __restrict__ pos0, int nchunk_max,
-                                                              uint16_t* __restrict__ out, uint32_t* __restrict__ reset,
-                                                              int reset_ld, int reset_words) {
-  const int hq = blockIdx.x, t = blockIdx.y, lane = threadIdx.x & 63, v = W > 1 ? wave_id() : 0;
-  const int G = Hq / Hkv, h = hq / G, row = t * G + hq % G;
-  const size_t head_base = (size_t)h * nchunk_max * kRowsMax + row;  // chunk c at + c * kRowsMax
+// The merge of one row (chunk c's partial at head_base + c * kRowsMax; pos0[0] + tokens keys) into
+// dst[128]; false in the waves that only helped. kPrompt reads the chunk count first, since a prompt's
+// early tokens see few of the chunk slots.
+template <int W, bool kPrompt>
+__device__ __forceinline__ bool combine_row(const float* __restrict__ part_o, const float* __restrict__ part_ml,
+                                            size_t head_base, const int32_t* __restrict__ pos0, int tokens,
+                                            int nchunk_max, uint16_t* __restrict__ dst) {
+  const int lane = threadIdx.x & 63, v = W > 1 ? wave_id() : 0;
   const int first = v * kCombineBlock;                                // this wave's first block
   // The first block's partials are loaded before the chunk count is known (it needs *pos0):
   // every chunk the workspace holds up to kCombineBlock, the ones past the context discarded below
   // by selection (their stale values never enter an arithmetic operation).
-  const int pre = max(0, min(kCombineBlock, nchunk_max - first));
+  const int pre = kPrompt ? 0 : max(0, min(kCombineBlock, nchunk_max - first));
   float mc_pre = -INFINITY, lc_pre = 0.f;
   float o0[kCombineBlock], o1[kCombineBlock];
   if (lane < pre) {
@@ -121,13 +120,14 @@ __global__ __launch_bounds__(64 * W) void attn_combine_kernel(const float* __res
       o1[j] = po[lane + 64];
     }
   }
-  const int total = pos0[0] + M;
-  const int nch = (total + kChunk - 1) / kChunk;
+  const int total = pos0[0] + tokens;
+  // (a prompt's workspace holds the chunks its caller named; no read past them whatever *pos0 says)
+  const int nch = kPrompt ? min((total + kChunk - 1) / kChunk, nchunk_max) : (total + kChunk - 1) / kChunk;
   float run_m = -INFINITY, run_l = 0.f, a0 = 0.f, a1 = 0.f;
   for (int c0 = first; c0 < nch; c0 += W * kCombineBlock) {
     const int nb = min(kCombineBlock, nch - c0);
     float mc = -INFINITY, lc = 0.f;
-    if (c0 == first) {
+    if (!kPrompt && c0 == first) {
       mc = lane < nb ? mc_pre : -INFINITY;
       lc = lane < nb ? lc_pre : 0.f;
 #pragma unroll
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(64 * W) void attn_combine_kernel(const float* __res
     sa[v][0][lane] = a0;
     sa[v][1][lane] = a1;
     __syncthreads();
-    if (v > 0) return;
+    if (v > 0) return false;
 #pragma unroll
     for (int u = 1; u < W; ++u) {
       const float mu = sm[u], lu = sl[u];
@@ -193,9 +193,21 @@ __global__ __launch_bounds__(64 * W) void attn_combine_kernel(const float* __res
     }
   }
   const float inv = run_l > 0.f ? 1.0f / run_l : 0.f;
-  uint16_t* dst = out + ((size_t)t * Hq + hq) * kD;
   dst[lane] = f32_to_bf16_bits(a0 * inv);
   dst[lane + 64] = f32_to_bf16_bits(a1 * inv);
+  return true;
+}
+
+template <int W>
+__global__ __launch_bounds__(64 * W) void attn_combine_kernel(const float* __restrict__ part_o,
+                                                              const float* __restrict__ part_ml, int M, int Hq, int Hkv,
+                                                              const int32_t* __restrict__ pos0, int nchunk_max,
+                                                              uint16_t* __restrict__ out, uint32_t* __restrict__ reset,
+                                                              int reset_ld, int reset_words) {
+  const int hq = blockIdx.x, t = blockIdx.y, lane = threadIdx.x & 63;
+  const int G = Hq / Hkv, h = hq / G, row = t * G + hq % G;
+  const size_t head_base = (size_t)h * nchunk_max * kRowsMax + row;  // chunk c at + c * kRowsMax
+  if (!combine_row<W, false>(part_o, part_ml, head_base, pos0, M, nchunk_max, out + ((size_t)t * Hq + hq) * kD)) return;
   if (reset) {  // every chunk workgroup has read the hand-off rows: back to "not yet written"
     const int per = (reset_words + Hq - 1) / Hq;
     const int w1 = min(reset_words, (hq + 1) * per);
@@ -203,6 +215,163 @@ __global__ __launch_bounds__(64 * W) void attn_combine_kernel(const float* __res
     for (int w = hq * per + lane; w < w1; w += 64)
       __hip_atomic_store(r + w, 0xffffffffu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+// --- the attention of a prompt: more tokens than one step holds ---------------------------------
+//
+// The prompt's tokens are taken in pieces of kPiece, and every row's arithmetic is that of the fused
+// step kernels over its piece (the same query and key rows, chunk partials and merge, which depend on
+// absolute key positions only), so a prompt's rows and cache entries are bitwise those of 16-token steps.
+// Three launches instead of two per piece: (1) queries into a workspace, keys and values into the
+// caches; (2) one workgroup per (kPieceGroup pieces, chunk, kv head), which stages the chunk once for all
+// of them; (3) one workgroup per (query head, token) for the merge.
+constexpr int kPiece = 16;      // tokens per piece
+constexpr int kPieceGroup = 4;  // pieces that share a staged chunk
+
+struct PromptArgs {
+  int M, Hq, Hkv;
+  const uint16_t* qn;
+  const uint16_t* kn;
+  float eps;
+  const float* rope;  // [positions][64] (cos, sin)
+  uint16_t* q_out;    // [M][Hq][128]
+  uint16_t* kc;
+  uint16_t* vt;
+  int maxlen;
+};
+
+// (1) Workgroups [0, nq): 64 query rows each, a wave per 16 (lane (col, quad) as in the chunk kernel);
+// [nq, nq + nk): a key row per wave (lanes d and d + 64); the rest: 64 tokens of one value head, turned in
+// LDS so that the stores into V^T run along the cache slots.
+__global__ __launch_bounds__(256) void prompt_qkv_kernel(const int32_t* __restrict__ pos0, const uint16_t* __restrict__ qkv,
+                                                         int ldq, int nq, int nk, const PromptArgs pa) {
+  __shared__ uint16_t vl[64][kD + 2];
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int p0 = pos0[0];
+  const int M = pa.M, Hq = pa.Hq, Hkv = pa.Hkv;
+  const int b = blockIdx.x;
+  if (b < nq) {
+    const int col = lane & 15, quad = lane >> 4;
+    const int r = b * 64 + wave * 16 + col;
+    const bool live = r < M * Hq;
+    const int t = live ? r / Hq : 0, hq = live ? r % Hq : 0;
+    const uint16_t* src = qkv + (size_t)t * ldq + (size_t)hq * kD;
+    const uint16_t* qn = pa.qn ? pa.qn : src;
+    const f32x4_t* rp = reinterpret_cast<const f32x4_t*>(pa.rope + (size_t)(p0 + t) * 128);
+    u32x4_t raw[4], wq[4];
+    f32x4_t cs[2][4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      raw[ks] = *reinterpret_cast<const u32x4_t*>(src + ks * 32 + quad * 8);
+      wq[ks] = *reinterpret_cast<const u32x4_t*>(qn + ks * 32 + quad * 8);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) cs[ks][j] = rp[(ks * 32 + quad * 8) / 2 + j];
+    bf16x8_t qf[4];
+    rotate_query(raw, wq, cs, pa.qn != nullptr, pa.eps, qf);
+    if (live) {
+      uint16_t* dst = pa.q_out + (size_t)r * kD;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) *reinterpret_cast<bf16x8_t*>(dst + ks * 32 + quad * 8) = qf[ks];
+    }
+  } else if (b < nq + nk) {
+    const int r = (b - nq) * 4 + wave;
+    if (r >= M * Hkv) return;
+    const int t = r / Hkv, h = r % Hkv, slot = p0 + t;
+    const uint16_t* src = qkv + (size_t)t * ldq + (size_t)(Hq + h) * kD;
+    float ka = bf16_bits_to_f32(src[lane]), kb = bf16_bits_to_f32(src[lane + 64]);
+    const float2 cs = reinterpret_cast<const float2*>(pa.rope)[(size_t)slot * 64 + lane];
+    if (pa.kn) {
+      const float w0 = bf16_bits_to_f32(pa.kn[lane]), w1 = bf16_bits_to_f32(pa.kn[lane + 64]);
+      const float inv = rsqrtf(wave_sum(fmaf(kb, kb, ka * ka)) / (float)kD + pa.eps);
+      ka = bf16_bits_to_f32(f32_to_bf16_bits(ka * inv * w0));
+      kb = bf16_bits_to_f32(f32_to_bf16_bits(kb * inv * w1));
+    }
+    uint16_t* dst = pa.kc + ((size_t)h * pa.maxlen + slot) * kD;
+    dst[lane] = f32_to_bf16_bits(fmaf(ka, cs.x, -(kb * cs.y)));
+    dst[lane + 64] = f32_to_bf16_bits(fmaf(kb, cs.x, ka * cs.y));
+  } else {
+    const int i = b - nq - nk, h = i % Hkv, t0 = i / Hkv * 64;
+    for (int e = threadIdx.x; e < 64 * (kD / 8); e += 256) {
+      const int t = e / (kD / 8), piece = e % (kD / 8);
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(qkv + (size_t)min(t0 + t, M - 1) * ldq + (size_t)(Hq + Hkv + h) * kD + piece * 8);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) *reinterpret_cast<uint32_t*>(&vl[t][piece * 8 + 2 * k]) = v[k];
+    }
+    __syncthreads();
+    if (t0 + lane < M)
+      for (int d = wave; d < kD; d += 4) pa.vt[((size_t)h * kD + d) * pa.maxlen + p0 + t0 + lane] = vl[lane][d];
+  }
+}
+
+// (2) Workgroup (chunk c, kv head h, group g of pieces): pieces z0 + kPieceGroup g .. of the launch's
+// pieces [z0, z1); piece z's partials at (z - z0) * Hkv * nch chunk slots.
+__global__ __launch_bounds__(64 * kWaves) void prompt_chunk_kernel(const int32_t* __restrict__ pos0,
+                                                                   const uint16_t* __restrict__ q, int M, int Hq, int Hkv,
+                                                                   const uint16_t* __restrict__ kc,
+                                                                   const uint16_t* __restrict__ vt, int maxlen, float scale,
+                                                                   int z0, int z1, int nch, float* __restrict__ part_o,
+                                                                   float* __restrict__ part_ml) {
+  __shared__ __attribute__((aligned(16))) uint16_t ks_lds[kChunk * kPitch];
+  __shared__ __attribute__((aligned(16))) uint16_t vs_lds[kD * kPitch];
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int c = blockIdx.x, h = blockIdx.y, p0 = pos0[0], G = Hq / Hkv;
+  const int za = z0 + (int)blockIdx.z * kPieceGroup, zb = min(za + kPieceGroup, z1);
+  const int key0 = c * kChunk;
+  if (key0 >= p0 + min(M, zb * kPiece)) return;  // past the last piece's keys
+  const u32x4_t* kh = reinterpret_cast<const u32x4_t*>(kc + ((size_t)h * maxlen + key0) * kD);
+  const uint16_t* vh = vt + (size_t)h * kD * maxlen + key0;
+  u32x4_t kr[8], vr[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int e = threadIdx.x + i * 64 * kWaves;  // piece e: row e / 16, column piece e % 16
+    kr[i] = kh[e];
+    vr[i] = *reinterpret_cast<const u32x4_t*>(vh + (size_t)(e >> 4) * maxlen + (e & 15) * 8);
+  }
+  const int col = lane & 15, quad = lane >> 4, qrow = wave * 16 + col;
+  bf16x8_t qf[kPieceGroup][4];
+#pragma unroll
+  for (int i = 0; i < kPieceGroup; ++i) {
+    const int t0 = (za + i) * kPiece, rows = G * min(kPiece, M - t0);
+    const bool live = za + i < zb && qrow < rows;
+    const uint16_t* qr = q + ((size_t)(live ? t0 + qrow / G : 0) * Hq + h * G + (live ? qrow % G : 0)) * kD;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      qf[i][ks] = *reinterpret_cast<const bf16x8_t*>(qr + ks * 32 + quad * 8);
+      if (!live) qf[i][ks] = bf16x8_t{};
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int e = threadIdx.x + i * 64 * kWaves;
+    *reinterpret_cast<u32x4_t*>(&ks_lds[(e >> 4) * kPitch + (e & 15) * 8]) = kr[i];
+    *reinterpret_cast<u32x4_t*>(&vs_lds[(e >> 4) * kPitch + (e & 15) * 8]) = vr[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kPieceGroup; ++i) {
+    const int z = za + i, t0 = z * kPiece;
+    if (z >= zb) break;
+    const int mb = min(kPiece, M - t0);
+    if (key0 >= p0 + t0 + mb || wave * 16 >= G * mb) continue;
+    const int tbase = qrow < G * mb ? p0 + t0 + qrow / G + 1 : key0;
+    const size_t base = (((size_t)(z - z0) * Hkv + h) * nch + c) * kRowsMax + wave * 16;
+    attn_rows(ks_lds, vs_lds, qf[i], key0, tbase, 0u, scale, part_o + base * kD, part_ml + base * 2);
+  }
+}
+
+// (3) Token t0 + blockIdx.y (t0 = kPiece z0).
+template <int W>
+__global__ __launch_bounds__(64 * W) void prompt_combine_kernel(const float* __restrict__ part_o,
+                                                                const float* __restrict__ part_ml, int M, int Hq, int Hkv,
+                                                                const int32_t* __restrict__ pos0, int z0, int nch,
+                                                                uint16_t* __restrict__ out) {
+  const int hq = blockIdx.x, t = z0 * kPiece + (int)blockIdx.y, z = t / kPiece;
+  const int G = Hq / Hkv, h = hq / G, row = (t % kPiece) * G + hq % G;
+  const size_t head_base = (((size_t)(z - z0) * Hkv + h) * nch) * kRowsMax + row;
+  combine_row<W, true>(part_o, part_ml, head_base, pos0, min(M, (z + 1) * kPiece), nch, out + ((size_t)t * Hq + hq) * kD);
 }
 
 // cos/sin table of rotate-half RoPE: table[pos][i] = (cos, sin)(pos * theta^(-2i/128)), i < 64,
@@ -325,6 +494,74 @@ extern "C" int skinny_attention_fused_bf16(const uint16_t* qkv, int ldq, int M, 
                                            void* stream) {
   return attention_fused(qkv, ldq, M, Hq, Hkv, D, q_norm, k_norm, eps, rope_table, rope_positions, pos0, tree,
                          k_cache, vt_cache, maxlen, scale, workspace, workspace_bytes, out, stream);
+}
+
+// Workspace of a prompt's attention: the rotated queries, then the partials of as many pieces as fit
+// kPromptPartBytes (at least one group of pieces).
+constexpr size_t kPromptPartBytes = (size_t)256 << 20;
+
+static size_t prompt_piece_bytes(int Hkv, int nch) { return (size_t)Hkv * nch * kRowsMax * (kD + 2) * sizeof(float); }
+
+static size_t prompt_query_bytes(int M, int Hq) { return ((size_t)M * Hq * kD * 2 + 255) & ~(size_t)255; }
+
+extern "C" size_t skinny_attn_prompt_workspace_bytes(int M, int Hq, int Hkv, int keys) {
+  if (M < 1 || Hq < 1 || Hkv < 1 || keys < 1) return 0;
+  const size_t piece = prompt_piece_bytes(Hkv, (keys + kChunk - 1) / kChunk);
+  const size_t all = (size_t)((M + kPiece - 1) / kPiece) * piece, group = kPieceGroup * piece;
+  const size_t most = kPromptPartBytes / group * group;
+  return prompt_query_bytes(M, Hq) + (all <= most ? all : most > group ? most : group < all ? group : all);
+}
+
+extern "C" int skinny_attention_prompt_bf16(const uint16_t* qkv, int ldq, int M, int Hq, int Hkv, int D,
+                                            const uint16_t* q_norm, const uint16_t* k_norm, float eps,
+                                            const float* rope_table, int rope_positions, const int32_t* pos0, int keys,
+                                            uint16_t* k_cache, uint16_t* vt_cache, int maxlen, float scale,
+                                            void* workspace, size_t workspace_bytes, uint16_t* out, void* stream) {
+  SKINNY_CHECK_ARG(qkv && rope_table && k_cache && vt_cache && pos0 && workspace && out, "attention prompt: null pointer");
+  SKINNY_CHECK_ARG(D == kD, "attention prompt: head dim %d unsupported (only %d)", D, kD);
+  SKINNY_CHECK_ARG(Hkv >= 1 && Hq % Hkv == 0 && (Hq / Hkv) * kPiece <= kRowsMax,
+                   "attention prompt: Hq=%d must be a multiple of Hkv=%d, at most %d query heads each", Hq, Hkv,
+                   kRowsMax / kPiece);
+  SKINNY_CHECK_ARG(M >= 1 && M <= 65535 && keys >= M && keys <= maxlen, "attention prompt: M=%d (at most 65535), keys=%d in [M, maxlen=%d]",
+                   M, keys, maxlen);
+  SKINNY_CHECK_ARG(ldq >= (Hq + 2 * Hkv) * D && ldq % 8 == 0, "attention prompt: ldq=%d too small or not a multiple of 8", ldq);
+  SKINNY_CHECK_ARG(maxlen >= kChunk && maxlen % kChunk == 0 && rope_positions >= maxlen,
+                   "attention prompt: maxlen=%d must be a multiple of %d and within the RoPE table (%d)", maxlen, kChunk,
+                   rope_positions);
+  SKINNY_CHECK_ARG(skinny_aligned(qkv, 16) && skinny_aligned(k_cache, 16) && skinny_aligned(vt_cache, 16) &&
+                       skinny_aligned(rope_table, 16) && (!q_norm || skinny_aligned(q_norm, 16)) && skinny_aligned(workspace, 16),
+                   "attention prompt: qkv, caches, table, q_norm and workspace must be 16-byte aligned");
+  const int nch = (keys + kChunk - 1) / kChunk, pieces = (M + kPiece - 1) / kPiece;
+  const size_t piece = prompt_piece_bytes(Hkv, nch), qbytes = prompt_query_bytes(M, Hq);
+  const size_t room = workspace_bytes > qbytes ? (workspace_bytes - qbytes) / piece : 0;
+  const int fit = room < (size_t)pieces ? (int)room / kPieceGroup * kPieceGroup : pieces;
+  SKINNY_CHECK_ARG(fit >= 1, "attention prompt: workspace of %zu bytes, needs %zu", workspace_bytes,
+                   skinny_attn_prompt_workspace_bytes(M, Hq, Hkv, keys));
+  uint16_t* q = static_cast<uint16_t*>(workspace);
+  float* part_o = reinterpret_cast<float*>(static_cast<char*>(workspace) + qbytes);
+  float* part_ml = part_o + (size_t)fit * Hkv * nch * kRowsMax * kD;
+  const hipStream_t s = (hipStream_t)stream;
+  const PromptArgs pa{M, Hq, Hkv, q_norm, k_norm, eps, rope_table, q, k_cache, vt_cache, maxlen};
+  const int nq = (M * Hq + 63) / 64, nk = (M * Hkv + 3) / 4, nv = Hkv * ((M + 63) / 64);
+  hipLaunchKernelGGL(prompt_qkv_kernel, dim3(nq + nk + nv), dim3(256), 0, s, pos0, qkv, ldq, nq, nk, pa);
+  if (int rc = skinny_check_launch("attention prompt q/k/v")) return rc;
+  for (int z0 = 0; z0 < pieces; z0 += fit) {
+    const int z1 = z0 + fit < pieces ? z0 + fit : pieces;
+    const int last = z1 * kPiece < M ? z1 * kPiece : M;             // tokens up to this launch's end
+    const int n = (keys - M + last + kChunk - 1) / kChunk;          // chunks its last piece sees
+    hipLaunchKernelGGL(prompt_chunk_kernel, dim3(n, Hkv, (z1 - z0 + kPieceGroup - 1) / kPieceGroup), dim3(64 * kWaves), 0, s,
+                       pos0, q, M, Hq, Hkv, k_cache, vt_cache, maxlen, scale, z0, z1, nch, part_o, part_ml);
+    if (int rc = skinny_check_launch("attention prompt chunks")) return rc;
+    // the wave count of the merge goes by the cache size, as in the step kernels
+    if (maxlen / kChunk > kCombineBlock)
+      hipLaunchKernelGGL(prompt_combine_kernel<kCombineWaves>, dim3(Hq, last - z0 * kPiece), dim3(64 * kCombineWaves), 0, s,
+                         part_o, part_ml, M, Hq, Hkv, pos0, z0, nch, out);
+    else
+      hipLaunchKernelGGL(prompt_combine_kernel<1>, dim3(Hq, last - z0 * kPiece), dim3(64), 0, s, part_o, part_ml, M, Hq, Hkv,
+                         pos0, z0, nch, out);
+    if (int rc = skinny_check_launch("attention prompt merge")) return rc;
+  }
+  return SKINNY_OK;
 }
 
 // --- the allocation-free form -----------------------------------------------------------------

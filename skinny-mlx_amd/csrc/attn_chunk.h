@@ -59,6 +59,133 @@ struct FusedArgs {
 constexpr int kFusedMaxTokens = 4 * kWaves;  // new tokens per step in the fused form (4 per wave)
 constexpr int kHandoffPolls = 1 << 14;       // polls (each a device-coherent round trip) before the wait form gives up
 
+// A query row's RMSNorm (the lane's 32 squares plus two shuffles across the quads) and RoPE (dims d and
+// d + 64 in the same lane), from the raw row's words at dims 32ks + 8quad + e into the B operand.
+__device__ __forceinline__ void rotate_query(const u32x4_t (&raw)[4], const u32x4_t (&wq)[4], const f32x4_t (&cs)[2][4],
+                                             bool norm, float eps, bf16x8_t (&qf)[4]) {
+  float x[4][8];
+  float ss = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      x[ks][e] = bf16_bits_to_f32((e & 1) ? (raw[ks][e >> 1] >> 16) : (raw[ks][e >> 1] & 0xffffu));
+      ss = fmaf(x[ks][e], x[ks][e], ss);
+    }
+  ss += __shfl_xor(ss, 16, 64);
+  ss += __shfl_xor(ss, 32, 64);
+  if (norm) {
+    const float inv = rsqrtf(ss / (float)kD + eps);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float wv = bf16_bits_to_f32((e & 1) ? (wq[ks][e >> 1] >> 16) : (wq[ks][e >> 1] & 0xffffu));
+        x[ks][e] = bf16_bits_to_f32(f32_to_bf16_bits(x[ks][e] * inv * wv));
+      }
+  }
+  u32x4_t lo[2], hi[2];  // rotated dims 32ks + 8quad + e (lo) and those + 64 (hi)
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int e2 = 0; e2 < 4; ++e2) {
+      uint32_t wl = 0, wh = 0;
+#pragma unroll
+      for (int bb = 0; bb < 2; ++bb) {
+        const int e = 2 * e2 + bb;
+        const float c2 = cs[ks][e >> 1][(e & 1) * 2], sn = cs[ks][e >> 1][(e & 1) * 2 + 1];
+        const float av = x[ks][e], bv = x[ks + 2][e];
+        wl |= (uint32_t)f32_to_bf16_bits(fmaf(av, c2, -(bv * sn))) << (16 * bb);
+        wh |= (uint32_t)f32_to_bf16_bits(fmaf(bv, c2, av * sn)) << (16 * bb);
+      }
+      lo[ks][e2] = wl;
+      hi[ks][e2] = wh;
+    }
+  qf[0] = __builtin_bit_cast(bf16x8_t, lo[0]);
+  qf[1] = __builtin_bit_cast(bf16x8_t, lo[1]);
+  qf[2] = __builtin_bit_cast(bf16x8_t, hi[0]);
+  qf[3] = __builtin_bit_cast(bf16x8_t, hi[1]);
+}
+
+// One wave's 16 query rows against the staged chunk (keys key0 ..): the partial O rows to rows_o
+// [16][128], the row maxima (log2 units) and sums to rows_ml [16][2]. Visibility per lane as the caller
+// set it up: key kp is visible iff kp < tbase, or kp - tbase < 32 and that bit of tmask is set.
+__device__ __forceinline__ void attn_rows(const uint16_t* ks_lds, const uint16_t* vs_lds, const bf16x8_t (&qf)[4], int key0,
+                                          int tbase, uint32_t tmask, float scale, float* __restrict__ rows_o,
+                                          float* __restrict__ rows_ml) {
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  // 2. S^T tiles: element i of tile kt is the score of key 32(kt/2) + 8quad + 4(kt%2) + i.
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  float s[8][4];
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt) {
+    const int krow = 32 * (kt >> 1) + 8 * (col >> 2) + 4 * (kt & 1) + (col & 3);
+    f32x4_t acc = zero;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      acc = mfma16x16x32(*reinterpret_cast<const bf16x8_t*>(&ks_lds[krow * kPitch + ks * 32 + quad * 8]), qf[ks], acc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
+  }
+
+  // 3. Visibility, the row maximum (log2 units), bf16 P packed as the P.V A operand, its sum.
+  const float sc = scale * kLog2e;
+  const int kq = key0 + 8 * quad;  // key of element (kt, i) = kq + 32(kt/2) + 4(kt%2) + i
+  float mx = -INFINITY;
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = kq + 32 * (kt >> 1) + 4 * (kt & 1) + i - tbase;
+      const uint32_t vis = (uint32_t)(j < 0) | ((uint32_t)(j < 32) & (tmask >> (j & 31)));
+      s[kt][i] = (vis & 1u) ? s[kt][i] * sc : -INFINITY;
+      mx = fmaxf(mx, s[kt][i]);
+    }
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  const float mref = mx == -INFINITY ? 0.f : mx;  // a row with no visible key here: every P is 0
+  u32x4_t pa[4];
+  float sum = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {  // word w: elements 2(w%2), 2(w%2)+1 of tile 2ks + w/2
+      const int kt = 2 * ks + (w >> 1), i = 2 * (w & 1);
+      const uint16_t b0 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i] - mref));
+      const uint16_t b1 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i + 1] - mref));
+      sum += bf16_bits_to_f32(b0);
+      sum += bf16_bits_to_f32(b1);
+      pa[ks][w] = (uint32_t)b0 | ((uint32_t)b1 << 16);
+    }
+  sum += __shfl_xor(sum, 16, 64);
+  sum += __shfl_xor(sum, 32, 64);
+
+  // 4. O = P V over the 4 key steps of 32; lane holds O rows 4quad + i, dim 16dt + col.
+  f32x4_t o[8];
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt) o[dt] = zero;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pa[ks]);
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt)
+      o[dt] = mfma16x16x32(pf, *reinterpret_cast<const bf16x8_t*>(&vs_lds[(dt * 16 + col) * kPitch + ks * 32 + quad * 8]),
+                           o[dt]);
+  }
+
+  // 5. The chunk partial of this wave's rows.
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float* dst = rows_o + (quad * 4 + i) * kD;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) dst[dt * 16 + col] = o[dt][i];
+  }
+  if (quad == 0) {
+    rows_ml[col * 2] = mx;
+    rows_ml[col * 2 + 1] = sum;
+  }
+}
+
 // The body of the chunk kernel for workgroup (chunk c, kv head h), shared by attn_chunk_kernel and
 // the q|k|v projection + attention kernel of qmm.hip (kWait: see there).
 template <bool kFused, bool kWait = false>
@@ -226,52 +353,9 @@ __device__ __forceinline__ void attn_chunk_body(int c, int h, const int32_t* __r
       if (!mine) ncs[i] = float2{1.f, 0.f};
     }
   }
-  // Fused: the query row's RMSNorm (the lane's 32 squares plus two shuffles across the quads)
-  // and RoPE (dims d and d + 64 in the same lane), into the B operand.
   if constexpr (kFused) {
     if (live) {
-      float x[4][8];
-      float ss = 0.f;
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          x[ks][e] = bf16_bits_to_f32((e & 1) ? (raw[ks][e >> 1] >> 16) : (raw[ks][e >> 1] & 0xffffu));
-          ss = fmaf(x[ks][e], x[ks][e], ss);
-        }
-      ss += __shfl_xor(ss, 16, 64);
-      ss += __shfl_xor(ss, 32, 64);
-      if (fa.qn) {
-        const float inv = rsqrtf(ss / (float)kD + fa.eps);
-#pragma unroll
-        for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float wv = bf16_bits_to_f32((e & 1) ? (wq[ks][e >> 1] >> 16) : (wq[ks][e >> 1] & 0xffffu));
-            x[ks][e] = bf16_bits_to_f32(f32_to_bf16_bits(x[ks][e] * inv * wv));
-          }
-      }
-      u32x4_t lo[2], hi[2];  // rotated dims 32ks + 8quad + e (lo) and those + 64 (hi)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int e2 = 0; e2 < 4; ++e2) {
-          uint32_t wl = 0, wh = 0;
-#pragma unroll
-          for (int bb = 0; bb < 2; ++bb) {
-            const int e = 2 * e2 + bb;
-            const float c2 = cs[ks][e >> 1][(e & 1) * 2], sn = cs[ks][e >> 1][(e & 1) * 2 + 1];
-            const float av = x[ks][e], bv = x[ks + 2][e];
-            wl |= (uint32_t)f32_to_bf16_bits(fmaf(av, c2, -(bv * sn))) << (16 * bb);
-            wh |= (uint32_t)f32_to_bf16_bits(fmaf(bv, c2, av * sn)) << (16 * bb);
-          }
-          lo[ks][e2] = wl;
-          hi[ks][e2] = wh;
-        }
-      qf[0] = __builtin_bit_cast(bf16x8_t, lo[0]);
-      qf[1] = __builtin_bit_cast(bf16x8_t, lo[1]);
-      qf[2] = __builtin_bit_cast(bf16x8_t, hi[0]);
-      qf[3] = __builtin_bit_cast(bf16x8_t, hi[1]);
+      rotate_query(raw, wq, cs, fa.qn != nullptr, fa.eps, qf);
     }
   }
   // Fused: the new key rows, exactly as skinny_qk_rope_store makes them (the same 64-lane sum of
@@ -332,77 +416,8 @@ __device__ __forceinline__ void attn_chunk_body(int c, int h, const int32_t* __r
   }
   if (!busy) return;
 
-  // 2. S^T tiles: element i of tile kt is the score of key 32(kt/2) + 8quad + 4(kt%2) + i.
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  float s[8][4];
-#pragma unroll
-  for (int kt = 0; kt < 8; ++kt) {
-    const int krow = 32 * (kt >> 1) + 8 * (col >> 2) + 4 * (kt & 1) + (col & 3);
-    f32x4_t acc = zero;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      acc = mfma16x16x32(*reinterpret_cast<const bf16x8_t*>(&ks_lds[krow * kPitch + ks * 32 + quad * 8]), qf[ks], acc);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
-  }
-
-  // 3. Visibility, the row maximum (log2 units), bf16 P packed as the P.V A operand, its sum.
-  const float sc = scale * kLog2e;
-  const int kq = key0 + 8 * quad;  // key of element (kt, i) = kq + 32(kt/2) + 4(kt%2) + i
-  float mx = -INFINITY;
-#pragma unroll
-  for (int kt = 0; kt < 8; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int j = kq + 32 * (kt >> 1) + 4 * (kt & 1) + i - tbase;
-      const uint32_t vis = (uint32_t)(j < 0) | ((uint32_t)(j < 32) & (tmask >> (j & 31)));
-      s[kt][i] = (vis & 1u) ? s[kt][i] * sc : -INFINITY;
-      mx = fmaxf(mx, s[kt][i]);
-    }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-  const float mref = mx == -INFINITY ? 0.f : mx;  // a row with no visible key here: every P is 0
-  u32x4_t pa[4];
-  float sum = 0.f;
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {  // word w: elements 2(w%2), 2(w%2)+1 of tile 2ks + w/2
-      const int kt = 2 * ks + (w >> 1), i = 2 * (w & 1);
-      const uint16_t b0 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i] - mref));
-      const uint16_t b1 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i + 1] - mref));
-      sum += bf16_bits_to_f32(b0);
-      sum += bf16_bits_to_f32(b1);
-      pa[ks][w] = (uint32_t)b0 | ((uint32_t)b1 << 16);
-    }
-  sum += __shfl_xor(sum, 16, 64);
-  sum += __shfl_xor(sum, 32, 64);
-
-  // 4. O = P V over the 4 key steps of 32; lane holds O rows 4quad + i, dim 16dt + col.
-  f32x4_t o[8];
-#pragma unroll
-  for (int dt = 0; dt < 8; ++dt) o[dt] = zero;
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pa[ks]);
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt)
-      o[dt] = mfma16x16x32(pf, *reinterpret_cast<const bf16x8_t*>(&vs_lds[(dt * 16 + col) * kPitch + ks * 32 + quad * 8]),
-                           o[dt]);
-  }
-
-  // 5. The chunk partial of this wave's rows.
   const size_t base = ((size_t)h * nchunk_max + c) * kRowsMax + wave * 16;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float* dst = part_o + (base + quad * 4 + i) * kD;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) dst[dt * 16 + col] = o[dt][i];
-  }
-  if (quad == 0) {
-    part_ml[(base + col) * 2] = mx;
-    part_ml[(base + col) * 2 + 1] = sum;
-  }
+  attn_rows(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, part_o + base * kD, part_ml + base * 2);
 }
 
 }  // namespace

@@ -116,6 +116,85 @@ __global__ __launch_bounds__(64) void general_qk_store_kernel(const int32_t* __r
   for (int e = 0; e < E; ++e) dst[lane + 64 * e] = outv[e];
 }
 
+// One wave's 16 query rows against the staged chunk of keys key0 .. (attn.hip's attn_rows over D dims):
+// the partial O rows to rows_o [16][D], the row maxima (log2 units) and sums to rows_ml [16][2].
+template <int D>
+__device__ __forceinline__ void general_rows(const uint16_t* ks_lds, const uint16_t* vs_lds, const bf16x8_t (&qf)[D / 32],
+                                             int key0, int tbase, uint32_t tmask, float scale, float* __restrict__ rows_o,
+                                             float* __restrict__ rows_ml) {
+  constexpr int CH = general_chunk(D);
+  constexpr int KS = D / 32;   // 32-dim steps of a score
+  constexpr int DT = D / 16;   // 16-dim tiles of an output row
+  constexpr int KT = CH / 16;  // 16-key tiles of the chunk
+  constexpr int PS = CH / 32;  // 32-key steps of P.V
+  constexpr int KP = D + 8, VP = CH + 8;
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  float s[KT][4];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    const int krow = 32 * (kt >> 1) + 8 * (col >> 2) + 4 * (kt & 1) + (col & 3);
+    f32x4_t acc = zero;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      acc = mfma16x16x32(*reinterpret_cast<const bf16x8_t*>(&ks_lds[krow * KP + ks * 32 + quad * 8]), qf[ks], acc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
+  }
+  const float sc = scale * kGLog2e;
+  const int kq = key0 + 8 * quad;
+  float mx = -INFINITY;
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = kq + 32 * (kt >> 1) + 4 * (kt & 1) + i - tbase;
+      const uint32_t vis = (uint32_t)(j < 0) | ((uint32_t)(j < 32) & (tmask >> (j & 31)));
+      s[kt][i] = (vis & 1u) ? s[kt][i] * sc : -INFINITY;
+      mx = fmaxf(mx, s[kt][i]);
+    }
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  const float mref = mx == -INFINITY ? 0.f : mx;
+  u32x4_t pa[PS];
+  float sum = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < PS; ++ks)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int kt = 2 * ks + (w >> 1), i = 2 * (w & 1);
+      const uint16_t b0 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i] - mref));
+      const uint16_t b1 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i + 1] - mref));
+      sum += bf16_bits_to_f32(b0);
+      sum += bf16_bits_to_f32(b1);
+      pa[ks][w] = (uint32_t)b0 | ((uint32_t)b1 << 16);
+    }
+  sum += __shfl_xor(sum, 16, 64);
+  sum += __shfl_xor(sum, 32, 64);
+  // O = P V: lane holds O rows 4quad + i, dim 16dt + col; V^T row (16dt + col) keys 32ks + 8quad.
+  f32x4_t o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] = zero;
+#pragma unroll
+  for (int ks = 0; ks < PS; ++ks) {
+    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pa[ks]);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      o[dt] = mfma16x16x32(pf, *reinterpret_cast<const bf16x8_t*>(&vs_lds[(dt * 16 + col) * VP + ks * 32 + quad * 8]),
+                           o[dt]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    float* dst = rows_o + (quad * 4 + i) * D;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) dst[dt * 16 + col] = o[dt][i];
+  }
+  if (quad == 0) {
+    rows_ml[col * 2] = mx;
+    rows_ml[col * 2 + 1] = sum;
+  }
+}
+
 // (2) Workgroup (chunk c, kv head h), keys [CH c, CH c + CH); wave w takes the query rows
 // 16w .. 16w + 15 of the (token, group head) rows. attn.hip's chunk kernel over D dims: every thread
 // issues its 16-byte pieces of the chunk's K rows and V^T rows at once (PIECES of each), they go to
@@ -132,10 +211,7 @@ __global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32
                                                                      float* __restrict__ part_o,
                                                                      float* __restrict__ part_ml, int nchunk_max) {
   constexpr int CH = general_chunk(D);
-  constexpr int KS = D / 32;   // 32-dim steps of a score
-  constexpr int DT = D / 16;   // 16-dim tiles of an output row
-  constexpr int KT = CH / 16;  // 16-key tiles of the chunk
-  constexpr int PS = CH / 32;  // 32-key steps of P.V
+  constexpr int KS = D / 32;  // 32-dim steps of a score
   constexpr int KP = D + 8, VP = CH + 8;
   constexpr int PIECES = CH * D / 8 / (64 * kGWaves);  // 16-byte pieces per thread of K, and of V^T
   static_assert(PIECES * 8 * 64 * kGWaves == CH * D, "the chunk splits evenly over the threads");
@@ -196,71 +272,8 @@ __global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32
   __syncthreads();
   if (!busy) return;
 
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  float s[KT][4];
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt) {
-    const int krow = 32 * (kt >> 1) + 8 * (col >> 2) + 4 * (kt & 1) + (col & 3);
-    f32x4_t acc = zero;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      acc = mfma16x16x32(*reinterpret_cast<const bf16x8_t*>(&ks_lds[krow * KP + ks * 32 + quad * 8]), qf[ks], acc);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
-  }
-  const float sc = scale * kGLog2e;
-  const int kq = key0 + 8 * quad;
-  float mx = -INFINITY;
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int j = kq + 32 * (kt >> 1) + 4 * (kt & 1) + i - tbase;
-      const uint32_t vis = (uint32_t)(j < 0) | ((uint32_t)(j < 32) & (tmask >> (j & 31)));
-      s[kt][i] = (vis & 1u) ? s[kt][i] * sc : -INFINITY;
-      mx = fmaxf(mx, s[kt][i]);
-    }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-  const float mref = mx == -INFINITY ? 0.f : mx;
-  u32x4_t pa[PS];
-  float sum = 0.f;
-#pragma unroll
-  for (int ks = 0; ks < PS; ++ks)
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int kt = 2 * ks + (w >> 1), i = 2 * (w & 1);
-      const uint16_t b0 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i] - mref));
-      const uint16_t b1 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i + 1] - mref));
-      sum += bf16_bits_to_f32(b0);
-      sum += bf16_bits_to_f32(b1);
-      pa[ks][w] = (uint32_t)b0 | ((uint32_t)b1 << 16);
-    }
-  sum += __shfl_xor(sum, 16, 64);
-  sum += __shfl_xor(sum, 32, 64);
-  // O = P V: lane holds O rows 4quad + i, dim 16dt + col; V^T row (16dt + col) keys 32ks + 8quad.
-  f32x4_t o[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] = zero;
-#pragma unroll
-  for (int ks = 0; ks < PS; ++ks) {
-    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pa[ks]);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-      o[dt] = mfma16x16x32(pf, *reinterpret_cast<const bf16x8_t*>(&vs_lds[(dt * 16 + col) * VP + ks * 32 + quad * 8]),
-                           o[dt]);
-  }
   const size_t base = ((size_t)h * nchunk_max + c) * kGRowsMax + wave * 16;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float* dst = part_o + (base + quad * 4 + i) * D;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) dst[dt * 16 + col] = o[dt][i];
-  }
-  if (quad == 0) {
-    part_ml[(base + col) * 2] = mx;
-    part_ml[(base + col) * 2 + 1] = sum;
-  }
+  general_rows<D>(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, part_o + base * D, part_ml + base * 2);
 }
 
 // (3) One workgroup per (query head, token), max(1, D / 128) waves, lane l of wave w holding dims
@@ -274,19 +287,19 @@ __global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32
 template <int D>
 constexpr int general_combine_waves() { return D > 128 ? D / 128 : 1; }
 
-template <int D>
-__global__ __launch_bounds__(64 * general_combine_waves<D>()) void general_combine_kernel(
-    const int32_t* __restrict__ pos0, const float* __restrict__ part_o, const float* __restrict__ part_ml, int M,
-    int Hq, int Hkv, int nchunk_max, const uint16_t* __restrict__ qkv, HeadLayout hl, uint16_t* __restrict__ out) {
+// (chunk c's partial row at head_base + c * kGRowsMax; pos0[0] + tokens keys; gate_at(): the row's gate
+// values or NULL, and out_at(): its output, asked for last, since their arguments lie past the preloaded ones)
+template <int D, typename GateAt, typename OutAt>
+__device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ pos0, const float* __restrict__ part_o,
+                                                    const float* __restrict__ part_ml, size_t head_base, int tokens,
+                                                    int nchunk_max, GateAt gate_at, OutAt out_at) {
   constexpr int CH = general_chunk(D);
   constexpr int B = kGCombineBlock, GR = 8;
   constexpr int CW = D / 64 / general_combine_waves<D>();  // dims per lane: 1 or 2
   typedef __attribute__((ext_vector_type(CW))) float dims_t;
-  const int hq = blockIdx.x, t = blockIdx.y, lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63;
   const int d0 = (int)threadIdx.x * CW;  // this lane's first dim
-  const int G = Hq / Hkv, h = hq / G, row = t * G + hq % G;
-  const size_t head_base = (size_t)h * nchunk_max * kGRowsMax + row;  // chunk c at + c * kGRowsMax
-  const int nch = min((pos0[0] + M + CH - 1) / CH, nchunk_max);
+  const int nch = min((pos0[0] + tokens + CH - 1) / CH, nchunk_max);
   float run_m = -INFINITY, run_l = 0.f, a[CW];
 #pragma unroll
   for (int k = 0; k < CW; ++k) a[k] = 0.f;
@@ -326,18 +339,116 @@ __global__ __launch_bounds__(64 * general_combine_waves<D>()) void general_combi
     run_m = new_m;
   }
   const float inv = run_l > 0.f ? 1.0f / run_l : 0.f;
-  uint16_t* dst = out + ((size_t)t * Hq + hq) * D + d0;
+  const uint16_t* gate = gate_at();
+  uint16_t* dst = out_at() + d0;
 #pragma unroll
   for (int k = 0; k < CW; ++k) {
     const uint16_t ob = f32_to_bf16_bits(a[k] * inv);
-    if (hl.goff >= 0) {
-      const float g = bf16_bits_to_f32(qkv[(size_t)t * hl.ldq + hl.goff + (size_t)hq * hl.qs + d0 + k]);
+    if (gate) {
+      const float g = bf16_bits_to_f32(gate[d0 + k]);
       const float sg = bf16_bits_to_f32(f32_to_bf16_bits(1.0f / (1.0f + expf(-g))));
       dst[k] = f32_to_bf16_bits(bf16_bits_to_f32(ob) * sg);
     } else {
       dst[k] = ob;
     }
   }
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * general_combine_waves<D>()) void general_combine_kernel(
+    const int32_t* __restrict__ pos0, const float* __restrict__ part_o, const float* __restrict__ part_ml, int M,
+    int Hq, int Hkv, int nchunk_max, const uint16_t* __restrict__ qkv, HeadLayout hl, uint16_t* __restrict__ out) {
+  const int hq = blockIdx.x, t = blockIdx.y;
+  const int G = Hq / Hkv, h = hq / G, row = t * G + hq % G;
+  general_combine_row<D>(
+      pos0, part_o, part_ml, (size_t)h * nchunk_max * kGRowsMax + row, M, nchunk_max,
+      [&] { return hl.goff >= 0 ? qkv + (size_t)t * hl.ldq + hl.goff + (size_t)hq * hl.qs : nullptr; },
+      [&] { return out + ((size_t)t * Hq + hq) * D; });
+}
+
+// --- the attention of a prompt: more tokens than one step holds ---------------------------------
+// As attn.hip's prompt kernels: pieces of kGMaxTokens tokens, every row's arithmetic that of the step
+// kernels over its piece, one staged chunk shared by a group of pieces.
+constexpr int kGPieceGroup = 4;  // pieces that share a staged chunk
+
+// The values of 64 tokens of head blockIdx.x from token 64 blockIdx.y on, turned in LDS so that the stores
+// into V^T run along the cache slots.
+template <int D>
+__global__ __launch_bounds__(256) void general_prompt_v_kernel(const int32_t* __restrict__ pos0,
+                                                               const uint16_t* __restrict__ qkv, HeadLayout hl, int M,
+                                                               uint16_t* __restrict__ vt, int maxlen) {
+  __shared__ uint16_t vl[64][D + 2];
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int h = blockIdx.x, t0 = blockIdx.y * 64, p0 = pos0[0];
+  for (int e = threadIdx.x; e < 64 * D; e += 256) {
+    const int t = e / D, d = e % D;
+    vl[t][d] = qkv[(size_t)min(t0 + t, M - 1) * hl.ldq + hl.voff + (size_t)h * D + d];
+  }
+  __syncthreads();
+  if (t0 + lane < M)
+    for (int d = wave; d < D; d += 4) vt[((size_t)h * D + d) * maxlen + p0 + t0 + lane] = vl[lane][d];
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * kGWaves) void general_prompt_chunk_kernel(
+    const int32_t* __restrict__ pos0, const uint16_t* __restrict__ q, int M, int Hq, int Hkv,
+    const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vt, int maxlen, float scale, int z0, int z1, int nch,
+    float* __restrict__ part_o, float* __restrict__ part_ml) {
+  constexpr int CH = general_chunk(D);
+  constexpr int KS = D / 32;
+  constexpr int KP = D + 8, VP = CH + 8;
+  constexpr int PIECES = CH * D / 8 / (64 * kGWaves);
+  __shared__ __attribute__((aligned(16))) uint16_t ks_lds[CH * KP];
+  __shared__ __attribute__((aligned(16))) uint16_t vs_lds[D * VP];
+  const int c = blockIdx.x, h = blockIdx.y, p0 = pos0[0], G = Hq / Hkv;
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int za = z0 + (int)blockIdx.z * kGPieceGroup, zb = min(za + kGPieceGroup, z1);
+  const int key0 = c * CH;
+  if (key0 >= p0 + min(M, zb * kGMaxTokens)) return;  // past the last piece's keys
+  const u32x4_t* kh = reinterpret_cast<const u32x4_t*>(kc + ((size_t)h * maxlen + key0) * D);
+  const uint16_t* vh = vt + (size_t)h * D * maxlen + key0;
+  u32x4_t kr[PIECES], vr[PIECES];
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int e = threadIdx.x + i * 64 * kGWaves;
+    kr[i] = kh[e];
+    vr[i] = *reinterpret_cast<const u32x4_t*>(vh + (size_t)(e / (CH / 8)) * maxlen + (e % (CH / 8)) * 8);
+  }
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int e = threadIdx.x + i * 64 * kGWaves;
+    *reinterpret_cast<u32x4_t*>(&ks_lds[(e / (D / 8)) * KP + (e % (D / 8)) * 8]) = kr[i];
+    *reinterpret_cast<u32x4_t*>(&vs_lds[(e / (CH / 8)) * VP + (e % (CH / 8)) * 8]) = vr[i];
+  }
+  __syncthreads();
+  const int col = lane & 15, quad = lane >> 4, qrow = wave * 16 + col;
+  for (int z = za; z < zb; ++z) {
+    const int t0 = z * kGMaxTokens, mb = min(kGMaxTokens, M - t0), rows = G * mb;
+    if (key0 >= p0 + t0 + mb || wave * 16 >= rows) continue;
+    const bool live = qrow < rows;
+    const uint16_t* qr = q + ((size_t)(live ? t0 + qrow / G : 0) * Hq + h * G + (live ? qrow % G : 0)) * D;
+    bf16x8_t qf[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      qf[ks] = *reinterpret_cast<const bf16x8_t*>(qr + ks * 32 + quad * 8);
+      if (!live) qf[ks] = bf16x8_t{};
+    }
+    const size_t base = (((size_t)(z - z0) * Hkv + h) * nch + c) * kGRowsMax + wave * 16;
+    general_rows<D>(ks_lds, vs_lds, qf, key0, live ? p0 + t0 + qrow / G + 1 : key0, 0u, scale, part_o + base * D,
+                    part_ml + base * 2);
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(64 * general_combine_waves<D>()) void general_prompt_combine_kernel(
+    const int32_t* __restrict__ pos0, const float* __restrict__ part_o, const float* __restrict__ part_ml, int M, int Hq,
+    int Hkv, int z0, int nch, const uint16_t* __restrict__ qkv, HeadLayout hl, uint16_t* __restrict__ out) {
+  const int hq = blockIdx.x, t = z0 * kGMaxTokens + (int)blockIdx.y, z = t / kGMaxTokens;
+  const int G = Hq / Hkv, h = hq / G, row = (t % kGMaxTokens) * G + hq % G;
+  general_combine_row<D>(
+      pos0, part_o, part_ml, (((size_t)(z - z0) * Hkv + h) * nch) * kGRowsMax + row, min(M, (z + 1) * kGMaxTokens), nch,
+      [&] { return hl.goff >= 0 ? qkv + (size_t)t * hl.ldq + hl.goff + (size_t)hq * hl.qs : nullptr; },
+      [&] { return out + ((size_t)t * Hq + hq) * D; });
 }
 
 // cos/sin table of a RoPE over R dims: table[pos][i] = (cos, sin)(pos * theta^(-2i/R)), i < R/2,
@@ -372,6 +483,44 @@ int launch_general(const int32_t* pos0, const uint16_t* qkv, const HeadLayout& h
   hipLaunchKernelGGL(general_combine_kernel<D>, dim3(Hq, M), dim3(64 * general_combine_waves<D>()), 0, stream, pos0,
                      part_o, part_ml, M, Hq, Hkv, nch, qkv, hl, out);
   return skinny_check_launch("attention_general merge");
+}
+
+// Workspace of a prompt's attention: the rotated queries, then the partials of as many pieces as fit
+// kGPromptPartBytes (at least one group of pieces).
+constexpr size_t kGPromptPartBytes = (size_t)256 << 20;
+
+size_t gprompt_piece_bytes(int Hkv, int D, int nch) { return (size_t)Hkv * nch * kGRowsMax * (D + 2) * sizeof(float); }
+
+size_t gprompt_query_bytes(int M, int Hq, int D) { return ((size_t)M * Hq * D * 2 + 255) & ~(size_t)255; }
+
+template <int D>
+int launch_general_prompt(const int32_t* pos0, const uint16_t* qkv, const HeadLayout& hl, int M, int Hq, int Hkv,
+                          const uint16_t* qn, const uint16_t* kn, float eps, int R, const float* rope, int keys,
+                          uint16_t* kc, uint16_t* vt, int maxlen, float scale, char* ws, int fit, uint16_t* out,
+                          hipStream_t stream) {
+  constexpr int CH = general_chunk(D);
+  const int nch = (keys + CH - 1) / CH, pieces = (M + kGMaxTokens - 1) / kGMaxTokens;
+  uint16_t* q = reinterpret_cast<uint16_t*>(ws);
+  float* part_o = reinterpret_cast<float*>(ws + gprompt_query_bytes(M, Hq, D));
+  float* part_ml = part_o + (size_t)fit * Hkv * nch * kGRowsMax * D;
+  hipLaunchKernelGGL(general_qk_store_kernel<D>, dim3(Hq + Hkv, M), dim3(64), 0, stream, pos0, qkv, hl, Hq, Hkv, qn, kn,
+                     eps, R, rope, nullptr, M, q, kc, vt, maxlen);
+  if (int rc = skinny_check_launch("attention_general prompt q/k")) return rc;
+  hipLaunchKernelGGL(general_prompt_v_kernel<D>, dim3(Hkv, (M + 63) / 64), dim3(256), 0, stream, pos0, qkv, hl, M, vt, maxlen);
+  if (int rc = skinny_check_launch("attention_general prompt v")) return rc;
+  for (int z0 = 0; z0 < pieces; z0 += fit) {
+    const int z1 = z0 + fit < pieces ? z0 + fit : pieces;
+    const int last = z1 * kGMaxTokens < M ? z1 * kGMaxTokens : M;
+    const int n = (keys - M + last + CH - 1) / CH;
+    hipLaunchKernelGGL(general_prompt_chunk_kernel<D>, dim3(n, Hkv, (z1 - z0 + kGPieceGroup - 1) / kGPieceGroup),
+                       dim3(64 * kGWaves), 0, stream, pos0, q, M, Hq, Hkv, kc, vt, maxlen, scale, z0, z1, nch, part_o, part_ml);
+    if (int rc = skinny_check_launch("attention_general prompt chunks")) return rc;
+    hipLaunchKernelGGL(general_prompt_combine_kernel<D>, dim3(Hq, last - z0 * kGMaxTokens),
+                       dim3(64 * general_combine_waves<D>()), 0, stream, pos0, part_o, part_ml, M, Hq, Hkv, z0, nch, qkv, hl,
+                       out);
+    if (int rc = skinny_check_launch("attention_general prompt merge")) return rc;
+  }
+  return SKINNY_OK;
 }
 
 }  // namespace
@@ -439,5 +588,63 @@ extern "C" int skinny_attention_general_bf16(const uint16_t* qkv, int ldq, int M
     default:
       return launch_general<256>(pos0, qkv, hl, M, Hq, Hkv, q_norm, k_norm, eps, rotary_dim, rope_table, tree, k_cache,
                                  vt_cache, maxlen, scale, ws, nch, out, s);
+  }
+}
+
+extern "C" size_t skinny_attn_general_prompt_workspace_bytes(int M, int Hq, int Hkv, int D, int keys) {
+  if (M < 1 || Hq < 1 || Hkv < 1 || (D != 64 && D != 128 && D != 256) || keys < 1) return 0;
+  const int ch = general_chunk(D);
+  const size_t piece = gprompt_piece_bytes(Hkv, D, (keys + ch - 1) / ch);
+  const size_t all = (size_t)((M + kGMaxTokens - 1) / kGMaxTokens) * piece, group = kGPieceGroup * piece;
+  const size_t most = kGPromptPartBytes / group * group;
+  return gprompt_query_bytes(M, Hq, D) + (all <= most ? all : most > group ? most : group < all ? group : all);
+}
+
+extern "C" int skinny_attention_general_prompt_bf16(const uint16_t* qkv, int ldq, int M, int Hq, int Hkv, int D,
+                                                    int q_stride, int k_offset, int v_offset, int gate_offset,
+                                                    const uint16_t* q_norm, const uint16_t* k_norm, float eps,
+                                                    int rotary_dim, const float* rope_table, int rope_positions,
+                                                    const int32_t* pos0, int keys, uint16_t* k_cache, uint16_t* vt_cache,
+                                                    int maxlen, float scale, void* workspace, size_t workspace_bytes,
+                                                    uint16_t* out, void* stream) {
+  SKINNY_CHECK_ARG(qkv && rope_table && pos0 && k_cache && vt_cache && workspace && out,
+                   "attention_general prompt: null pointer");
+  SKINNY_CHECK_ARG(D == 64 || D == 128 || D == 256, "attention_general prompt: head dim %d unsupported (64, 128 or 256)", D);
+  SKINNY_CHECK_ARG(Hkv >= 1 && Hq >= Hkv && Hq % Hkv == 0 && (Hq / Hkv) * kGMaxTokens <= kGRowsMax,
+                   "attention_general prompt: Hq=%d must be a multiple of Hkv=%d, at most %d query heads each", Hq, Hkv,
+                   kGRowsMax / kGMaxTokens);
+  SKINNY_CHECK_ARG(M >= 1 && M <= 65535 && keys >= M && keys <= maxlen,
+                   "attention_general prompt: M=%d (at most 65535), keys=%d in [M, maxlen=%d]", M, keys, maxlen);
+  SKINNY_CHECK_ARG(rotary_dim >= 2 && rotary_dim % 2 == 0 && rotary_dim <= D,
+                   "attention_general prompt: rotary_dim=%d must be even, in [2, D=%d]", rotary_dim, D);
+  SKINNY_CHECK_ARG(q_stride >= D && (gate_offset < 0 || gate_offset + (size_t)(Hq - 1) * q_stride + D <= (size_t)ldq) &&
+                       k_offset >= 0 && v_offset >= 0 && (size_t)(Hq - 1) * q_stride + D <= (size_t)ldq &&
+                       (size_t)k_offset + (size_t)Hkv * D <= (size_t)ldq && (size_t)v_offset + (size_t)Hkv * D <= (size_t)ldq,
+                   "attention_general prompt: heads do not fit the q|k|v row of %d", ldq);
+  SKINNY_CHECK_ARG(maxlen >= kGChunk && maxlen % kGChunk == 0 && rope_positions >= maxlen,
+                   "attention_general prompt: maxlen=%d must be a multiple of %d and within the RoPE table (%d)", maxlen,
+                   kGChunk, rope_positions);
+  SKINNY_CHECK_ARG(skinny_aligned(k_cache, 16) && skinny_aligned(vt_cache, 16) && skinny_aligned(workspace, 16) &&
+                       skinny_aligned(qkv, 2) && skinny_aligned(rope_table, 8),
+                   "attention_general prompt: misaligned buffer");
+  const int ch = general_chunk(D), nch = (keys + ch - 1) / ch, pieces = (M + kGMaxTokens - 1) / kGMaxTokens;
+  const size_t piece = gprompt_piece_bytes(Hkv, D, nch), qb = gprompt_query_bytes(M, Hq, D);
+  const size_t room = workspace_bytes > qb ? (workspace_bytes - qb) / piece : 0;
+  int fit = room < (size_t)pieces ? (int)room / kGPieceGroup * kGPieceGroup : pieces;
+  SKINNY_CHECK_ARG(fit >= 1, "attention_general prompt: workspace of %zu bytes, needs %zu", workspace_bytes,
+                   skinny_attn_general_prompt_workspace_bytes(M, Hq, Hkv, D, keys));
+  const HeadLayout hl{ldq, q_stride, k_offset, v_offset, gate_offset};
+  char* ws = static_cast<char*>(workspace);
+  const hipStream_t s = (hipStream_t)stream;
+  switch (D) {
+    case 64:
+      return launch_general_prompt<64>(pos0, qkv, hl, M, Hq, Hkv, q_norm, k_norm, eps, rotary_dim, rope_table, keys, k_cache,
+                                       vt_cache, maxlen, scale, ws, fit, out, s);
+    case 128:
+      return launch_general_prompt<128>(pos0, qkv, hl, M, Hq, Hkv, q_norm, k_norm, eps, rotary_dim, rope_table, keys, k_cache,
+                                        vt_cache, maxlen, scale, ws, fit, out, s);
+    default:
+      return launch_general_prompt<256>(pos0, qkv, hl, M, Hq, Hkv, q_norm, k_norm, eps, rotary_dim, rope_table, keys, k_cache,
+                                        vt_cache, maxlen, scale, ws, fit, out, s);
   }
 }

@@ -38,6 +38,10 @@ __device__ __forceinline__ f32x4_t mfma16x16x32(bf16x8_t a, bf16x8_t b, f32x4_t 
 // it can live in SGPRs, e.g. buffer-load soffsets, which otherwise become per-load waterfall loops.
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
+// LDS writes of this wave complete, then every wave of the workgroup meets. Global loads still in
+// flight are not waited for (unlike __syncthreads()).
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // fp32 -> bf16 bits, round to nearest even: gfx950's v_cvt_pk_bf16_f32 (one instruction, where
 // the integer rounding sequence took five or six).
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }

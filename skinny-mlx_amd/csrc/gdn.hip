@@ -126,6 +126,44 @@ __global__ __launch_bounds__(kConvThreads) void conv_silu_kernel(const uint16_t*
   for (int j = 0; j < KW - 1; ++j) conv_state[(size_t)j * C + c] = hist[j];
 }
 
+// The same conv for a prompt: one thread per (channel, block of kTokBlock tokens). A token's taps are input
+// rows (or conv-state rows for the first KW - 1), so the blocks need nothing from each other; block 0 reads
+// the state before the call and writes the one after it (the last KW - 1 input rows; M >= KW - 1). The
+// sequential kernel above takes a memory round trip per block of 16 tokens with C / 256 workgroups. out must
+// not overlap x.
+template <int KW>
+__global__ __launch_bounds__(kConvThreads) void conv_silu_rows_kernel(const uint16_t* __restrict__ x, int ldx, int M, int C,
+                                                                      uint16_t* conv_state, const uint16_t* __restrict__ w,
+                                                                      uint16_t* __restrict__ out, int ldo) {
+  const int c = blockIdx.x * blockDim.x + threadIdx.x, t0 = blockIdx.y * kTokBlock;
+  if (c >= C) return;
+  float wv[KW];
+  uint16_t v[KW - 1 + kTokBlock], tail[KW - 1];
+#pragma unroll
+  for (int j = 0; j < KW; ++j) wv[j] = bf16_bits_to_f32(w[(size_t)c * KW + j]);
+#pragma unroll
+  for (int j = 0; j < KW - 1; ++j)
+    v[j] = t0 == 0 ? conv_state[(size_t)j * C + c] : x[(size_t)(t0 - (KW - 1) + j) * ldx + c];
+#pragma unroll
+  for (int i = 0; i < kTokBlock; ++i) v[KW - 1 + i] = x[(size_t)min(t0 + i, M - 1) * ldx + c];
+  if (t0 == 0) {
+#pragma unroll
+    for (int j = 0; j < KW - 1; ++j) tail[j] = x[(size_t)(M - (KW - 1) + j) * ldx + c];
+  }
+#pragma unroll
+  for (int i = 0; i < kTokBlock; ++i) {
+    if (t0 + i >= M) break;
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < KW; ++j) acc = fmaf(wv[j], bf16_bits_to_f32(v[i + j]), acc);
+    out[(size_t)(t0 + i) * ldo + c] = f32_to_bf16_bits(acc / (1.0f + expf(-acc)));
+  }
+  if (t0 == 0) {
+#pragma unroll
+    for (int j = 0; j < KW - 1; ++j) conv_state[(size_t)j * C + c] = tail[j];
+  }
+}
+
 // One token of the gated delta rule for the 8 key dims a lane holds of one value column (the
 // column's 16 lanes together hold all 128): S <- decay S + k delta with delta = beta (v - k.(decay
 // S)), then y = q.S. k.S is formed on the undecayed state and scaled once (decay (k.S)), in four
@@ -165,7 +203,9 @@ constexpr int kGdnThreads = kCols * kPart;
 
 // kTree: the draft-tree form (parent pointers, per-node snapshots in LDS) is its own kernel, so
 // the chain form carries none of its code (measured: 0.1-0.3 us faster per launch that way).
-template <bool kTree>
+// kLong: a chain of more than one block of tokens (a prompt) loads the next block's rows while the current
+// one runs, so that only the first block waits for memory.
+template <bool kTree, bool kLong = false>
 __global__ __launch_bounds__(kGdnThreads) void gdn_kernel(const uint16_t* __restrict__ qkv, int ldq,
                                                           const uint16_t* __restrict__ bcol,
                                                           const uint16_t* __restrict__ acol, int ldab,
@@ -197,23 +237,54 @@ __global__ __launch_bounds__(kGdnThreads) void gdn_kernel(const uint16_t* __rest
   float s0[8];  // the state before the step: a draft tree's root and its restarts branch from it
 #pragma unroll
   for (int e = 0; e < 8; ++e) s0[e] = s[e];
+  constexpr int kNextQk = kTokBlock * 32 / kGdnThreads;
+  static_assert(kTokBlock * kCols == kGdnThreads, "one value of v per thread and block");
+  u32x4_t nqk[kLong ? kNextQk : 1];  // kLong: the next block, tokens past the end repeat the last one
+  uint16_t nv = 0, na = 0, nb = 0;
+  auto load_next = [&](int t0) {
+#pragma unroll
+    for (int r = 0; r < kNextQk; ++r) {
+      const int i = tid + r * kGdnThreads, t = min(t0 + (i >> 5), M - 1);
+      nqk[r] = *reinterpret_cast<const u32x4_t*>(qkv + (size_t)t * ldq + (size_t)((i >> 4) & 1) * Hk * kDk + (size_t)hk * kDk +
+                                                 (i & 15) * 8);
+    }
+    nv = qkv[(size_t)min(t0 + tid / kCols, M - 1) * ldq + (size_t)2 * Hk * kDk + (size_t)h * kDv + blockIdx.y * kCols + tid % kCols];
+    const size_t g = (size_t)min(t0 + (tid & (kTokBlock - 1)), M - 1) * ldab + h;
+    na = acol[g];
+    nb = bcol[g];
+  };
+  if constexpr (kLong) load_next(0);
   for (int t0 = 0; t0 < M; t0 += kTokBlock) {
     const int mb = min(kTokBlock, M - t0);
     if (t0 > 0) __syncthreads();  // the previous block's staged rows are no longer read
-    for (int i = tid; i < mb * 32; i += kGdnThreads) {  // q and k: 16 pieces of 16 bytes each per token
-      const int t = i >> 5, sel = (i >> 4) & 1, piece = i & 15;
-      *reinterpret_cast<u32x4_t*>(&qk_lds[t][sel][piece * 8]) = *reinterpret_cast<const u32x4_t*>(
-          qkv + (size_t)(t0 + t) * ldq + (size_t)sel * Hk * kDk + (size_t)hk * kDk + piece * 8);
+    if constexpr (kLong) {
+#pragma unroll
+      for (int r = 0; r < kNextQk; ++r) {
+        const int i = tid + r * kGdnThreads;
+        *reinterpret_cast<u32x4_t*>(&qk_lds[i >> 5][(i >> 4) & 1][(i & 15) * 8]) = nqk[r];
+      }
+      v_lds[tid / kCols][tid % kCols] = nv;
+      if (tid < mb) {
+        gate_lds[tid][0] = expf(neg_a * softplus(bf16_bits_to_f32(na) + dtb));
+        gate_lds[tid][1] = 1.0f / (1.0f + expf(-bf16_bits_to_f32(nb)));
+      }
+      if (t0 + kTokBlock < M) load_next(t0 + kTokBlock);
+    } else {
+      for (int i = tid; i < mb * 32; i += kGdnThreads) {  // q and k: 16 pieces of 16 bytes each per token
+        const int t = i >> 5, sel = (i >> 4) & 1, piece = i & 15;
+        *reinterpret_cast<u32x4_t*>(&qk_lds[t][sel][piece * 8]) = *reinterpret_cast<const u32x4_t*>(
+            qkv + (size_t)(t0 + t) * ldq + (size_t)sel * Hk * kDk + (size_t)hk * kDk + piece * 8);
+      }
+      for (int i = tid; i < mb * kCols; i += kGdnThreads)
+        v_lds[i / kCols][i % kCols] =
+            qkv[(size_t)(t0 + i / kCols) * ldq + (size_t)2 * Hk * kDk + (size_t)h * kDv + blockIdx.y * kCols + i % kCols];
+      if (tid < mb) {
+        gate_lds[tid][0] = expf(neg_a * softplus(bf16_bits_to_f32(acol[(size_t)(t0 + tid) * ldab + h]) + dtb));
+        gate_lds[tid][1] = 1.0f / (1.0f + expf(-bf16_bits_to_f32(bcol[(size_t)(t0 + tid) * ldab + h])));
+        if constexpr (kTree) par_lds[tid] = parent[t0 + tid];
+      }
     }
-    for (int i = tid; i < mb * kCols; i += kGdnThreads)
-      v_lds[i / kCols][i % kCols] =
-          qkv[(size_t)(t0 + i / kCols) * ldq + (size_t)2 * Hk * kDk + (size_t)h * kDv + blockIdx.y * kCols + i % kCols];
-    if (tid < mb) {
-      gate_lds[tid][0] = expf(neg_a * softplus(bf16_bits_to_f32(acol[(size_t)(t0 + tid) * ldab + h]) + dtb));
-      gate_lds[tid][1] = 1.0f / (1.0f + expf(-bf16_bits_to_f32(bcol[(size_t)(t0 + tid) * ldab + h])));
-      if constexpr (kTree) par_lds[tid] = parent[t0 + tid];
-    }
-    __syncthreads();
+    lds_barrier();  // (a next block's loads stay in flight)
     // Normalised q and k of every token of the block, in parallel (they do not depend on the
     // state): 16-lane group g takes tokens g, g + kCols, ...; lane p its 8 dims.
     for (int i = cc; i < mb; i += kCols) {
@@ -237,7 +308,7 @@ __global__ __launch_bounds__(kGdnThreads) void gdn_kernel(const uint16_t* __rest
       kd[0] = f32x4_t{k[0] * kn, k[1] * kn, k[2] * kn, k[3] * kn};
       kd[1] = f32x4_t{k[4] * kn, k[5] * kn, k[6] * kn, k[7] * kn};
     }
-    __syncthreads();
+    lds_barrier();
     if constexpr (kTree) {
       if (record) {  // the commit's replay operands (a tree is one block: t0 == 0)
         const GdnRecord rl(kTokBlock, H);
@@ -578,6 +649,13 @@ extern "C" int skinny_gdn_conv_silu(const uint16_t* x, int ldx, int M, int C, in
   SKINNY_CHECK_ARG(M >= 1 && C >= 1 && ldx >= C && ldo >= C, "gdn_conv: bad shape");
   SKINNY_CHECK_ARG(!parent || window, "gdn_conv: a draft tree needs the window buffer");
   SKINNY_CHECK_ARG(!parent || M <= kTokBlock, "gdn_conv: a draft tree holds at most %d tokens (M=%d)", kTokBlock, M);
+  // more than one block of tokens, nothing recorded: the blocks side by side (bitwise the same)
+  const uint16_t *xe = x + (size_t)(M - 1) * ldx + C, *oe = out + (size_t)(M - 1) * ldo + C;
+  if (M > kTokBlock && M <= 65535 * kTokBlock && !parent && !window && (oe <= x || xe <= out)) {
+    hipLaunchKernelGGL(conv_silu_rows_kernel<4>, dim3((C + kConvThreads - 1) / kConvThreads, (M + kTokBlock - 1) / kTokBlock),
+                       dim3(kConvThreads), 0, (hipStream_t)stream, x, ldx, M, C, conv_state, weight, out, ldo);
+    return skinny_check_launch("gdn_conv");
+  }
   hipLaunchKernelGGL(conv_silu_kernel<4>, dim3((C + kConvThreads - 1) / kConvThreads), dim3(kConvThreads), 0,
                      (hipStream_t)stream, x, ldx, M, C, conv_state, weight, out, ldo, window, parent);
   return skinny_check_launch("gdn_conv");
@@ -608,7 +686,8 @@ extern "C" int skinny_gdn_recurrence(const uint16_t* qkv, int ldq, const uint16_
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)snap_bytes);
     if (e != hipSuccess) return skinny_set_error(SKINNY_ELAUNCH, "gdn: %zu bytes of snapshots: %s", snap_bytes, hipGetErrorString(e));
   }
-  hipLaunchKernelGGL(parent ? gdn_kernel<true> : gdn_kernel<false>, dim3(H, kDv / kCols), dim3(kGdnThreads), snap_bytes,
+  const auto kern = parent ? gdn_kernel<true, false> : M > kTokBlock ? gdn_kernel<false, true> : gdn_kernel<false, false>;
+  hipLaunchKernelGGL(kern, dim3(H, kDv / kCols), dim3(kGdnThreads), snap_bytes,
                      (hipStream_t)stream, qkv, ldq, b, a, ldab, A_log, dt_bias, state, states_out, y, parent, M, H,
                      record, Hk);
   return skinny_check_launch("gdn");

@@ -219,10 +219,6 @@ __device__ __forceinline__ void compute(const XStage& xs, const WStage<RF>& ws, 
   }
 }
 
-// LDS writes of this wave complete, then every wave of the workgroup meets. Global loads
-// still in flight are not waited for (unlike __syncthreads()).
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // ---------------------------------------------------------------------------------------------
 // RF row tiles per wave; SK waves per workgroup split the K/128 group pairs as
 // evenly as possible (wave w owns [w*GP/SK, (w+1)*GP/SK)). Each wave streams its pairs through

@@ -24,8 +24,6 @@ namespace {
 
 enum RowsEpi { kRowsPlain = 0, kRowsGluSplit = 1, kRowsSwiGlu = 2 };
 
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // X of one pair for this wave's share of the 16 MT rows: fragment f = 4 mt + 2 j + h of the pair (lane
 // 16 quad + tok: row 16 mt + tok, columns 64 j + 32 h + 8 quad ..), MT fragments per wave.
 template <int MT>

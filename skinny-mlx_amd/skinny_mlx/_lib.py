@@ -90,6 +90,15 @@ SIGNATURES: dict[str, tuple] = {
     "skinny_attn_workspace_bytes": (_c_size_t, [_c_int, _c_int]),
     "skinny_attention_bf16": (_c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_int,
                                        _c_void_p, _c_float, _c_void_p, _c_void_p, _c_size_t, _c_void_p, _c_void_p]),
+    "skinny_attn_prompt_workspace_bytes": (_c_size_t, [_c_int, _c_int, _c_int, _c_int]),
+    "skinny_attention_prompt_bf16": (_c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p,
+                                              _c_float, _c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_void_p,
+                                              _c_int, _c_float, _c_void_p, _c_size_t, _c_void_p, _c_void_p]),
+    "skinny_attn_general_prompt_workspace_bytes": (_c_size_t, [_c_int, _c_int, _c_int, _c_int, _c_int]),
+    "skinny_attention_general_prompt_bf16": (
+        _c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p,
+                 _c_float, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_float,
+                 _c_void_p, _c_size_t, _c_void_p, _c_void_p]),
     "skinny_kv_commit": (_c_int, [_c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                                   _c_size_t, _c_void_p]),
     "skinny_gdn_conv_silu": (_c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p,

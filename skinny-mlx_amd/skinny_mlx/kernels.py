@@ -286,6 +286,46 @@ def attention_fused(qkv: torch.Tensor, n_q: int, n_kv: int, head_dim: int, q_nor
     return out
 
 
+def attention_prompt(qkv: torch.Tensor, n_q: int, n_kv: int, head_dim: int, q_norm, k_norm, eps: float,
+                     table: torch.Tensor, pos: torch.Tensor, keys: int, k_cache: torch.Tensor,
+                     vt_cache: torch.Tensor, scale: float) -> torch.Tensor:
+    """attention_fused for a prompt of T tokens, bitwise 16-token steps of it: raw q|k|v rows [T,
+    (Hq+2Hkv)*D] -> [T, Hq*D] bf16; the new keys and values go into the caches. `keys` is the host's
+    count of cached tokens after the call, pos[0] + T."""
+    _bf16_2d(qkv, "qkv")
+    T = qkv.shape[0]
+    L = _lib.lib()
+    out = torch.empty((T, n_q * head_dim), dtype=BF16, device=qkv.device)
+    ws = torch.empty(int(L.skinny_attn_prompt_workspace_bytes(T, n_q, n_kv, keys)), dtype=torch.uint8, device=qkv.device)
+    _lib.check(L.skinny_attention_prompt_bf16(
+        qkv.data_ptr(), qkv.stride(0), T, n_q, n_kv, head_dim, _lib.ptr(q_norm), _lib.ptr(k_norm), eps,
+        table.data_ptr(), table.shape[0], pos.data_ptr(), keys, k_cache.data_ptr(), vt_cache.data_ptr(),
+        k_cache.shape[1], scale, ws.data_ptr(), ws.numel(), out.data_ptr(), _lib.stream_of(qkv)), "attention_prompt")
+    return out
+
+
+def attention_general_prompt(qkv: torch.Tensor, n_q: int, n_kv: int, head_dim: int, q_stride: int, k_offset: int,
+                             v_offset: int, gate_offset: int | None, q_norm, k_norm, eps: float, rotary_dim: int,
+                             table: torch.Tensor, pos: torch.Tensor, keys: int, k_cache: torch.Tensor,
+                             vt_cache: torch.Tensor, scale: float) -> torch.Tensor:
+    """attention_general for a prompt of T tokens (see attention_prompt), bitwise 16-token steps of it."""
+    _bf16_2d(qkv, "qkv")
+    T = qkv.shape[0]
+    _req(table.dim() == 3 and table.shape[1] * 2 == rotary_dim and table.dtype == torch.float32,
+         f"table must be a rope_table_dim table for rotary_dim={rotary_dim}")
+    L = _lib.lib()
+    out = torch.empty((T, n_q * head_dim), dtype=BF16, device=qkv.device)
+    ws = torch.empty(int(L.skinny_attn_general_prompt_workspace_bytes(T, n_q, n_kv, head_dim, keys)), dtype=torch.uint8,
+                     device=qkv.device)
+    _lib.check(L.skinny_attention_general_prompt_bf16(
+        qkv.data_ptr(), qkv.stride(0), T, n_q, n_kv, head_dim, q_stride, k_offset, v_offset,
+        -1 if gate_offset is None else gate_offset, _lib.ptr(q_norm), _lib.ptr(k_norm), eps, rotary_dim,
+        table.data_ptr(), table.shape[0], pos.data_ptr(), keys, k_cache.data_ptr(), vt_cache.data_ptr(),
+        k_cache.shape[1], scale, ws.data_ptr(), ws.numel(), out.data_ptr(), _lib.stream_of(qkv)),
+        "attention_general_prompt")
+    return out
+
+
 _QKV_ATTN_OK: dict = {}
 
 

@@ -29,7 +29,12 @@ from . import kernels as K
 from .cache import ArraysCache, KVCache, PromptCache
 from .qmm import GROUP, random_w4g64
 
-MAX_STEP = 16  # tokens per forward pass (longer inputs are processed in pieces)
+MAX_STEP = 16  # tokens per step (longer inputs: pieces of this size, or Model._prompt)
+# Inputs of at least PROMPT_MIN tokens run through the many-row kernels in blocks of up to PROMPT_BLOCK
+# tokens (Model._prompt; five 16-token passes and a capture cost about 14 ms on the 36-layer decoders, one
+# block of 80 tokens 4-5 ms).
+PROMPT_MIN = 80
+PROMPT_BLOCK = 1024
 # Forwards of at most this many tokens form each RMSNorm inside the fused projection after it (its
 # norm-in form: every workgroup repeats the norm, which for one token costs less than a launch).
 FOLD_TOKENS = 1
@@ -239,6 +244,23 @@ class Attention(nn.Module):
         return residual_out(self.o_proj, o)
 
 
+    def prompt(self, x: torch.Tensor, cache: KVCache, keys: int) -> torch.Tensor:
+        """forward over a prompt's rows (more than MAX_STEP tokens), bitwise 16-token steps of it; the
+        residual comes summed. `keys` = cached tokens after the call."""
+        a, sh = self.a, cache.shared
+        Hq, Hkv, D = a.num_attention_heads, a.num_key_value_heads, a.head_dim
+        qkv = joined([self.q_proj(x), self.k_proj(x), self.v_proj(x)])
+        if a.general_attention:
+            qs = 2 * D if a.attn_output_gate else D
+            o = K.attention_general_prompt(qkv, Hq, Hkv, D, qs, Hq * qs, Hq * qs + Hkv * D,
+                                           D if a.attn_output_gate else None, self.q_norm, self.k_norm, a.rms_norm_eps,
+                                           a.rotary_dim, sh.rope, sh.pos, keys, cache.k, cache.vt, D ** -0.5)
+        else:
+            o = K.attention_prompt(qkv, Hq, Hkv, D, self.q_norm, self.k_norm, a.rms_norm_eps, sh.rope, sh.pos, keys,
+                                   cache.k, cache.vt, D ** -0.5)
+        return self.o_proj.prompt_residual(o)
+
+
 class GatedDeltaNet(nn.Module):
     def __init__(self, a: ModelArgs, g: torch.Generator, dev, recorder: "Recorder"):
         super().__init__()
@@ -316,6 +338,25 @@ class GatedDeltaNet(nn.Module):
         return residual_out(self.out_proj, o)
 
 
+    def prompt(self, x: torch.Tensor, cache: ArraysCache) -> torch.Tensor:
+        """forward over a prompt's rows (more than MAX_STEP tokens, nothing recorded), bitwise 16-token
+        steps of it; the residual comes summed."""
+        a = self.a
+        members = (self.in_proj_qkv, self.in_proj_z, self.in_proj_b, self.in_proj_a)
+        proj = getattr(self.in_proj_qkv, "projection", None)
+        y = None
+        if (self.fuse_conv and proj is not None and all(getattr(m, "projection", None) is proj for m in members)
+                and self.in_proj_qkv.columns == slice(0, self.conv_dim)):
+            y = proj.conv_product(x)
+        qkv, z, b, ag = (y[:, m.columns] for m in members) if y is not None else (m(x) for m in members)
+        if b.stride(0) != ag.stride(0):
+            b, ag = b.contiguous(), ag.contiguous()
+        xc = K.gdn_conv_silu(qkv, cache.conv_state, self.conv1d_weight, None)
+        r = K.gdn_recurrence(xc, b, ag, self.A_log, self.dt_bias, cache.state, None, a.linear_num_heads,
+                             a.linear_key_head_dim, a.linear_value_head_dim, None, None, a.gdn_key_heads)
+        return self.out_proj.prompt_residual(K.gated_rmsnorm(r, z, self.norm_weight, a.rms_norm_eps))
+
+
 def swiglu(gate: nn.Module, up: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """silu(gate(x)) * up(x). When both are slices of one fused gate|up projection (see
     skinny_mlx.patch), its matmul applies the activation in the same launch."""
@@ -347,6 +388,10 @@ class MLP(nn.Module):
             if r is not None:
                 return r
         return residual_out(self.down_proj, swiglu(self.gate_proj, self.up_proj, x))
+
+    def prompt(self, x: torch.Tensor) -> torch.Tensor:
+        """forward over a prompt's rows (more than MAX_STEP tokens), the residual summed."""
+        return self.down_proj.prompt_residual(swiglu(self.gate_proj, self.up_proj, x))
 
 
 class DecoderLayer(nn.Module):
@@ -411,7 +456,8 @@ class Model(nn.Module):
 
     def hidden(self, ids, cache: PromptCache, tree=None) -> torch.Tensor:
         """Final normed hidden states of the tokens `ids`, appended to `cache`. Inputs longer
-        than MAX_STEP tokens run as consecutive pieces (each a full pass over the layers).
+        than MAX_STEP tokens run as consecutive pieces (each a full pass over the layers), or, of
+        PROMPT_MIN tokens and more on a patched model, through the many-row kernels with the same bits.
         `tree` (skinny_mlx.tree.DraftTree) makes the tokens a draft tree instead of a chain."""
         ids = self._ids(ids)
         T = ids.shape[0]
@@ -420,7 +466,7 @@ class Model(nn.Module):
         if T > MAX_STEP:
             if self.recorder.recording or tree is not None:
                 raise ValueError("a recording or draft-tree forward takes at most MAX_STEP tokens")
-            return self._pieces(ids, cache)
+            return self._prompt(ids, cache) if T >= PROMPT_MIN and self._prompt_ok(ids) else self._pieces(ids, cache)
         a = self.args
         eps = a.rms_norm_eps
         cache.begin_step(T)
@@ -453,6 +499,44 @@ class Model(nn.Module):
         if self.recorder.recording and cache.shared.gdn is not None:
             cache.shared.gdn.recorded = T
         return out
+
+    def _prompt_ok(self, ids: torch.Tensor) -> bool:
+        """Whether long inputs take the many-row kernels: on the GPU, outside a capture (the attention's grid
+        follows the host's cache length), every linear of the layers patched, at most 4 query heads per
+        kv head (16 tokens x 4 heads fill a chunk's 64 query rows)."""
+        a = self.args
+        return (ids.is_cuda and a.num_attention_heads <= 4 * a.num_key_value_heads
+                and not torch.cuda.is_current_stream_capturing()
+                and not any(isinstance(m, QuantizedLinear) for m in self.layers.modules()))
+
+    def _prompt(self, ids: torch.Tensor, cache: PromptCache) -> torch.Tensor:
+        """A long input in blocks of up to PROMPT_BLOCK tokens, each weight read once per block of rows:
+        bitwise the 16-token passes of _pieces (every kernel keeps a row's sums whatever shares the call;
+        the 509-token prompt of the 36-layer hybrid decoder took 62.9 ms in 32 passes)."""
+        eps = self.args.rms_norm_eps
+        T = ids.shape[0]
+        outs = []
+        i = 0
+        while i < T:
+            # a last block too short for the many-row kernels' route runs as steps
+            n = min(PROMPT_BLOCK, T - i)
+            if n <= MAX_STEP:
+                outs.append(self.hidden(ids[i:i + n], cache))
+                break
+            cache.begin_step(n)
+            keys = cache.attention_offset() + n
+            h = K.embed(ids[i:i + n], self.embed_tokens)
+            r = None
+            for layer, c in zip(self.layers, cache):
+                x = K.rmsnorm(h, layer.input_layernorm, eps, residual=r, sum_out=None if r is None else h)
+                r = layer.linear_attn.prompt(x, c) if layer.is_linear else layer.self_attn.prompt(x, c, keys)
+                x = K.rmsnorm(h, layer.post_attention_layernorm, eps, residual=r, sum_out=h)
+                r = layer.mlp.prompt(x)
+            outs.append(K.rmsnorm(h, self.norm, eps, residual=r, sum_out=h))
+            cache.advance(n)
+            cache.end_step(n)
+            i += n
+        return outs[0] if len(outs) == 1 else torch.cat(outs)
 
     def _pieces(self, ids: torch.Tensor, cache: PromptCache) -> torch.Tensor:
         """A long input as consecutive MAX_STEP-token passes. With four or more full pieces on the

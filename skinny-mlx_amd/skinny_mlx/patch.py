@@ -37,7 +37,7 @@ from .model import QuantizedLinear
 from .qmm import (GROUP, MAX_M, NORMIN_CONV, NORMIN_PLAIN, NORMIN_SWIGLU, gated_partial_supported, mlp_fused_buffers,
                   mlp_fused_supported, normin_supported, packed_k, repack_for_skinny, repack_gate_up, skinny_glu,
                   skinny_glu_normin, skinny_mlp_fused_partial, skinny_qmm, skinny_qmm_conv, skinny_qmm_conv_normin,
-                  skinny_qmm_normin, skinny_qmm_partial, skinny_qmm_partial_gated)
+                  skinny_qmm_normin, skinny_qmm_partial, skinny_qmm_partial_gated, skinny_qmm_rows)
 
 SKINNY_RANGE = (1, 16)
 # Token counts up to which a fused projection forms a kernels.NormIn input in its own launch, per
@@ -98,6 +98,13 @@ class SkinnyQuantizedLinear(nn.Module):
         otherwise the ordinary output."""
         if self.bias is None and x.dim() == 2 and _skinny_ok(_tokens(x)):
             return skinny_qmm_partial(x, self.rweight)
+        return self(x)
+
+    def prompt_residual(self, x: torch.Tensor) -> torch.Tensor:
+        """partial's output summed and rounded (what the residual norm makes of the slices, bitwise),
+        for a prompt's rows (more than MAX_M)."""
+        if self.bias is None and _skinny_ok(_tokens(x)):
+            return skinny_qmm_rows(x, self.rweight, "partial")
         return self(x)
 
     def partial_gated(self, y: torch.Tensor, z: torch.Tensor, norm_w: torch.Tensor, eps: float):
@@ -180,6 +187,13 @@ class _Projection:
                 return skinny_qmm_conv_normin(x, self.packed, c, conv_state, conv_w, window, parent)
             x = x.value()
         return skinny_qmm_conv(x, self.packed, c, conv_state, conv_w, window, parent)
+
+    def conv_product(self, x: torch.Tensor):
+        """conv_output's product before the conv (bitwise), for a prompt's rows (more than MAX_M), or None
+        where conv_output does not apply."""
+        if self.gate_up or not _skinny_ok(_tokens(x)):
+            return None
+        return skinny_qmm_rows(x, self.packed, "conv")
 
     def attention_output(self, x, attn: dict):
         """The attention over this q|k|v projection's rows in one launch with the projection

@@ -1,0 +1,161 @@
+"""Prompts through the many-row kernels (Model._prompt) are bitwise the 16-token passes they replace:
+hidden states, logits, keys, values and Gated-DeltaNet states, at lengths that end inside a 16-token piece, a
+64-token group and a 128-key chunk, from an empty cache and after cached tokens; and the prompt kernels
+alone, with workspaces that take several launches."""
+
+import pytest
+import torch
+
+from skinny_mlx import kernels as K
+from skinny_mlx import patch as P
+from skinny_mlx.cache import make_prompt_cache
+from skinny_mlx.model import PROMPT_MIN, build_model
+from skinny_mlx.spec import forward
+
+pytestmark = pytest.mark.gpu
+
+
+# the small decoders with Gated-DeltaNet heads enough for every linear to be patched (16 rows of b and a)
+SMALL = {"tiny-dense": {}, "tiny-hybrid": dict(linear_num_heads=16),
+         "tiny-qwen35": dict(linear_num_heads=16, linear_num_key_heads=8)}
+
+
+def _model(preset):
+    model = build_model(preset, **SMALL[preset])
+    P.patch_model(model)
+    return model
+
+
+def _state(cache, t):
+    sh = cache.shared
+    out = [sh.k_all[:, :, :t], sh.vt_all[..., :t]]
+    if sh.gdn is not None:
+        out += [sh.gdn.state, sh.gdn.conv]
+    return out
+
+
+@pytest.mark.parametrize("preset", list(SMALL))
+@pytest.mark.parametrize("t,before", [(80, 0), (129, 0), (143, 17), (333, 100)])
+def test_prompt_equals_pieces(preset, t, before):
+    model = _model(preset)
+    assert t >= PROMPT_MIN and model._prompt_ok(model._ids([0]))
+    ids = torch.randint(0, model.args.vocab_size, (before + t,), generator=torch.Generator().manual_seed(t)).tolist()
+    c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
+    for c in (c1, c2):
+        if before:
+            forward(model, ids[:before], c)
+    h1, l1 = forward(model, ids[before:], c1)
+    assert getattr(c1, "_piece_step", None) is None
+    h2 = model._pieces(model._ids(ids[before:]), c2)
+    assert torch.equal(h1, h2) and torch.equal(l1, torch.cat([model.logits(h2[i:i + 16]) for i in range(0, t, 16)]))
+    for a, b in zip(_state(c1, before + t), _state(c2, before + t)):
+        assert torch.equal(a, b)
+    # both caches go on alike
+    assert c1.attention_offset() == c2.attention_offset() == before + t
+    assert torch.equal(forward(model, [7], c1)[1], forward(model, [7], c2)[1])
+
+
+def test_prompt_blocks_and_short_tail(monkeypatch):
+    import skinny_mlx.model as M
+
+    monkeypatch.setattr(M, "PROMPT_BLOCK", 96)
+    model = _model("tiny-hybrid")
+    ids = torch.randint(0, model.args.vocab_size, (96 + 96 + 9,), generator=torch.Generator().manual_seed(2)).tolist()
+    c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
+    h1, _ = forward(model, ids, c1)
+    assert torch.equal(h1, model._pieces(model._ids(ids), c2))
+    for a, b in zip(_state(c1, len(ids)), _state(c2, len(ids))):
+        assert torch.equal(a, b)
+
+
+def test_unpatched_and_captured_inputs_keep_the_pieces():
+    model = build_model("tiny-dense")
+    ids = model._ids(list(range(100)))
+    assert not model._prompt_ok(ids)
+    P.patch_model(model)
+    assert model._prompt_ok(ids) and not model._prompt_ok(ids.cpu())
+    hybrid = build_model("tiny-hybrid")  # 2 rows of b and a: those linears stay unpatched
+    P.patch_model(hybrid)
+    assert not hybrid._prompt_ok(ids)
+
+
+@pytest.mark.parametrize("maxlen,past", [(1024, 0), (1024, 250), (8192, 4300)])  # one- and four-wave merges
+@pytest.mark.parametrize("layout", ["dense", "general"])
+def test_prompt_attention_equals_steps(dev, layout, maxlen, past):
+    hq, hkv, d = (8, 2, 128) if layout == "dense" else (4, 1, 256)
+    t = 150
+    g = torch.Generator(device=dev).manual_seed(maxlen + past)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev).to(torch.bfloat16)
+    cols = (hq + 2 * hkv) * d if layout == "dense" else (2 * hq + 2 * hkv) * d
+    qkv, k0, v0, qn, kn = rnd(t, cols), rnd(hkv, maxlen, d), rnd(hkv, d, maxlen), rnd(d), rnd(d)
+    pos = torch.tensor([past], dtype=torch.int32, device=dev)
+    res = []
+    for prompt in (True, False):
+        k, vt = k0.clone(), v0.clone()
+        if layout == "dense":
+            table = K.rope_table(1e6, maxlen, dev)
+            if prompt:
+                o = K.attention_prompt(qkv, hq, hkv, d, qn, kn, 1e-6, table, pos, past + t, k, vt, d ** -0.5)
+            else:
+                ws = K.attn_workspace(hkv, maxlen, dev)
+                o = torch.cat([K.attention_fused(qkv[i:i + 16], hq, hkv, d, qn, kn, 1e-6, table, pos + i, k, vt, d ** -0.5, ws)
+                               for i in range(0, t, 16)])
+        else:
+            table = K.rope_table_dim(1e7, 64, maxlen, dev)
+            args = (hq, hkv, d, 2 * d, 2 * hq * d, 2 * hq * d + hkv * d, d, qn, kn, 1e-6, 64, table)
+            if prompt:
+                o = K.attention_general_prompt(qkv, *args, pos, past + t, k, vt, d ** -0.5)
+            else:
+                ws = K.attn_general_workspace(hq, hkv, d, maxlen, dev)
+                o = torch.cat([K.attention_general(qkv[i:i + 16], *args, pos + i, k, vt, d ** -0.5, ws)
+                               for i in range(0, t, 16)])
+        res.append((o, k, vt))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
+def test_prompt_attention_in_several_launches(dev):
+    """A workspace of one group of pieces (four) instead of all ten: three launches, the same bits."""
+    from skinny_mlx import _lib
+
+    hq, hkv, d, t, maxlen, past = 8, 2, 128, 150, 512, 130
+    g = torch.Generator(device=dev).manual_seed(5)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev).to(torch.bfloat16)
+    qkv, k0, v0 = rnd(t, (hq + 2 * hkv) * d), rnd(hkv, maxlen, d), rnd(hkv, d, maxlen)
+    pos = torch.tensor([past], dtype=torch.int32, device=dev)
+    table = K.rope_table(1e6, maxlen, dev)
+    k, vt = k0.clone(), v0.clone()
+    ref = K.attention_prompt(qkv, hq, hkv, d, None, None, 1e-6, table, pos, past + t, k, vt, d ** -0.5)
+    L = _lib.lib()
+    one = int(L.skinny_attn_prompt_workspace_bytes(t, hq, hkv, past + t))
+    query = ((t * hq * d * 2) + 255) // 256 * 256
+    ws = torch.empty(query + (one - query) * 4 // 10, dtype=torch.uint8, device=dev)
+    out, k2, vt2 = torch.empty_like(ref), k0.clone(), v0.clone()
+    _lib.check(L.skinny_attention_prompt_bf16(
+        qkv.data_ptr(), qkv.stride(0), t, hq, hkv, d, None, None, 1e-6, table.data_ptr(), maxlen, pos.data_ptr(), past + t,
+        k2.data_ptr(), vt2.data_ptr(), maxlen, d ** -0.5, ws.data_ptr(), ws.numel(), out.data_ptr(),
+        _lib.stream_of(qkv)), "prompt")
+    assert torch.equal(out, ref) and torch.equal(k2, k) and torch.equal(vt2, vt)
+
+
+@pytest.mark.parametrize("h,hk", [(4, 4), (4, 2)])
+@pytest.mark.parametrize("t", [17, 33, 130])
+def test_long_conv_and_recurrence_equal_blocks(dev, h, hk, t):
+    c = 2 * hk * 128 + h * 128
+    g = torch.Generator(device=dev).manual_seed(t + h)
+    x = torch.randn((t, c), generator=g, device=dev).to(torch.bfloat16)
+    ab = torch.randn((t, 2 * h), generator=g, device=dev).to(torch.bfloat16)
+    w = torch.randn((c, 4), generator=g, device=dev).to(torch.bfloat16)
+    A, dtb = torch.rand((h,), generator=g, device=dev), torch.rand((h,), generator=g, device=dev)
+    conv0 = torch.randn((3, c), generator=g, device=dev).to(torch.bfloat16)
+    s0 = torch.randn((h, 128, 128), generator=g, device=dev) * 0.1
+    res = []
+    for step in (t, 16):
+        conv, s, xs, ys = conv0.clone(), s0.clone(), [], []
+        for i in range(0, t, step):
+            xs.append(K.gdn_conv_silu(x[i:i + step], conv, w, None))
+            ys.append(K.gdn_recurrence(xs[-1], ab[i:i + step, :h], ab[i:i + step, h:], A, dtb, s, None, h, 128, 128,
+                                       n_key_heads=hk))
+        res.append((torch.cat(xs), torch.cat(ys), conv, s))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
