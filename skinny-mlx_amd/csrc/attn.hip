@@ -80,6 +80,117 @@ __global__ __launch_bounds__(64 * kWaves) void attn_chunk_kernel(const int32_t* 
                           part_ml, nchunk_max);
 }
 
+// The fused chunk stage of a step of at most 16 query rows per kv head (one token, or a short draft):
+// there only one wave of a chunk's workgroup has rows, so instead of staging the chunk in LDS for four,
+// each wave takes a chunk of its own, its K and V^T fragments straight from memory into registers (the
+// same fragments, MFMAs and softmax, so the partials are bitwise attn_chunk_body's). Nothing waits at a
+// barrier, and a CU holds 8 chunks' loads in flight instead of 2. Only chunks without new tokens are taken
+// this way: workgroups 0 and 1 of a head run attn_chunk_body over the chunks that hold the new slots,
+// workgroup 2 + g the chunks g * per .. below them, one per wave (per = 1 keeps a short context's chunks
+// on CUs of their own). What bounds it at a long context is the read of K and V^T; at a short one the chain
+// position, chunk, partial, merge. Measured on MI355X, one token, chunk stage and merge of a layer: 32768 keys
+// 41.6 -> 36.7 us (3.66 TB/s of KV; with it, partials of the live rows only and eight merge waves); 2048 keys
+// level (9.8 us); 256-dim heads (general_few_kernel) 512 / 2000 / 5003 keys 10.6 / 11.9 / 16.6 -> 10.5 / 11.5 /
+// 15.2 us. With more rows per kv head several waves of a staged chunk have work, and staging serves them all.
+constexpr int kFewRows = 16;
+constexpr int kFewMaxlen = 1 << 22;  // V^T of a head within a buffer descriptor
+
+__device__ __forceinline__ void attn_direct_chunk(int c, int h, int p0, const uint16_t* __restrict__ q, const FusedArgs& fa,
+                                                  int M, int Hq, int Hkv, const uint16_t* __restrict__ kc,
+                                                  const uint16_t* __restrict__ vt, int maxlen, float scale,
+                                                  const int32_t* __restrict__ tree, float* __restrict__ part_o,
+                                                  float* __restrict__ part_ml, int nchunk_max) {
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  const int G = Hq / Hkv, rows = G * M, key0 = c * kChunk;
+  const bool live = col < rows;
+  const int t = live ? col / G : 0, qg = live ? col % G : 0;
+  // The query side first, then K and V^T: buffer loads whose lane offset is fixed, the tile's in an SGPR.
+  const uint16_t* qr = q + (size_t)t * fa.ldq + ((size_t)h * G + qg) * kD;
+  const uint16_t* qn = fa.qn ? fa.qn : qr;
+  const int pos = p0 + (tree ? tree[1 + M + t] : t);
+  u32x4_t raw[4], wq[4];
+  f32x4_t cs[2][4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    raw[ks] = *reinterpret_cast<const u32x4_t*>(qr + ks * 32 + quad * 8);
+    wq[ks] = *reinterpret_cast<const u32x4_t*>(qn + ks * 32 + quad * 8);
+  }
+  const f32x4_t* rp = reinterpret_cast<const f32x4_t*>(fa.rope + (size_t)pos * 128);
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cs[ks][j] = rp[(ks * 32 + quad * 8) / 2 + j];
+  int tbase = key0;
+  uint32_t tmask = 0;
+  const int tree0 = tree ? tree[0] : 0;
+  const uint32_t mask = tree ? (uint32_t)tree[1 + t] : 0u;
+  if (live) {
+    tbase = tree ? p0 - tree0 : p0 + t + 1;
+    tmask = mask;
+  }
+  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(kc) + ((size_t)h * maxlen + key0) * kD, (short)0, kChunk * kD * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(vt) + (size_t)h * kD * maxlen + key0, (short)0, ((kD - 1) * maxlen + kChunk) * 2, 0x00020000);
+  const uint32_t koff = (uint32_t)((8 * (col >> 2) + (col & 3)) * kD + quad * 8) * 2u;
+  const uint32_t voff = (uint32_t)(col * maxlen + quad * 8) * 2u;
+  bf16x8_t kf[8][4], vf[8][4];
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt)
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      kf[kt][ks] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                    rk, koff, ((32 * (kt >> 1) + 4 * (kt & 1)) * kD + ks * 32) * 2, 0));
+  bf16x8_t qf[4] = {};
+  if (live) rotate_query(raw, wq, cs, fa.qn != nullptr, fa.eps, qf);
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  float s[8][4];
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt) {
+    f32x4_t acc = zero;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) acc = mfma16x16x32(kf[kt][ks], qf[ks], acc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
+    // the V^T fragments follow the K tiles into flight, in the registers those leave
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      vf[kt][ks] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rv, voff, (kt * 16 * maxlen + ks * 32) * 2, 0));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  u32x4_t pa[4];
+  float mx, sum;
+  attn_softmax(s, key0, tbase, tmask, scale, pa, mx, sum);
+  f32x4_t o[8];
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt) {
+    o[dt] = zero;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) o[dt] = mfma16x16x32(__builtin_bit_cast(bf16x8_t, pa[ks]), vf[dt][ks], o[dt]);
+  }
+  const size_t base = ((size_t)h * nchunk_max + c) * kRowsMax;
+  attn_store_rows(o, mx, sum, rows, part_o + base * kD, part_ml + base * 2);
+}
+
+__global__ __launch_bounds__(64 * kWaves) void attn_few_kernel(const int32_t* __restrict__ pos0,
+                                                               const uint16_t* __restrict__ q, FusedArgs fa, int M, int Hq,
+                                                               int Hkv, uint16_t* __restrict__ kc, uint16_t* __restrict__ vt,
+                                                               int maxlen, float scale, const int32_t* __restrict__ tree,
+                                                               float* __restrict__ part_o, float* __restrict__ part_ml,
+                                                               int nchunk_max, int per) {
+  const int b = blockIdx.x, h = blockIdx.y, wave = wave_id();
+  if (b >= 2 && wave >= per) return;
+  const int p0 = pos0[0];
+  const int fresh = p0 / kChunk;  // the first chunk with new slots
+  if (b < 2) {
+    attn_chunk_body<true>(fresh + b, h, pos0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
+    return;
+  }
+  const int c = (b - 2) * per + wave;
+  if (c >= fresh) return;
+  attn_direct_chunk(c, h, p0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
+}
+
 // One workgroup per (q head, token): merge the chunk partials, normalise, store bf16. Chunks are
 // taken in blocks of 32 by absolute index: all of a block's loads are issued together (lane c holds
 // chunk c's statistics, every lane its two dims of every chunk's partial row), then the block is
@@ -90,7 +201,9 @@ __global__ __launch_bounds__(64 * kWaves) void attn_chunk_kernel(const int32_t* 
 // sums in that order, a wave without keys for the row by exactly 1 and 0: W is fixed by the cache
 // size, so every step over one cache merges a row's blocks the same way.
 constexpr int kCombineBlock = 32;
-constexpr int kCombineWaves = 4;  // waves of the merge for caches of more than kCombineBlock chunks
+constexpr int kCombineWaves = 4;      // waves of the merge for caches of more than kCombineBlock chunks
+constexpr int kCombineWavesLong = 8;  // and of more than kCombineLong chunks
+constexpr int kCombineLong = 128;
 
 // The merge of one row (chunk c's partial at head_base + c * kRowsMax; pos0[0] + tokens keys) into
 // dst[128]; false in the waves that only helped. kPrompt reads the chunk count first, since a prompt's
@@ -358,7 +471,7 @@ __global__ __launch_bounds__(64 * kWaves) void prompt_chunk_kernel(const int32_t
     if (key0 >= p0 + t0 + mb || wave * 16 >= G * mb) continue;
     const int tbase = qrow < G * mb ? p0 + t0 + qrow / G + 1 : key0;
     const size_t base = (((size_t)(z - z0) * Hkv + h) * nch + c) * kRowsMax + wave * 16;
-    attn_rows(ks_lds, vs_lds, qf[i], key0, tbase, 0u, scale, part_o + base * kD, part_ml + base * 2);
+    attn_rows(ks_lds, vs_lds, qf[i], key0, tbase, 0u, scale, G * mb - wave * 16, part_o + base * kD, part_ml + base * 2);
   }
 }
 
@@ -392,7 +505,10 @@ __global__ void rope_table_kernel(float theta, int positions, float* __restrict_
 int attn_combine_launch(const float* part_o, const float* part_ml, int M, int Hq, int Hkv, const int32_t* pos0,
                         int nchunk_max, uint16_t* out, uint32_t* reset, int reset_ld, int reset_words,
                         hipStream_t stream) {
-  if (nchunk_max > kCombineBlock)
+  if (nchunk_max > kCombineLong)
+    hipLaunchKernelGGL(attn_combine_kernel<kCombineWavesLong>, dim3(Hq, M), dim3(64 * kCombineWavesLong), 0, stream, part_o,
+                       part_ml, M, Hq, Hkv, pos0, nchunk_max, out, reset, reset_ld, reset_words);
+  else if (nchunk_max > kCombineBlock)
     hipLaunchKernelGGL(attn_combine_kernel<kCombineWaves>, dim3(Hq, M), dim3(64 * kCombineWaves), 0, stream, part_o,
                        part_ml, M, Hq, Hkv, pos0, nchunk_max, out, reset, reset_ld, reset_words);
   else
@@ -479,8 +595,14 @@ static int attention_fused(const uint16_t* qkv, int ldq, int M, int Hq, int Hkv,
   float* part_o = workspace;
   float* part_ml = workspace + (size_t)Hkv * nch * kRowsMax * kD;
   const FusedArgs fa{ldq, q_norm, k_norm, eps, rope_table};
-  hipLaunchKernelGGL(attn_chunk_kernel<true>, dim3(nch, Hkv), dim3(64 * kWaves), 0, (hipStream_t)stream, pos0, qkv, fa, M,
-                     Hq, Hkv, k_cache, vt_cache, maxlen, scale, tree, part_o, part_ml, nch);
+  if ((Hq / Hkv) * M <= kFewRows && maxlen <= kFewMaxlen) {
+    const int per = nch * Hkv <= 512 ? 1 : nch * Hkv <= 1024 ? 2 : kWaves;
+    hipLaunchKernelGGL(attn_few_kernel, dim3(2 + (nch + per - 1) / per, Hkv), dim3(64 * kWaves), 0, (hipStream_t)stream, pos0,
+                       qkv, fa, M, Hq, Hkv, k_cache, vt_cache, maxlen, scale, tree, part_o, part_ml, nch, per);
+  } else {
+    hipLaunchKernelGGL(attn_chunk_kernel<true>, dim3(nch, Hkv), dim3(64 * kWaves), 0, (hipStream_t)stream, pos0, qkv, fa, M,
+                       Hq, Hkv, k_cache, vt_cache, maxlen, scale, tree, part_o, part_ml, nch);
+  }
   int rc = skinny_check_launch("attention");
   if (rc) return rc;
   return attn_combine_launch(part_o, part_ml, M, Hq, Hkv, pos0, nch, out, nullptr, 0, 0, (hipStream_t)stream);
@@ -553,12 +675,12 @@ extern "C" int skinny_attention_prompt_bf16(const uint16_t* qkv, int ldq, int M,
                        pos0, q, M, Hq, Hkv, k_cache, vt_cache, maxlen, scale, z0, z1, nch, part_o, part_ml);
     if (int rc = skinny_check_launch("attention prompt chunks")) return rc;
     // the wave count of the merge goes by the cache size, as in the step kernels
-    if (maxlen / kChunk > kCombineBlock)
-      hipLaunchKernelGGL(prompt_combine_kernel<kCombineWaves>, dim3(Hq, last - z0 * kPiece), dim3(64 * kCombineWaves), 0, s,
-                         part_o, part_ml, M, Hq, Hkv, pos0, z0, nch, out);
-    else
-      hipLaunchKernelGGL(prompt_combine_kernel<1>, dim3(Hq, last - z0 * kPiece), dim3(64), 0, s, part_o, part_ml, M, Hq, Hkv,
-                         pos0, z0, nch, out);
+    const int W = maxlen / kChunk > kCombineLong ? kCombineWavesLong : maxlen / kChunk > kCombineBlock ? kCombineWaves : 1;
+    const auto merge = W == kCombineWavesLong ? prompt_combine_kernel<kCombineWavesLong>
+                       : W == kCombineWaves   ? prompt_combine_kernel<kCombineWaves>
+                                              : prompt_combine_kernel<1>;
+    hipLaunchKernelGGL(merge, dim3(Hq, last - z0 * kPiece), dim3(64 * W), 0, s, part_o, part_ml, M, Hq, Hkv, pos0, z0, nch,
+                       out);
     if (int rc = skinny_check_launch("attention prompt merge")) return rc;
   }
   return SKINNY_OK;

@@ -107,28 +107,12 @@ __device__ __forceinline__ void rotate_query(const u32x4_t (&raw)[4], const u32x
   qf[3] = __builtin_bit_cast(bf16x8_t, hi[1]);
 }
 
-// One wave's 16 query rows against the staged chunk (keys key0 ..): the partial O rows to rows_o
-// [16][128], the row maxima (log2 units) and sums to rows_ml [16][2]. Visibility per lane as the caller
-// set it up: key kp is visible iff kp < tbase, or kp - tbase < 32 and that bit of tmask is set.
-__device__ __forceinline__ void attn_rows(const uint16_t* ks_lds, const uint16_t* vs_lds, const bf16x8_t (&qf)[4], int key0,
-                                          int tbase, uint32_t tmask, float scale, float* __restrict__ rows_o,
-                                          float* __restrict__ rows_ml) {
-  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
-  // 2. S^T tiles: element i of tile kt is the score of key 32(kt/2) + 8quad + 4(kt%2) + i.
-  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
-  float s[8][4];
-#pragma unroll
-  for (int kt = 0; kt < 8; ++kt) {
-    const int krow = 32 * (kt >> 1) + 8 * (col >> 2) + 4 * (kt & 1) + (col & 3);
-    f32x4_t acc = zero;
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
-      acc = mfma16x16x32(*reinterpret_cast<const bf16x8_t*>(&ks_lds[krow * kPitch + ks * 32 + quad * 8]), qf[ks], acc);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
-  }
-
-  // 3. Visibility, the row maximum (log2 units), bf16 P packed as the P.V A operand, its sum.
+// Steps 3 and 5 of a wave's chunk, shared by every form of it. attn_softmax: visibility, the row maximum
+// (log2 units), bf16 P packed as the P.V A operand, its sum; s[kt][i] is the raw score of key key0 + 32(kt/2) +
+// 8quad + 4(kt%2) + i. Key kp is visible iff kp < tbase, or kp - tbase < 32 and that bit of tmask is set.
+__device__ __forceinline__ void attn_softmax(float (&s)[8][4], int key0, int tbase, uint32_t tmask, float scale,
+                                             u32x4_t (&pa)[4], float& row_max, float& row_sum) {
+  const int quad = (threadIdx.x & 63) >> 4;
   const float sc = scale * kLog2e;
   const int kq = key0 + 8 * quad;  // key of element (kt, i) = kq + 32(kt/2) + 4(kt%2) + i
   float mx = -INFINITY;
@@ -144,7 +128,6 @@ __device__ __forceinline__ void attn_rows(const uint16_t* ks_lds, const uint16_t
   mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
   const float mref = mx == -INFINITY ? 0.f : mx;  // a row with no visible key here: every P is 0
-  u32x4_t pa[4];
   float sum = 0.f;
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks)
@@ -159,7 +142,49 @@ __device__ __forceinline__ void attn_rows(const uint16_t* ks_lds, const uint16_t
     }
   sum += __shfl_xor(sum, 16, 64);
   sum += __shfl_xor(sum, 32, 64);
+  row_max = mx;
+  row_sum = sum;
+}
 
+// The chunk partial of the wave's first `rows` rows (the merge reads no others): O rows 4quad + i, dim
+// 16dt + col, to rows_o [16][128]; the row maxima and sums to rows_ml [16][2].
+__device__ __forceinline__ void attn_store_rows(const f32x4_t (&o)[8], float row_max, float row_sum, int rows,
+                                                float* __restrict__ rows_o, float* __restrict__ rows_ml) {
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (quad * 4 + i >= rows) break;
+    float* dst = rows_o + (quad * 4 + i) * kD;
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) dst[dt * 16 + col] = o[dt][i];
+  }
+  if (quad == 0) {
+    rows_ml[col * 2] = row_max;
+    rows_ml[col * 2 + 1] = row_sum;
+  }
+}
+
+// One wave's 16 query rows against the staged chunk (keys key0 ..), visibility as attn_softmax has it.
+__device__ __forceinline__ void attn_rows(const uint16_t* ks_lds, const uint16_t* vs_lds, const bf16x8_t (&qf)[4], int key0,
+                                          int tbase, uint32_t tmask, float scale, int rows, float* __restrict__ rows_o,
+                                          float* __restrict__ rows_ml) {
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  // 2. S^T tiles: element i of tile kt is the score of key 32(kt/2) + 8quad + 4(kt%2) + i.
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  float s[8][4];
+#pragma unroll
+  for (int kt = 0; kt < 8; ++kt) {
+    const int krow = 32 * (kt >> 1) + 8 * (col >> 2) + 4 * (kt & 1) + (col & 3);
+    f32x4_t acc = zero;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+      acc = mfma16x16x32(*reinterpret_cast<const bf16x8_t*>(&ks_lds[krow * kPitch + ks * 32 + quad * 8]), qf[ks], acc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
+  }
+  u32x4_t pa[4];
+  float mx, sum;
+  attn_softmax(s, key0, tbase, tmask, scale, pa, mx, sum);
   // 4. O = P V over the 4 key steps of 32; lane holds O rows 4quad + i, dim 16dt + col.
   f32x4_t o[8];
 #pragma unroll
@@ -172,18 +197,7 @@ __device__ __forceinline__ void attn_rows(const uint16_t* ks_lds, const uint16_t
       o[dt] = mfma16x16x32(pf, *reinterpret_cast<const bf16x8_t*>(&vs_lds[(dt * 16 + col) * kPitch + ks * 32 + quad * 8]),
                            o[dt]);
   }
-
-  // 5. The chunk partial of this wave's rows.
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float* dst = rows_o + (quad * 4 + i) * kD;
-#pragma unroll
-    for (int dt = 0; dt < 8; ++dt) dst[dt * 16 + col] = o[dt][i];
-  }
-  if (quad == 0) {
-    rows_ml[col * 2] = mx;
-    rows_ml[col * 2 + 1] = sum;
-  }
+  attn_store_rows(o, mx, sum, rows, rows_o, rows_ml);
 }
 
 // The body of the chunk kernel for workgroup (chunk c, kv head h), shared by attn_chunk_kernel and
@@ -417,7 +431,7 @@ __device__ __forceinline__ void attn_chunk_body(int c, int h, const int32_t* __r
   if (!busy) return;
 
   const size_t base = ((size_t)h * nchunk_max + c) * kRowsMax + wave * 16;
-  attn_rows(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, part_o + base * kD, part_ml + base * 2);
+  attn_rows(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, rows - wave * 16, part_o + base * kD, part_ml + base * 2);
 }
 
 }  // namespace

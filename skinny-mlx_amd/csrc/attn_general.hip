@@ -74,6 +74,8 @@ __global__ __launch_bounds__(64) void general_qk_store_kernel(const int32_t* __r
   uint16_t raw[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) raw[e] = src[lane + 64 * e];
+  const int half = R >> 1;
+  const uint16_t* nw = head < Hq ? qn : kn;
   if (head >= Hq + Hkv) {  // value: into the transposed cache as it is
     const int h = head - Hq - Hkv;
 #pragma unroll
@@ -87,17 +89,14 @@ __global__ __launch_bounds__(64) void general_qk_store_kernel(const int32_t* __r
     x[e] = bf16_bits_to_f32(raw[e]);
     ss = fmaf(x[e], x[e], ss);
   }
-  const uint16_t* nw = head < Hq ? qn : kn;
   if (nw) {
     const float inv = rsqrtf(wave_sum(ss) / (float)D + eps);
 #pragma unroll
-    for (int e = 0; e < E; ++e)
-      x[e] = bf16_bits_to_f32(f32_to_bf16_bits(x[e] * inv * bf16_bits_to_f32(nw[lane + 64 * e])));
+    for (int e = 0; e < E; ++e) x[e] = bf16_bits_to_f32(f32_to_bf16_bits(x[e] * inv * bf16_bits_to_f32(nw[lane + 64 * e])));
   }
 #pragma unroll
   for (int e = 0; e < E; ++e) row[lane + 64 * e] = x[e];
   __syncthreads();
-  const int half = R >> 1;
   uint16_t outv[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -116,11 +115,71 @@ __global__ __launch_bounds__(64) void general_qk_store_kernel(const int32_t* __r
   for (int e = 0; e < E; ++e) dst[lane + 64 * e] = outv[e];
 }
 
+// A wave's softmax of a chunk and the store of its partial, shared by every form of the chunk stage
+// (attn.hip's attn_softmax and attn_store_rows over D dims): s[kt][i] is the raw score of key key0 +
+// 32(kt/2) + 8quad + 4(kt%2) + i; key kp is visible iff kp < tbase, or kp - tbase < 32 and that bit of
+// tmask is set.
+template <int D>
+__device__ __forceinline__ void general_softmax(float (&s)[general_chunk(D) / 16][4], int key0, int tbase, uint32_t tmask,
+                                                float scale, u32x4_t (&pa)[general_chunk(D) / 32], float& row_max,
+                                                float& row_sum) {
+  constexpr int KT = general_chunk(D) / 16, PS = general_chunk(D) / 32;
+  const int quad = (threadIdx.x & 63) >> 4;
+  const float sc = scale * kGLog2e;
+  const int kq = key0 + 8 * quad;
+  float mx = -INFINITY;
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = kq + 32 * (kt >> 1) + 4 * (kt & 1) + i - tbase;
+      const uint32_t vis = (uint32_t)(j < 0) | ((uint32_t)(j < 32) & (tmask >> (j & 31)));
+      s[kt][i] = (vis & 1u) ? s[kt][i] * sc : -INFINITY;
+      mx = fmaxf(mx, s[kt][i]);
+    }
+  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+  const float mref = mx == -INFINITY ? 0.f : mx;
+  float sum = 0.f;
+#pragma unroll
+  for (int ks = 0; ks < PS; ++ks)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const int kt = 2 * ks + (w >> 1), i = 2 * (w & 1);
+      const uint16_t b0 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i] - mref));
+      const uint16_t b1 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i + 1] - mref));
+      sum += bf16_bits_to_f32(b0);
+      sum += bf16_bits_to_f32(b1);
+      pa[ks][w] = (uint32_t)b0 | ((uint32_t)b1 << 16);
+    }
+  sum += __shfl_xor(sum, 16, 64);
+  sum += __shfl_xor(sum, 32, 64);
+  row_max = mx;
+  row_sum = sum;
+}
+
+template <int D>
+__device__ __forceinline__ void general_store_rows(const f32x4_t (&o)[D / 16], float row_max, float row_sum, int rows,
+                                                   float* __restrict__ rows_o, float* __restrict__ rows_ml) {
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (quad * 4 + i >= rows) break;  // the merge reads no other rows
+    float* dst = rows_o + (quad * 4 + i) * D;
+#pragma unroll
+    for (int dt = 0; dt < D / 16; ++dt) dst[dt * 16 + col] = o[dt][i];
+  }
+  if (quad == 0) {
+    rows_ml[col * 2] = row_max;
+    rows_ml[col * 2 + 1] = row_sum;
+  }
+}
+
 // One wave's 16 query rows against the staged chunk of keys key0 .. (attn.hip's attn_rows over D dims):
 // the partial O rows to rows_o [16][D], the row maxima (log2 units) and sums to rows_ml [16][2].
 template <int D>
 __device__ __forceinline__ void general_rows(const uint16_t* ks_lds, const uint16_t* vs_lds, const bf16x8_t (&qf)[D / 32],
-                                             int key0, int tbase, uint32_t tmask, float scale, float* __restrict__ rows_o,
+                                             int key0, int tbase, uint32_t tmask, float scale, int rows, float* __restrict__ rows_o,
                                              float* __restrict__ rows_ml) {
   constexpr int CH = general_chunk(D);
   constexpr int KS = D / 32;   // 32-dim steps of a score
@@ -141,36 +200,9 @@ __device__ __forceinline__ void general_rows(const uint16_t* ks_lds, const uint1
 #pragma unroll
     for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
   }
-  const float sc = scale * kGLog2e;
-  const int kq = key0 + 8 * quad;
-  float mx = -INFINITY;
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int j = kq + 32 * (kt >> 1) + 4 * (kt & 1) + i - tbase;
-      const uint32_t vis = (uint32_t)(j < 0) | ((uint32_t)(j < 32) & (tmask >> (j & 31)));
-      s[kt][i] = (vis & 1u) ? s[kt][i] * sc : -INFINITY;
-      mx = fmaxf(mx, s[kt][i]);
-    }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-  const float mref = mx == -INFINITY ? 0.f : mx;
   u32x4_t pa[PS];
-  float sum = 0.f;
-#pragma unroll
-  for (int ks = 0; ks < PS; ++ks)
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const int kt = 2 * ks + (w >> 1), i = 2 * (w & 1);
-      const uint16_t b0 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i] - mref));
-      const uint16_t b1 = f32_to_bf16_bits(__builtin_amdgcn_exp2f(s[kt][i + 1] - mref));
-      sum += bf16_bits_to_f32(b0);
-      sum += bf16_bits_to_f32(b1);
-      pa[ks][w] = (uint32_t)b0 | ((uint32_t)b1 << 16);
-    }
-  sum += __shfl_xor(sum, 16, 64);
-  sum += __shfl_xor(sum, 32, 64);
+  float mx, sum;
+  general_softmax<D>(s, key0, tbase, tmask, scale, pa, mx, sum);
   // O = P V: lane holds O rows 4quad + i, dim 16dt + col; V^T row (16dt + col) keys 32ks + 8quad.
   f32x4_t o[DT];
 #pragma unroll
@@ -183,16 +215,91 @@ __device__ __forceinline__ void general_rows(const uint16_t* ks_lds, const uint1
       o[dt] = mfma16x16x32(pf, *reinterpret_cast<const bf16x8_t*>(&vs_lds[(dt * 16 + col) * VP + ks * 32 + quad * 8]),
                            o[dt]);
   }
+  general_store_rows<D>(o, mx, sum, rows, rows_o, rows_ml);
+}
+
+// (2, few rows) A step of at most 16 query rows per kv head: as attn.hip's attn_few_kernel, each wave takes
+// a chunk of its own with its K and V^T fragments straight from memory (the new rows are in the caches
+// already), `per` chunks per workgroup; partials bitwise general_chunk_kernel's.
+constexpr int kGFewRows = 16;
+constexpr int kGFewMaxlen = 1 << 21;  // V^T of a head within a buffer descriptor
+
+template <int D>
+__global__ __launch_bounds__(64 * kGWaves, 2) void general_few_kernel(const int32_t* __restrict__ pos0,
+                                                                      const uint16_t* __restrict__ q, int M, int Hq,
+                                                                      int Hkv, const uint16_t* __restrict__ kc,
+                                                                      const uint16_t* __restrict__ vt, int maxlen,
+                                                                      float scale, const int32_t* __restrict__ tree,
+                                                                      float* __restrict__ part_o,
+                                                                      float* __restrict__ part_ml, int nchunk_max, int per) {
+  constexpr int CH = general_chunk(D);
+  constexpr int KS = D / 32, DT = D / 16, KT = CH / 16, PS = CH / 32;
+  constexpr int VPT = DT * PS / KT;  // V^T fragments issued per K tile
+  const int h = blockIdx.y, wave = wave_id();
+  const int c = (int)blockIdx.x * per + wave;
+  const int p0 = pos0[0];
+  const int key0 = c * CH;
+  if (key0 >= p0 + M) return;
+  const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  const int G = Hq / Hkv;
+  const bool live = col < G * M;
+  const int t = live ? col / G : 0;
+  const uint16_t* qr = q + ((size_t)t * Hq + h * G + (live ? col % G : 0)) * D;
+  bf16x8_t qf[KS];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float* dst = rows_o + (quad * 4 + i) * D;
+  for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8_t*>(qr + ks * 32 + quad * 8);
+  const int tree0 = tree ? tree[0] : 0;
+  const uint32_t mask = tree ? (uint32_t)tree[1 + t] : 0u;
+  const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(kc) + ((size_t)h * maxlen + key0) * D, (short)0, CH * D * 2, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint16_t*>(vt) + (size_t)h * D * maxlen + key0, (short)0, ((D - 1) * maxlen + CH) * 2, 0x00020000);
+  const uint32_t koff = (uint32_t)((8 * (col >> 2) + (col & 3)) * D + quad * 8) * 2u;
+  const uint32_t voff = (uint32_t)(col * maxlen + quad * 8) * 2u;
+  bf16x8_t kf[KT][KS], vf[DT][PS];
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) dst[dt * 16 + col] = o[dt][i];
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      kf[kt][ks] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
+                                                    rk, koff, ((32 * (kt >> 1) + 4 * (kt & 1)) * D + ks * 32) * 2, 0));
+  int tbase = key0;
+  uint32_t tmask = 0;
+  if (live) {
+    tbase = tree ? p0 - tree0 : p0 + t + 1;
+    tmask = mask;
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = bf16x8_t{};
   }
-  if (quad == 0) {
-    rows_ml[col * 2] = mx;
-    rows_ml[col * 2 + 1] = sum;
+  const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+  float s[KT][4];
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) {
+    f32x4_t acc = zero;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) acc = mfma16x16x32(kf[kt][ks], qf[ks], acc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[kt][i] = acc[i];
+    // the V^T fragments follow the K tiles into flight, in the registers those leave
+#pragma unroll
+    for (int v = kt * VPT; v < (kt + 1) * VPT; ++v)
+      vf[v / PS][v % PS] = __builtin_bit_cast(
+          bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rv, voff, ((v / PS) * 16 * maxlen + (v % PS) * 32) * 2, 0));
+    __builtin_amdgcn_sched_barrier(0);
   }
+  u32x4_t pa[PS];
+  float mx, sum;
+  general_softmax<D>(s, key0, tbase, tmask, scale, pa, mx, sum);
+  f32x4_t o[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    o[dt] = zero;
+#pragma unroll
+    for (int ks = 0; ks < PS; ++ks) o[dt] = mfma16x16x32(__builtin_bit_cast(bf16x8_t, pa[ks]), vf[dt][ks], o[dt]);
+  }
+  const size_t base = ((size_t)h * nchunk_max + c) * kGRowsMax;
+  general_store_rows<D>(o, mx, sum, G * M, part_o + base * D, part_ml + base * 2);
 }
 
 // (2) Workgroup (chunk c, kv head h), keys [CH c, CH c + CH); wave w takes the query rows
@@ -273,7 +380,7 @@ __global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32
   if (!busy) return;
 
   const size_t base = ((size_t)h * nchunk_max + c) * kGRowsMax + wave * 16;
-  general_rows<D>(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, part_o + base * D, part_ml + base * 2);
+  general_rows<D>(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, rows - wave * 16, part_o + base * D, part_ml + base * 2);
 }
 
 // (3) One workgroup per (query head, token), max(1, D / 128) waves, lane l of wave w holding dims
@@ -284,12 +391,18 @@ __global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32
 // end repeat its last chunk), all before the first is used; the block is folded into running sums
 // in chunk order, rescaled when the running maximum grows, the weights broadcast by v_readlane.
 // With a gate, out = bf16(bf16(o) * bf16(sigmoid(gate))).
+//
+// W > 1 (caches of more than one block): W such groups of waves, group v folding blocks v, v + W, ... into sums
+// of its own, group 0 then folding the others' in order, as attn_combine_kernel's waves do; W goes by the cache
+// size alone. At 5003 keys of 256-dim heads, 79 chunks: 6.7 us with one group, two blocks in a row.
+constexpr int kGCombineGroups = 4;
+
 template <int D>
 constexpr int general_combine_waves() { return D > 128 ? D / 128 : 1; }
 
 // (chunk c's partial row at head_base + c * kGRowsMax; pos0[0] + tokens keys; gate_at(): the row's gate
 // values or NULL, and out_at(): its output, asked for last, since their arguments lie past the preloaded ones)
-template <int D, typename GateAt, typename OutAt>
+template <int D, int W, typename GateAt, typename OutAt>
 __device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ pos0, const float* __restrict__ part_o,
                                                     const float* __restrict__ part_ml, size_t head_base, int tokens,
                                                     int nchunk_max, GateAt gate_at, OutAt out_at) {
@@ -298,12 +411,15 @@ __device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ 
   constexpr int CW = D / 64 / general_combine_waves<D>();  // dims per lane: 1 or 2
   typedef __attribute__((ext_vector_type(CW))) float dims_t;
   const int lane = threadIdx.x & 63;
-  const int d0 = (int)threadIdx.x * CW;  // this lane's first dim
+  constexpr int DW = general_combine_waves<D>();
+  const int v = W > 1 ? wave_id() / DW : 0;                     // this wave group's first block of chunks
+  const int td = (int)threadIdx.x - v * 64 * DW;                // thread within the group
+  const int d0 = td * CW;                                       // this lane's first dim
   const int nch = min((pos0[0] + tokens + CH - 1) / CH, nchunk_max);
   float run_m = -INFINITY, run_l = 0.f, a[CW];
 #pragma unroll
   for (int k = 0; k < CW; ++k) a[k] = 0.f;
-  for (int c0 = 0; c0 < nch; c0 += B) {
+  for (int c0 = v * B; c0 < nch; c0 += W * B) {
     const int nb = min(B, nch - c0);
     const size_t es = head_base + (size_t)(c0 + min(lane, nb - 1)) * kGRowsMax;
     float mc = part_ml[es * 2], lc = part_ml[es * 2 + 1];
@@ -338,6 +454,28 @@ __device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ 
     }
     run_m = new_m;
   }
+  if constexpr (W > 1) {  // group 0 folds the others' sums in their order
+    __shared__ float sm[W], sl[W], sa[W][64 * DW][CW];
+    if (td == 0) {
+      sm[v] = run_m;
+      sl[v] = run_l;
+    }
+#pragma unroll
+    for (int k = 0; k < CW; ++k) sa[v][td][k] = a[k];
+    __syncthreads();
+    if (v > 0) return;
+#pragma unroll
+    for (int u = 1; u < W; ++u) {
+      const float mu = sm[u], lu = sl[u];
+      const float new_m = fmaxf(run_m, mu);
+      const float k0 = run_m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(run_m - new_m);
+      const float ku = mu == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mu - new_m);
+      run_l = fmaf(lu, ku, run_l * k0);
+#pragma unroll
+      for (int k = 0; k < CW; ++k) a[k] = fmaf(sa[u][td][k], ku, a[k] * k0);
+      run_m = new_m;
+    }
+  }
   const float inv = run_l > 0.f ? 1.0f / run_l : 0.f;
   const uint16_t* gate = gate_at();
   uint16_t* dst = out_at() + d0;
@@ -354,13 +492,13 @@ __device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ 
   }
 }
 
-template <int D>
-__global__ __launch_bounds__(64 * general_combine_waves<D>()) void general_combine_kernel(
+template <int D, int W>
+__global__ __launch_bounds__(64 * general_combine_waves<D>() * W) void general_combine_kernel(
     const int32_t* __restrict__ pos0, const float* __restrict__ part_o, const float* __restrict__ part_ml, int M,
     int Hq, int Hkv, int nchunk_max, const uint16_t* __restrict__ qkv, HeadLayout hl, uint16_t* __restrict__ out) {
   const int hq = blockIdx.x, t = blockIdx.y;
   const int G = Hq / Hkv, h = hq / G, row = t * G + hq % G;
-  general_combine_row<D>(
+  general_combine_row<D, W>(
       pos0, part_o, part_ml, (size_t)h * nchunk_max * kGRowsMax + row, M, nchunk_max,
       [&] { return hl.goff >= 0 ? qkv + (size_t)t * hl.ldq + hl.goff + (size_t)hq * hl.qs : nullptr; },
       [&] { return out + ((size_t)t * Hq + hq) * D; });
@@ -434,18 +572,18 @@ __global__ __launch_bounds__(64 * kGWaves) void general_prompt_chunk_kernel(
       if (!live) qf[ks] = bf16x8_t{};
     }
     const size_t base = (((size_t)(z - z0) * Hkv + h) * nch + c) * kGRowsMax + wave * 16;
-    general_rows<D>(ks_lds, vs_lds, qf, key0, live ? p0 + t0 + qrow / G + 1 : key0, 0u, scale, part_o + base * D,
+    general_rows<D>(ks_lds, vs_lds, qf, key0, live ? p0 + t0 + qrow / G + 1 : key0, 0u, scale, rows - wave * 16, part_o + base * D,
                     part_ml + base * 2);
   }
 }
 
-template <int D>
-__global__ __launch_bounds__(64 * general_combine_waves<D>()) void general_prompt_combine_kernel(
+template <int D, int W>
+__global__ __launch_bounds__(64 * general_combine_waves<D>() * W) void general_prompt_combine_kernel(
     const int32_t* __restrict__ pos0, const float* __restrict__ part_o, const float* __restrict__ part_ml, int M, int Hq,
     int Hkv, int z0, int nch, const uint16_t* __restrict__ qkv, HeadLayout hl, uint16_t* __restrict__ out) {
   const int hq = blockIdx.x, t = z0 * kGMaxTokens + (int)blockIdx.y, z = t / kGMaxTokens;
   const int G = Hq / Hkv, h = hq / G, row = (t % kGMaxTokens) * G + hq % G;
-  general_combine_row<D>(
+  general_combine_row<D, W>(
       pos0, part_o, part_ml, (((size_t)(z - z0) * Hkv + h) * nch) * kGRowsMax + row, min(M, (z + 1) * kGMaxTokens), nch,
       [&] { return hl.goff >= 0 ? qkv + (size_t)t * hl.ldq + hl.goff + (size_t)hq * hl.qs : nullptr; },
       [&] { return out + ((size_t)t * Hq + hq) * D; });
@@ -477,11 +615,19 @@ int launch_general(const int32_t* pos0, const uint16_t* qkv, const HeadLayout& h
   hipLaunchKernelGGL(general_qk_store_kernel<D>, dim3(Hq + 2 * Hkv, M), dim3(64), 0, stream, pos0, qkv, hl, Hq, Hkv, qn,
                      kn, eps, R, rope, tree, M, q, kc, vt, maxlen);
   if (int rc = skinny_check_launch("attention_general q/k")) return rc;
-  hipLaunchKernelGGL(general_chunk_kernel<D>, dim3(nch, Hkv), dim3(64 * kGWaves), 0, stream, pos0, q, M, Hq, Hkv, kc,
-                     vt, maxlen, scale, tree, part_o, part_ml, nch);
+  if ((Hq / Hkv) * M <= kGFewRows && maxlen <= kGFewMaxlen) {
+    const int per = nch * Hkv <= 512 ? 1 : nch * Hkv <= 1024 ? 2 : kGWaves;
+    hipLaunchKernelGGL(general_few_kernel<D>, dim3((nch + per - 1) / per, Hkv), dim3(64 * per), 0, stream, pos0, q, M, Hq,
+                       Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nch, per);
+  } else {
+    hipLaunchKernelGGL(general_chunk_kernel<D>, dim3(nch, Hkv), dim3(64 * kGWaves), 0, stream, pos0, q, M, Hq, Hkv, kc,
+                       vt, maxlen, scale, tree, part_o, part_ml, nch);
+  }
   if (int rc = skinny_check_launch("attention_general chunks")) return rc;
-  hipLaunchKernelGGL(general_combine_kernel<D>, dim3(Hq, M), dim3(64 * general_combine_waves<D>()), 0, stream, pos0,
-                     part_o, part_ml, M, Hq, Hkv, nch, qkv, hl, out);
+  const int W = nch > kGCombineBlock ? kGCombineGroups : 1;  // nch: of the whole cache
+  const auto merge = W > 1 ? general_combine_kernel<D, kGCombineGroups> : general_combine_kernel<D, 1>;
+  hipLaunchKernelGGL(merge, dim3(Hq, M), dim3(64 * general_combine_waves<D>() * W), 0, stream, pos0, part_o, part_ml, M,
+                     Hq, Hkv, nch, qkv, hl, out);
   return skinny_check_launch("attention_general merge");
 }
 
@@ -503,6 +649,8 @@ int launch_general_prompt(const int32_t* pos0, const uint16_t* qkv, const HeadLa
   uint16_t* q = reinterpret_cast<uint16_t*>(ws);
   float* part_o = reinterpret_cast<float*>(ws + gprompt_query_bytes(M, Hq, D));
   float* part_ml = part_o + (size_t)fit * Hkv * nch * kGRowsMax * D;
+  const int W = maxlen / CH > kGCombineBlock ? kGCombineGroups : 1;  // as in the step's merge
+  const auto merge = W > 1 ? general_prompt_combine_kernel<D, kGCombineGroups> : general_prompt_combine_kernel<D, 1>;
   hipLaunchKernelGGL(general_qk_store_kernel<D>, dim3(Hq + Hkv, M), dim3(64), 0, stream, pos0, qkv, hl, Hq, Hkv, qn, kn,
                      eps, R, rope, nullptr, M, q, kc, vt, maxlen);
   if (int rc = skinny_check_launch("attention_general prompt q/k")) return rc;
@@ -515,9 +663,8 @@ int launch_general_prompt(const int32_t* pos0, const uint16_t* qkv, const HeadLa
     hipLaunchKernelGGL(general_prompt_chunk_kernel<D>, dim3(n, Hkv, (z1 - z0 + kGPieceGroup - 1) / kGPieceGroup),
                        dim3(64 * kGWaves), 0, stream, pos0, q, M, Hq, Hkv, kc, vt, maxlen, scale, z0, z1, nch, part_o, part_ml);
     if (int rc = skinny_check_launch("attention_general prompt chunks")) return rc;
-    hipLaunchKernelGGL(general_prompt_combine_kernel<D>, dim3(Hq, last - z0 * kGMaxTokens),
-                       dim3(64 * general_combine_waves<D>()), 0, stream, pos0, part_o, part_ml, M, Hq, Hkv, z0, nch, qkv, hl,
-                       out);
+    hipLaunchKernelGGL(merge, dim3(Hq, last - z0 * kGMaxTokens), dim3(64 * general_combine_waves<D>() * W), 0, stream, pos0,
+                       part_o, part_ml, M, Hq, Hkv, z0, nch, qkv, hl, out);
     if (int rc = skinny_check_launch("attention_general prompt merge")) return rc;
   }
   return SKINNY_OK;

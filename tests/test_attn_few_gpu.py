@@ -1,0 +1,68 @@
+"""Attention steps of few query rows (one wave per chunk, fragments straight from memory) give each token
+bitwise what a 16-token step over staged chunks gives it, and leave the same cache rows: chains and draft
+trees, new tokens inside a chunk and across a chunk edge, contexts below one chunk to several merge blocks,
+one, two and four chunks per workgroup."""
+
+import pytest
+import torch
+
+from skinny_mlx import kernels as K
+from skinny_mlx.tree import DraftTree
+
+pytestmark = pytest.mark.gpu
+
+# (kv heads, cache slots, cached tokens): chunks x heads <= 512, <= 1024, past it
+CASES = [(2, 1024, 0), (2, 1024, 100), (2, 1024, 250), (8, 8192, 5000), (8, 12288, 12200), (8, 33024, 32765)]
+
+
+def _call(layout, rnd, dev, hkv, maxlen):
+    if layout == "dense":
+        hq, d = 4 * hkv, 128
+        table, ws = K.rope_table(1e6, maxlen, dev), K.attn_workspace(hkv, maxlen, dev)
+        qn, kn = rnd(d), rnd(d)
+
+        def call(qkv, pos, k, vt, tree):
+            return K.attention_fused(qkv, hq, hkv, d, qn, kn, 1e-6, table, pos, k, vt, d ** -0.5, ws, tree)
+        return d, (hq + 2 * hkv) * d, call
+    d = int(layout)
+    hq, rd = 4 * hkv, d // 4
+    table, ws = K.rope_table_dim(1e7, rd, maxlen, dev), K.attn_general_workspace(hq, hkv, d, maxlen, dev)
+    qn, kn = rnd(d), rnd(d)
+
+    def call(qkv, pos, k, vt, tree):
+        return K.attention_general(qkv, hq, hkv, d, 2 * d, 2 * hq * d, 2 * hq * d + hkv * d, d, qn, kn, 1e-6, rd, table, pos,
+                                   k, vt, d ** -0.5, ws, tree)
+    return d, (2 * hq + 2 * hkv) * d, call
+
+
+@pytest.mark.parametrize("hkv,maxlen,past", CASES)
+@pytest.mark.parametrize("layout", ["dense", "64", "128", "256"])
+def test_few_rows_equal_a_long_step(dev, layout, hkv, maxlen, past):
+    g = torch.Generator(device=dev).manual_seed(past + hkv)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev).to(torch.bfloat16)
+    d, cols, call = _call(layout, rnd, dev, hkv, maxlen)
+    qkv, k0, v0 = rnd(16, cols), rnd(hkv, maxlen, d), rnd(hkv, d, maxlen)
+    k, vt = k0.clone(), v0.clone()
+    ref = call(qkv, torch.tensor([past], dtype=torch.int32, device=dev), k, vt, None)
+    for m in (1, 3, 4):
+        k2, v2, out = k0.clone(), v0.clone(), []
+        for i in range(0, 16, m):
+            out.append(call(qkv[i:i + m], torch.tensor([past + i], dtype=torch.int32, device=dev), k2, v2, None))
+        assert torch.equal(torch.cat(out), ref), m
+        assert torch.equal(k2, k) and torch.equal(v2, vt), m
+
+
+@pytest.mark.parametrize("layout", ["dense", "256"])
+@pytest.mark.parametrize("past", [5, 126, 1000])
+def test_few_rows_of_a_tree(dev, layout, past):
+    """The first four nodes of a five-node tree (20 rows: staged chunks) as a four-node tree (16 rows)."""
+    hkv, maxlen = 2, 1280
+    g = torch.Generator(device=dev).manual_seed(past)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev).to(torch.bfloat16)
+    d, cols, call = _call(layout, rnd, dev, hkv, maxlen)
+    qkv, k0, v0 = rnd(5, cols), rnd(hkv, maxlen, d), rnd(hkv, d, maxlen)
+    parents = [-1, 0, 0, 1, 3]
+    pos = torch.tensor([past], dtype=torch.int32, device=dev)
+    a = call(qkv, pos, k0.clone(), v0.clone(), DraftTree(parents, dev).desc)
+    b = call(qkv[:4], pos, k0.clone(), v0.clone(), DraftTree(parents[:4], dev).desc)
+    assert torch.equal(a[:4], b)

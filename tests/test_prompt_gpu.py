@@ -79,7 +79,7 @@ def test_unpatched_and_captured_inputs_keep_the_pieces():
     assert not hybrid._prompt_ok(ids)
 
 
-@pytest.mark.parametrize("maxlen,past", [(1024, 0), (1024, 250), (8192, 4300)])  # one- and four-wave merges
+@pytest.mark.parametrize("maxlen,past", [(1024, 0), (1024, 250), (8192, 4300), (17408, 16500)])  # one-, four- and eight-wave merges
 @pytest.mark.parametrize("layout", ["dense", "general"])
 def test_prompt_attention_equals_steps(dev, layout, maxlen, past):
     hq, hkv, d = (8, 2, 128) if layout == "dense" else (4, 1, 256)
