@@ -203,9 +203,7 @@ constexpr int kGdnThreads = kCols * kPart;
 
 // kTree: the draft-tree form (parent pointers, per-node snapshots in LDS) is its own kernel, so
 // the chain form carries none of its code (measured: 0.1-0.3 us faster per launch that way).
-// kLong: a chain of more than one block of tokens (a prompt) loads the next block's rows while the current
-// one runs, so that only the first block waits for memory.
-template <bool kTree, bool kLong = false>
+template <bool kTree>
 __global__ __launch_bounds__(kGdnThreads) void gdn_kernel(const uint16_t* __restrict__ qkv, int ldq,
                                                           const uint16_t* __restrict__ bcol,
                                                           const uint16_t* __restrict__ acol, int ldab,
@@ -237,54 +235,23 @@ __global__ __launch_bounds__(kGdnThreads) void gdn_kernel(const uint16_t* __rest
   float s0[8];  // the state before the step: a draft tree's root and its restarts branch from it
 #pragma unroll
   for (int e = 0; e < 8; ++e) s0[e] = s[e];
-  constexpr int kNextQk = kTokBlock * 32 / kGdnThreads;
-  static_assert(kTokBlock * kCols == kGdnThreads, "one value of v per thread and block");
-  u32x4_t nqk[kLong ? kNextQk : 1];  // kLong: the next block, tokens past the end repeat the last one
-  uint16_t nv = 0, na = 0, nb = 0;
-  auto load_next = [&](int t0) {
-#pragma unroll
-    for (int r = 0; r < kNextQk; ++r) {
-      const int i = tid + r * kGdnThreads, t = min(t0 + (i >> 5), M - 1);
-      nqk[r] = *reinterpret_cast<const u32x4_t*>(qkv + (size_t)t * ldq + (size_t)((i >> 4) & 1) * Hk * kDk + (size_t)hk * kDk +
-                                                 (i & 15) * 8);
-    }
-    nv = qkv[(size_t)min(t0 + tid / kCols, M - 1) * ldq + (size_t)2 * Hk * kDk + (size_t)h * kDv + blockIdx.y * kCols + tid % kCols];
-    const size_t g = (size_t)min(t0 + (tid & (kTokBlock - 1)), M - 1) * ldab + h;
-    na = acol[g];
-    nb = bcol[g];
-  };
-  if constexpr (kLong) load_next(0);
   for (int t0 = 0; t0 < M; t0 += kTokBlock) {
     const int mb = min(kTokBlock, M - t0);
     if (t0 > 0) __syncthreads();  // the previous block's staged rows are no longer read
-    if constexpr (kLong) {
-#pragma unroll
-      for (int r = 0; r < kNextQk; ++r) {
-        const int i = tid + r * kGdnThreads;
-        *reinterpret_cast<u32x4_t*>(&qk_lds[i >> 5][(i >> 4) & 1][(i & 15) * 8]) = nqk[r];
-      }
-      v_lds[tid / kCols][tid % kCols] = nv;
-      if (tid < mb) {
-        gate_lds[tid][0] = expf(neg_a * softplus(bf16_bits_to_f32(na) + dtb));
-        gate_lds[tid][1] = 1.0f / (1.0f + expf(-bf16_bits_to_f32(nb)));
-      }
-      if (t0 + kTokBlock < M) load_next(t0 + kTokBlock);
-    } else {
-      for (int i = tid; i < mb * 32; i += kGdnThreads) {  // q and k: 16 pieces of 16 bytes each per token
-        const int t = i >> 5, sel = (i >> 4) & 1, piece = i & 15;
-        *reinterpret_cast<u32x4_t*>(&qk_lds[t][sel][piece * 8]) = *reinterpret_cast<const u32x4_t*>(
-            qkv + (size_t)(t0 + t) * ldq + (size_t)sel * Hk * kDk + (size_t)hk * kDk + piece * 8);
-      }
-      for (int i = tid; i < mb * kCols; i += kGdnThreads)
-        v_lds[i / kCols][i % kCols] =
-            qkv[(size_t)(t0 + i / kCols) * ldq + (size_t)2 * Hk * kDk + (size_t)h * kDv + blockIdx.y * kCols + i % kCols];
-      if (tid < mb) {
-        gate_lds[tid][0] = expf(neg_a * softplus(bf16_bits_to_f32(acol[(size_t)(t0 + tid) * ldab + h]) + dtb));
-        gate_lds[tid][1] = 1.0f / (1.0f + expf(-bf16_bits_to_f32(bcol[(size_t)(t0 + tid) * ldab + h])));
-        if constexpr (kTree) par_lds[tid] = parent[t0 + tid];
-      }
+    for (int i = tid; i < mb * 32; i += kGdnThreads) {  // q and k: 16 pieces of 16 bytes each per token
+      const int t = i >> 5, sel = (i >> 4) & 1, piece = i & 15;
+      *reinterpret_cast<u32x4_t*>(&qk_lds[t][sel][piece * 8]) = *reinterpret_cast<const u32x4_t*>(
+          qkv + (size_t)(t0 + t) * ldq + (size_t)sel * Hk * kDk + (size_t)hk * kDk + piece * 8);
     }
-    lds_barrier();  // (a next block's loads stay in flight)
+    for (int i = tid; i < mb * kCols; i += kGdnThreads)
+      v_lds[i / kCols][i % kCols] =
+          qkv[(size_t)(t0 + i / kCols) * ldq + (size_t)2 * Hk * kDk + (size_t)h * kDv + blockIdx.y * kCols + i % kCols];
+    if (tid < mb) {
+      gate_lds[tid][0] = expf(neg_a * softplus(bf16_bits_to_f32(acol[(size_t)(t0 + tid) * ldab + h]) + dtb));
+      gate_lds[tid][1] = 1.0f / (1.0f + expf(-bf16_bits_to_f32(bcol[(size_t)(t0 + tid) * ldab + h])));
+      if constexpr (kTree) par_lds[tid] = parent[t0 + tid];
+    }
+    __syncthreads();
     // Normalised q and k of every token of the block, in parallel (they do not depend on the
     // state): 16-lane group g takes tokens g, g + kCols, ...; lane p its 8 dims.
     for (int i = cc; i < mb; i += kCols) {
@@ -308,7 +275,7 @@ __global__ __launch_bounds__(kGdnThreads) void gdn_kernel(const uint16_t* __rest
       kd[0] = f32x4_t{k[0] * kn, k[1] * kn, k[2] * kn, k[3] * kn};
       kd[1] = f32x4_t{k[4] * kn, k[5] * kn, k[6] * kn, k[7] * kn};
     }
-    lds_barrier();
+    __syncthreads();
     if constexpr (kTree) {
       if (record) {  // the commit's replay operands (a tree is one block: t0 == 0)
         const GdnRecord rl(kTokBlock, H);
@@ -423,6 +390,172 @@ __global__ __launch_bounds__(kGdnThreads) void gdn_kernel(const uint16_t* __rest
   if constexpr (kTree) return;  // a draft tree's state is chosen by the commit
   *reinterpret_cast<f32x4_t*>(state + sidx) = f32x4_t{s[0], s[1], s[2], s[3]};
   *reinterpret_cast<f32x4_t*>(state + sidx + 4) = f32x4_t{s[4], s[5], s[6], s[7]};
+}
+
+// The recurrence of a prompt (a chain of more than kTokBlock tokens): the same arithmetic over 32 lanes per
+// value column instead of 16, each holding 4 of a part's 8 key dims, {0, 1, 4, 5} or {2, 3, 6, 7}: half of
+// gdn_token's four partial sums, which the first exchange adds as gdn_token does, so states and y are bitwise
+// gdn_kernel's. A decode step is bound by its memory round trips; over many tokens the serial token loop is,
+// which gdn_kernel runs with one wave on every second SIMD. Here every SIMD has a wave with about 39
+// instructions per token: y's sum shares the lane exchanges of the next token's k.S, the gates are formed for
+// 256 tokens at a time, and a block's rows are loaded and normalised into the other buffer around the token loop,
+// one barrier per block. Measured, gdn_kernel against this: 509 tokens of 16 heads 133 us -> 70, of 32 heads
+// 149 -> 90, 2048 of 16 heads 623 -> 253, 64 of 16 heads 18.2 -> 12.6. Up to kTokBlock tokens stay with
+// gdn_kernel: one block has no loop to shorten, and drafts' trees are its own.
+constexpr int kLongPart = 32;
+constexpr int kLongThreads = kCols * kLongPart;
+
+// Two sums over the 32 lanes of a column (two rows of 16), the same in every lane: the rows' exchange leaves a's
+// pair sums in the first row and b's in the second, so that one row sum forms both.
+struct Sums {
+  float x, y;
+};
+__device__ __forceinline__ Sums sums32(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  const uint32_t v = __float_as_uint(row16_sum(__uint_as_float(r[0]) + __uint_as_float(r[1])));
+  const auto w = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return {__uint_as_float(w[0]), __uint_as_float(w[1])};
+}
+
+__global__ __launch_bounds__(kLongThreads) void gdn_long_kernel(const uint16_t* __restrict__ qkv, int ldq,
+                                                                const uint16_t* __restrict__ bcol,
+                                                                const uint16_t* __restrict__ acol, int ldab,
+                                                                const float* __restrict__ A_log,
+                                                                const float* __restrict__ dt_bias, float* state,
+                                                                float* __restrict__ states_out, float* __restrict__ y,
+                                                                int M, int H, int Hk) {
+  __shared__ __attribute__((aligned(16))) float qkn_lds[2][kTokBlock][2][kDk];  // lane l's four dims at 4l
+  __shared__ __attribute__((aligned(16))) f32x4_t vg_lds[2][kTokBlock][kCols];    // v, decay, beta
+  __shared__ float2 gate_lds[2][kLongThreads];                                    // decay, beta
+  const int h = blockIdx.x, tid = threadIdx.x;
+  const int hk = h / (H / Hk);
+  const int cc = tid / kLongPart, l = tid % kLongPart;
+  const int col = blockIdx.y * kCols + cc;
+  const size_t sidx = ((size_t)h * kDv + col) * kDk + (l % kPart) * 8 + l / kPart * 2;  // dims +0, +1, +4, +5
+  float s[4];
+  {
+    const float2 a = *reinterpret_cast<const float2*>(state + sidx), b = *reinterpret_cast<const float2*>(state + sidx + 4);
+    s[0] = a.x; s[1] = a.y; s[2] = b.x; s[3] = b.y;
+  }
+  const float neg_a = -expf(A_log[h]);
+  const float dtb = dt_bias[h];
+  const float qscale = rsqrtf((float)kDk);
+  // A block's rows: 16-lane group i holds token i, lane p its dims 8p .. 8p + 7 of q and k. Tokens past the end
+  // repeat the last one.
+  const int i = tid / kPart, p = tid % kPart;
+  const int vt = tid / kCols % kTokBlock, vc = tid % kCols;
+  u32x4_t qw, kw;
+  uint16_t nv, na, nb;
+  // The gates' exponentials and logarithm, kLongThreads tokens at a time: a thread per token.
+  auto load_gates = [&](int t0) {
+    const size_t g = (size_t)min(t0 + tid, M - 1) * ldab + h;
+    na = acol[g];
+    nb = bcol[g];
+  };
+  auto form_gates = [&](int t0) {
+    gate_lds[t0 / kLongThreads & 1][tid] =
+        float2{expf(neg_a * softplus(bf16_bits_to_f32(na) + dtb)), 1.0f / (1.0f + expf(-bf16_bits_to_f32(nb)))};
+  };
+  auto load = [&](int t0) {
+    const uint16_t* row = qkv + (size_t)min(t0 + i, M - 1) * ldq + (size_t)hk * kDk + p * 8;
+    qw = *reinterpret_cast<const u32x4_t*>(row);
+    kw = *reinterpret_cast<const u32x4_t*>(row + (size_t)Hk * kDk);
+    nv = qkv[(size_t)min(t0 + vt, M - 1) * ldq + (size_t)2 * Hk * kDk + (size_t)h * kDv + blockIdx.y * kCols + vc];
+  };
+  auto stage = [&](int t0) {
+    const int buf = t0 / kTokBlock & 1;
+    if (tid < kTokBlock * kCols) {
+      const float2 g = gate_lds[t0 / kLongThreads & 1][t0 % kLongThreads + vt];
+      vg_lds[buf][vt][vc] = f32x4_t{bf16_bits_to_f32(nv), g.x, g.y, 0.f};
+    }
+    float q[8], k[8];
+    float qq = 0.f, kk = 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      q[e] = bf16_bits_to_f32((e & 1) ? (qw[e >> 1] >> 16) : (qw[e >> 1] & 0xffffu));
+      k[e] = bf16_bits_to_f32((e & 1) ? (kw[e >> 1] >> 16) : (kw[e >> 1] & 0xffffu));
+      qq = fmaf(q[e], q[e], qq);
+      kk = fmaf(k[e], k[e], kk);
+    }
+    const float qn = rsqrtf(sum16(qq) + 1e-6f) * qscale;
+    const float kn = rsqrtf(sum16(kk) + 1e-6f);
+    f32x4_t* qd = reinterpret_cast<f32x4_t*>(&qkn_lds[buf][i][0][p * 4]);
+    f32x4_t* kd = reinterpret_cast<f32x4_t*>(&qkn_lds[buf][i][1][p * 4]);
+    qd[0] = f32x4_t{q[0] * qn, q[1] * qn, q[4] * qn, q[5] * qn};
+    qd[kPart] = f32x4_t{q[2] * qn, q[3] * qn, q[6] * qn, q[7] * qn};
+    kd[0] = f32x4_t{k[0] * kn, k[1] * kn, k[4] * kn, k[5] * kn};
+    kd[kPart] = f32x4_t{k[2] * kn, k[3] * kn, k[6] * kn, k[7] * kn};
+  };
+  float ysum = 0.f;  // this lane's share of the last token's y
+  float* yrow = y + (size_t)h * kDv;  // the last token's row
+  const size_t ystep = (size_t)H * kDv;
+  load(0);
+  load_gates(0);
+  form_gates(0);
+  lds_barrier();
+  stage(0);
+  for (int t0 = 0; t0 < M; t0 += kTokBlock) {
+    const int mb = min(kTokBlock, M - t0), buf = t0 / kTokBlock & 1;
+    if (t0 + kTokBlock < M) load(t0 + kTokBlock);
+    if ((t0 + kTokBlock) % kLongThreads == 0) form_gates(t0 + kTokBlock);  // loaded a block ago
+    if ((t0 + 2 * kTokBlock) % kLongThreads == 0) load_gates(t0 + 2 * kTokBlock);
+    lds_barrier();  // this block is staged and the last one, in the other buffer, read; the loads stay in flight
+    struct Ops {
+      f32x4_t q, k, vg;
+    };
+    auto fetch = [&](int i, Ops& o) {
+      o.q = *reinterpret_cast<const f32x4_t*>(&qkn_lds[buf][i][0][l * 4]);
+      o.k = *reinterpret_cast<const f32x4_t*>(&qkn_lds[buf][i][1][l * 4]);
+      o.vg = vg_lds[buf][i][cc];
+    };
+    auto run = [&](auto record) {
+      auto token = [&](int i, const Ops& o) {
+        float a0 = s[0] * o.k[0], a1 = s[1] * o.k[1];
+        a0 = fmaf(s[2], o.k[2], a0);
+        a1 = fmaf(s[3], o.k[3], a1);
+        const Sums sum = sums32(a0 + a1, ysum);
+        yrow[(unsigned)col] = sum.y;  // before token 0: zeros to its row, which its own y follows
+        if (i > 0 || t0 > 0) yrow += ystep;
+        const float delta = o.vg[2] * (o.vg[0] - o.vg[1] * sum.x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = fmaf(o.k[e], delta, s[e] * o.vg[1]);
+        float b0 = s[0] * o.q[0], b1 = s[1] * o.q[1];
+        b0 = fmaf(s[2], o.q[2], b0);
+        b1 = fmaf(s[3], o.q[3], b1);
+        ysum = b0 + b1;
+        if constexpr (decltype(record)::value) {
+          float* dst = states_out + (size_t)(t0 + i) * H * kDv * kDk + sidx;
+          *reinterpret_cast<float2*>(dst) = float2{s[0], s[1]};
+          *reinterpret_cast<float2*>(dst + 4) = float2{s[2], s[3]};
+        }
+      };
+      // operands two tokens ahead: a full block unrolled, the last one as it comes
+      if (mb == kTokBlock) {
+        Ops o[3];
+        fetch(0, o[0]);
+        fetch(1, o[1]);
+#pragma unroll
+        for (int i = 0; i < kTokBlock; ++i) {
+          if (i + 2 < kTokBlock) fetch(i + 2, o[(i + 2) % 3]);
+          token(i, o[i % 3]);
+        }
+      } else {
+        for (int i = 0; i < mb; ++i) {
+          Ops o;
+          fetch(i, o);
+          token(i, o);
+        }
+      }
+    };
+    if (states_out)
+      run(BoolTag<true>{});
+    else
+      run(BoolTag<false>{});
+    if (t0 + kTokBlock < M) stage(t0 + kTokBlock);
+  }
+  yrow[(unsigned)col] = sums32(0.f, ysum).y;
+  *reinterpret_cast<float2*>(state + sidx) = float2{s[0], s[1]};
+  *reinterpret_cast<float2*>(state + sidx + 4) = float2{s[2], s[3]};
 }
 
 // One token of the gated delta rule with the output norm in the same launch, for a step that keeps
@@ -686,8 +819,12 @@ extern "C" int skinny_gdn_recurrence(const uint16_t* qkv, int ldq, const uint16_
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)snap_bytes);
     if (e != hipSuccess) return skinny_set_error(SKINNY_ELAUNCH, "gdn: %zu bytes of snapshots: %s", snap_bytes, hipGetErrorString(e));
   }
-  const auto kern = parent ? gdn_kernel<true, false> : M > kTokBlock ? gdn_kernel<false, true> : gdn_kernel<false, false>;
-  hipLaunchKernelGGL(kern, dim3(H, kDv / kCols), dim3(kGdnThreads), snap_bytes,
+  if (!parent && M > kTokBlock) {
+    hipLaunchKernelGGL(gdn_long_kernel, dim3(H, kDv / kCols), dim3(kLongThreads), 0, (hipStream_t)stream, qkv, ldq, b, a,
+                       ldab, A_log, dt_bias, state, states_out, y, M, H, Hk);
+    return skinny_check_launch("gdn");
+  }
+  hipLaunchKernelGGL(parent ? gdn_kernel<true> : gdn_kernel<false>, dim3(H, kDv / kCols), dim3(kGdnThreads), snap_bytes,
                      (hipStream_t)stream, qkv, ldq, b, a, ldab, A_log, dt_bias, state, states_out, y, parent, M, H,
                      record, Hk);
   return skinny_check_launch("gdn");

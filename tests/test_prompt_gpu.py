@@ -139,7 +139,7 @@ def test_prompt_attention_in_several_launches(dev):
 
 
 @pytest.mark.parametrize("h,hk", [(4, 4), (4, 2)])
-@pytest.mark.parametrize("t", [17, 33, 130])
+@pytest.mark.parametrize("t", [17, 33, 130, 256, 257, 530])  # gates come in blocks of 256
 def test_long_conv_and_recurrence_equal_blocks(dev, h, hk, t):
     c = 2 * hk * 128 + h * 128
     g = torch.Generator(device=dev).manual_seed(t + h)
@@ -152,10 +152,11 @@ def test_long_conv_and_recurrence_equal_blocks(dev, h, hk, t):
     res = []
     for step in (t, 16):
         conv, s, xs, ys = conv0.clone(), s0.clone(), [], []
+        rec = torch.empty((t, h, 128, 128), device=dev)
         for i in range(0, t, step):
             xs.append(K.gdn_conv_silu(x[i:i + step], conv, w, None))
-            ys.append(K.gdn_recurrence(xs[-1], ab[i:i + step, :h], ab[i:i + step, h:], A, dtb, s, None, h, 128, 128,
-                                       n_key_heads=hk))
-        res.append((torch.cat(xs), torch.cat(ys), conv, s))
+            ys.append(K.gdn_recurrence(xs[-1], ab[i:i + step, :h], ab[i:i + step, h:], A, dtb, s,
+                                       rec[i:i + step] if t % 2 else None, h, 128, 128, n_key_heads=hk))
+        res.append((torch.cat(xs), torch.cat(ys), conv, s) + ((rec,) if t % 2 else ()))
     for a, b in zip(*res):
         assert torch.equal(a, b)
