@@ -214,8 +214,15 @@ def check(rc: int, what: str) -> None:
     raise SkinnyLaunchError(f"{what} (code {rc}): {msg}")
 
 
+# torch's current stream of a device index as an int: the lookup alone, without the Stream object that
+# torch.cuda.current_stream builds around it (0.2 us a call against 2.0).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
     """hipStream_t (as int) of torch's current stream on t's device."""
+    if _raw_stream is not None and t.is_cuda:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 

@@ -31,6 +31,7 @@ Differences from the reference, by design:
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -152,8 +153,10 @@ def packed_weights(w: torch.Tensor, k: int, scales: torch.Tensor | None = None,
                                                   n, k, _lib.stream_of(w)), "skinny_qmm")
         w._skinny_full = (key, full)
         return full
-    if packed_k(w) != k:
+    if words * 64 != k * 9:
         raise ValueError(f"x has K={k}, weights have K={packed_k(w)}")
+    if scales is None and biases is None:
+        return w
     src = getattr(w, "_skinny_packed_from", None)
     for t, name, i in ((scales, "scales", 0), (biases, "biases", 1)):
         if t is None:
@@ -238,6 +241,30 @@ def _table_tile(k: int, n: int):
     return t
 
 
+# A call of one small projection is bound by the host (14 us of Python and ctypes against 4.5 us of kernel at
+# 4096 x 2560, one row), so these make a tensor only where one is needed. Measured together with the plain
+# stream lookup and the workspace size looked up by (N, splits): 14.1 -> 8.8 us a call at that size.
+
+def _rows_of(x: torch.Tensor, k: int) -> torch.Tensor:
+    """x [..., k] as bf16 rows of 16-byte alignment: x itself where it already is."""
+    x2 = x if x.dim() == 2 and x.shape[1] == k else x.reshape(-1, k)
+    if x2.dtype != torch.bfloat16:
+        x2 = x2.to(torch.bfloat16)
+    if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
+        x2 = x2.contiguous()
+    return x2
+
+
+def _row_ptr(t: torch.Tensor, row: int) -> int:
+    """Address of row `row` of a 16-bit matrix."""
+    return t.data_ptr() + 2 * row * t.stride(0)
+
+
+def _like_rows(y: torch.Tensor, x: torch.Tensor, n: int) -> torch.Tensor:
+    """y [M, n] in the leading dimensions of x."""
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], n)
+
+
 def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = None,
                biases: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """x [..., K] @ dequant(w)[N, K]^T -> [..., N] in bf16 (fp32 accumulation).
@@ -250,15 +277,10 @@ def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = N
     k = x.shape[-1]
     w = packed_weights(w, k, scales, biases)
     n = w.shape[0]
-    lead = x.shape[:-1]
-    x2 = x.reshape(-1, k)
-    if x2.dtype != torch.bfloat16:
-        x2 = x2.to(torch.bfloat16)
-    if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
-        x2 = x2.contiguous()
+    x2 = _rows_of(x, k)
     m = x2.shape[0]
     if out is None:
-        y = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+        y = torch.empty((m, n), dtype=torch.bfloat16, device=x2.device)
     else:
         if out.dtype != torch.bfloat16 or tuple(out.shape) != (m, n) or out.stride(-1) != 1:
             raise ValueError("out must be bf16 [M, N] with unit inner stride")
@@ -268,23 +290,19 @@ def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = N
     splits, tile = _plain_config(k, n)
     if m >= rows_from(n, splits) and not CONFIG_OVERRIDE and not SPLITK_OVERRIDE:
         _rows(x2, w, y, splits, tile, EPI_PLAIN, "skinny_qmm")
-        return y.reshape(*lead, n)
+        return _like_rows(y, x, n)
     if splits > 1:
         ws = splitk_workspace(x2.device, n, splits, stream)
         for m0 in range(0, m, MAX_M):
-            mc = min(MAX_M, m - m0)
-            xc, yc = x2[m0:m0 + mc], y[m0:m0 + mc]
-            _lib.check(L.skinny_qmm_w4g64_splitk_bf16(xc.data_ptr(), mc, k, x2.stride(0), w.data_ptr(), n,
-                                                      yc.data_ptr(), y.stride(0), ws.data_ptr(),
+            _lib.check(L.skinny_qmm_w4g64_splitk_bf16(_row_ptr(x2, m0), min(MAX_M, m - m0), k, x2.stride(0), w.data_ptr(), n,
+                                                      _row_ptr(y, m0), y.stride(0), ws.data_ptr(),
                                                       ws.numel() * ws.element_size(), splits, ctypes.byref(tile),
                                                       stream), "skinny_qmm")
-        return y.reshape(*lead, n)
+        return _like_rows(y, x, n)
     for m0 in range(0, m, MAX_M):
-        mc = min(MAX_M, m - m0)
-        xc, yc = x2[m0:m0 + mc], y[m0:m0 + mc]
-        _lib.check(L.skinny_qmm_w4g64_bf16(xc.data_ptr(), mc, k, x2.stride(0), w.data_ptr(), n, yc.data_ptr(),
-                                           y.stride(0), ctypes.byref(tile), stream), "skinny_qmm")
-    return y.reshape(*lead, n)
+        _lib.check(L.skinny_qmm_w4g64_bf16(_row_ptr(x2, m0), min(MAX_M, m - m0), k, x2.stride(0), w.data_ptr(), n,
+                                           _row_ptr(y, m0), y.stride(0), ctypes.byref(tile), stream), "skinny_qmm")
+    return _like_rows(y, x, n)
 
 
 # The many-row kernel (skinny_qmm_w4g64_rows_bf16): epilogues, and the rows one launch takes.
@@ -315,8 +333,8 @@ def _rows(x2: torch.Tensor, w: torch.Tensor, y: torch.Tensor, splits: int, tile,
     L = _lib.lib()
     stream = _lib.stream_of(x2)
     for m0 in range(0, m, _ROWS_MAX):
-        _lib.check(L.skinny_qmm_w4g64_rows_bf16(x2[m0:].data_ptr(), min(_ROWS_MAX, m - m0), k, x2.stride(0), w.data_ptr(),
-                                                w.shape[0], y[m0:].data_ptr(), y.stride(0), splits, groups, epilogue,
+        _lib.check(L.skinny_qmm_w4g64_rows_bf16(_row_ptr(x2, m0), min(_ROWS_MAX, m - m0), k, x2.stride(0), w.data_ptr(),
+                                                w.shape[0], _row_ptr(y, m0), y.stride(0), splits, groups, epilogue,
                                                 stream), what)
 
 
@@ -344,6 +362,11 @@ def _plain_config(k: int, n: int):
 _SPLITK_WS_MIN_WORDS = 4 + 16 * 16384 * 3  # the header and three slices of N = 16384
 
 
+@functools.lru_cache(maxsize=256)
+def _splitk_bytes(n: int, splits: int) -> int:
+    return int(_lib.lib().skinny_qmm_splitk_workspace_bytes(n, splits))
+
+
 def splitk_workspace(device, n: int, splits: int, stream: int | None = None) -> torch.Tensor:
     """The split-K workspace of (device, stream), every word 0xFFFFFFFF (the kernel's "not yet
     written", restored by every call). Calls on one stream are ordered, so they share it; calls on
@@ -354,13 +377,13 @@ def splitk_workspace(device, n: int, splits: int, stream: int | None = None) -> 
     call, or grown when a call needs more. Inside a graph capture that allocation comes from the
     graph's memory pool and its fill is recorded ahead of the matmul, so every replay starts from
     a filled buffer; eager calls on the same stream later use the same buffer."""
-    key_dev = torch.device(device)
+    key_dev = device if isinstance(device, torch.device) else torch.device(device)
     if key_dev.type == "cuda" and key_dev.index is None:
         key_dev = torch.device("cuda", torch.cuda.current_device())
     if stream is None:
         stream = torch.cuda.current_stream(key_dev).cuda_stream
     key = (key_dev, int(stream))
-    need = int(_lib.lib().skinny_qmm_splitk_workspace_bytes(n, splits))
+    need = _splitk_bytes(n, splits)
     ws = _SPLITK_WS.get(key)
     if ws is None or ws.numel() * 4 < need:
         ws = _SPLITK_WS[key] = torch.full((max(need // 4, _SPLITK_WS_MIN_WORDS),), -1, dtype=torch.int32,
@@ -709,16 +732,11 @@ def skinny_glu(x: torch.Tensor, w: torch.Tensor, swiglu: bool, out: torch.Tensor
     f = w.shape[0] // 2
     if x.shape[-1] != k:
         raise ValueError(f"x has K={x.shape[-1]}, weights have K={k}")
-    lead = x.shape[:-1]
-    x2 = x.reshape(-1, k)
-    if x2.dtype != torch.bfloat16:
-        x2 = x2.to(torch.bfloat16)
-    if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
-        x2 = x2.contiguous()
+    x2 = _rows_of(x, k)
     m = x2.shape[0]
     width = f if swiglu else 2 * f
     if out is None:
-        y = torch.empty((m, width), dtype=torch.bfloat16, device=x.device)
+        y = torch.empty((m, width), dtype=torch.bfloat16, device=x2.device)
     else:
         if out.dtype != torch.bfloat16 or tuple(out.shape) != (m, width) or out.stride(-1) != 1:
             raise ValueError(f"out must be bf16 [M, {width}] with unit inner stride")
@@ -726,15 +744,14 @@ def skinny_glu(x: torch.Tensor, w: torch.Tensor, swiglu: bool, out: torch.Tensor
     tile = glu_tile(k, f)
     if m >= rows_from(2 * f, 1):
         _rows(x2, w, y, 1, tile, EPI_SWIGLU if swiglu else EPI_GLU_SPLIT, "skinny_glu")
-        return y.reshape(*lead, width)
+        return _like_rows(y, x, width)
     L = _lib.lib()
     stream = _lib.stream_of(x2)
     for m0 in range(0, m, MAX_M):
-        mc = min(MAX_M, m - m0)
-        _lib.check(L.skinny_qmm_w4g64_glu_bf16(x2[m0:].data_ptr(), mc, k, x2.stride(0), w.data_ptr(), f,
-                                               y[m0:].data_ptr(), y.stride(0), int(swiglu), ctypes.byref(tile),
+        _lib.check(L.skinny_qmm_w4g64_glu_bf16(_row_ptr(x2, m0), min(MAX_M, m - m0), k, x2.stride(0), w.data_ptr(), f,
+                                               _row_ptr(y, m0), y.stride(0), int(swiglu), ctypes.byref(tile),
                                                stream), "skinny_glu")
-    return y.reshape(*lead, width)
+    return _like_rows(y, x, width)
 
 
 # ---------------------------------------------------------------------------------------------
