@@ -12,12 +12,15 @@
 //
 // Layout. A workgroup of 4 waves holds 16 MT rows x 64 NT weight rows: the waves share the X block (staged
 // in LDS in MFMA fragment order, two buffers of one 128-wide pair) and own 16 NT weight rows each, whose
-// packed blocks go straight to registers (two pairs in flight), so a weight crosses the memory path once
-// per 16 MT rows. What bounds it is VALU issue beside the matrix cores: per 16x16 tile and scale group two
-// MFMAs (32 cycles) stand against 8 FMAs (32 cycles; the scale and bias terms in fp32, which the bits fix)
-// and the nibble unpacking (17 instructions per 16 weight rows, shared by MT tiles). MT = 2 keeps a wave at
-// 118-150 registers (three or four waves per SIMD); MT = 4 saves a fifth of the instructions but leaves two
-// waves per SIMD, and was slower everywhere (2560x19456, 501 rows: 104 against 94 us).
+// packed blocks go straight to registers, so a weight crosses the memory path once per 16 MT rows. What
+// bounds it is the issue of one SIMD's waves: per 16x16 tile and scale group two MFMAs (32 cycles) stand
+// against 8 FMAs (32 cycles; the scale and bias terms in fp32, which the bits fix) and the nibble unpacking
+// (17 instructions per 16 weight rows, shared by MT tiles), so everything else has to be hidden: X's LDS reads
+// run half a pair ahead of their MFMAs, X's rows are loaded in whole 128-byte lines, and the loop's loads stand
+// in the same order on every path, as a wait counts the loads issued after the one it is for. With three waves
+// per SIMD for the wide wave, that took 2560x19456 at 501 rows from 81 to 77 us, 9728x2560 at 1024 rows from 106
+// to 95 and at 96 rows from 33 to 25 (VALU active 67% of the CUs' busy time before, 86% after). MT = 4 saves a fifth
+// of the instructions but leaves two waves per SIMD, and was slower everywhere (2560x19456, 501 rows: 95 us).
 #include "qmm_frag.h"
 
 namespace {
@@ -38,6 +41,11 @@ __device__ __forceinline__ void load_xpart(XPart<MT>& xp, __amdgpu_buffer_rsrc_t
     xp.v[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rx, xoff[i], pair * 256, 0));
 }
 
+template <int V>
+struct IntTag {
+  static constexpr int value = V;
+};
+
 // The cut of K walked by one wave of the kernel below.
 struct RowsArgs {
   const uint16_t* x;
@@ -54,10 +62,20 @@ struct RowsArgs {
 // [p G / KS, (p + 1) G / KS) of the one split, and leaves its split's sum, or each of its groups' sums, in
 // LDS; part 0 then adds them in the cut's order, so the bits do not depend on KS. NACC: sums a wave keeps
 // apart (1 = one group in all, 2 = groups, 3 = groups and splits).
+//
+// The wide wave (NT = 4) and several parts keep one pair of weights per wave in flight, loaded again as soon
+// as its second half is unpacked: half a pair of time, which the other waves of the SIMD fill; one part of
+// NT = 2 has registers for two (9728x2560, 1024 rows: 97 against 104 us). The wide wave also keeps its group sums in
+// LDS, each lane its own words: in registers they spilled within the loop at three waves per SIMD (2560x19456,
+// 501 rows: 90 against 86 us).
 template <int MT, int NT, int NACC, int KS, int EPI>
-__global__ __launch_bounds__(256 * KS) void qmm_rows_kernel(const RowsArgs ra) {
+__global__ __launch_bounds__(256 * KS, NT == 4 ? 3 : 1) void qmm_rows_kernel(const RowsArgs ra) {
   static_assert(EPI == kRowsPlain || NT % 2 == 0, "gate|up epilogues pair two row tiles per wave");
   static_assert(KS == 1 || NACC == 2, "several parts: the groups of one split each");
+  static_assert(NT < 4 || NACC < 3, "the wide wave's registers hold two sums at most");
+  constexpr bool kGrpLds = NT == 4 && NACC == 2;     // the group sums live in LDS
+  constexpr bool kGrp = NACC >= 2 && !kGrpLds;
+  constexpr int kStages = NT == 4 || KS > 1 ? 1 : 2;  // pairs of weights in flight
   constexpr int kXWords = MT * 4 * 64;  // 16-byte words of one staged pair
   constexpr int kOutCols = EPI == kRowsSwiGlu ? 8 * NT : 16 * NT;
   constexpr int kOutPitch = kOutCols + 8;
@@ -87,23 +105,28 @@ __global__ __launch_bounds__(256 * KS) void qmm_rows_kernel(const RowsArgs ra) {
   const bf16x8_t ones = ones_operand();
   u32x4_t* const xl = reinterpret_cast<u32x4_t*>(lds) + part * 2 * kXWords;
   float* const sums = reinterpret_cast<float*>(lds + (size_t)KS * 2 * kXWords * 16);
-  // This wave stages fragments f = wave MT .. + MT - 1 of its part's pairs. Rows past M carry an
-  // out-of-range offset and read as zeros.
+  // This wave stages fragments wave MT .. + MT - 1 of its part's pairs, two (the 64 columns of a scale group)
+  // at a time as 8 rows of 128 bytes per load. Rows past M carry an out-of-range offset and read as zeros.
+  // Lane group g = lane / 8 takes rows 4 (g % 4) + g / 4 and two below, and a fragment's quad holds its rows in
+  // the order t ^ quad ^ 12 h: so both the 16 lanes of a read and any 16 of a write fall on different banks.
+  static_assert(MT % 2 == 0, "a wave stages pairs of fragments");
+  auto slot_of = [](int t, int qd, int h) { return qd * 16 + (t ^ qd ^ (12 * h)); };
+  const int srow = ((lane >> 3) & 3) * 4 + (lane >> 5);
   uint32_t xoff[MT];
 #pragma unroll
   for (int i = 0; i < MT; ++i) {
-    const int f = wave * MT + i, r = (f >> 2) * 16 + tok;
-    xoff[i] = r < rows ? (uint32_t)(r * ldx + (f & 3) * 32 + quad * 8) * 2u : 0x7ffffff0u;
+    const int f = wave * MT + i, r = (f >> 2) * 16 + (f & 1) * 2 + srow;
+    xoff[i] = r < rows ? (uint32_t)(r * ldx + (f & 2) * 32 + (lane & 7) * 8) * 2u : 0x7ffffff0u;
   }
 
-  f32x4_t acc[MT][NT], grp[NACC >= 2 ? MT : 1][NACC >= 2 ? NT : 1], spl[NACC >= 3 ? MT : 1][NACC >= 3 ? NT : 1];
+  f32x4_t acc[MT][NT], grp[kGrp ? MT : 1][kGrp ? NT : 1], spl[NACC >= 3 ? MT : 1][NACC >= 3 ? NT : 1];
   const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int n = 0; n < NT; ++n) {
       acc[m][n] = zero;
-      if constexpr (NACC >= 2) grp[m][n] = zero;
+      if constexpr (kGrp) grp[m][n] = zero;
       if constexpr (NACC >= 3) spl[m][n] = zero;
     }
 
@@ -137,9 +160,23 @@ __global__ __launch_bounds__(256 * KS) void qmm_rows_kernel(const RowsArgs ra) {
   auto close = [&](int p) {  // after pair p
     if constexpr (NACC >= 2) {
       if (p + 1 != gend) return;
+      if constexpr (kGrpLds) {  // this lane's own words; the last group's sum stays in acc
+        f32x4_t* d = reinterpret_cast<f32x4_t*>(sums) + wave * MT * NT * 64 + lane;
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            const f32x4_t v = (g > 0 ? d[(m * NT + n) * 64] : zero) + acc[m][n];
+            if (g + 1 < G) d[(m * NT + n) * 64] = v;
+            acc[m][n] = g + 1 < G ? zero : v;
+          }
+        ++g;
+        gend = (g + 1) * GP / G;
+        return;
+      }
       if (KS > 1 && S == 1 && part > 0) {
         dump(acc);
-      } else {
+      } else if constexpr (kGrp) {
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -169,44 +206,52 @@ __global__ __launch_bounds__(256 * KS) void qmm_rows_kernel(const RowsArgs ra) {
     }
   };
 
-  auto compute = [&](const u32x4_t* xs, const WStage<NT>& ws) {
+  using XOps = bf16x8_t[MT][2];  // X's operands of one scale group
+  auto fetch = [&](XOps& o, int buf, int j) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      bf16x8_t xa[MT][2];
-      f32x4_t xsum[MT];
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        o[m][h] = __builtin_bit_cast(bf16x8_t, xl[buf * kXWords + (m * 4 + j * 2 + h) * 64 + slot_of(tok, quad, h)]);
+  };
+  auto load_w1 = [&](WStage<NT>& ws, int n, int p) {
+    const int blk = (n * GP + p) * kBlockBytes;
+    ws.w[n] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, woff, blk, 0));
+    ws.sb[n] = __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(rw, sboff, blk, 0));
+  };
+  // Scale group j of a pair; with one stage the second group's tiles make way for those of pair `next`.
+  auto compute = [&](const XOps& xa, WStage<NT>& ws, int j, int next) {
+    f32x4_t xsum[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) xsum[m] = mfma16x16x32(xa[m][0], ones, zero);
+#pragma unroll
+    for (int m = 0; m < MT; ++m) xsum[m] = mfma16x16x32(xa[m][1], ones, xsum[m]);
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+      const bf16x8_t b0 = unpack_nibbles(j ? ws.w[n].z : ws.w[n].x), b1 = unpack_nibbles(j ? ws.w[n].w : ws.w[n].y);
+      const float s = __uint_as_float(j ? (ws.sb[n].x & 0xffff0000u) : (ws.sb[n].x << 16));
+      const float b = __uint_as_float(j ? (ws.sb[n].y & 0xffff0000u) : (ws.sb[n].y << 16));
+      const float bp = fmaf(-128.0f, s, b);
+      if (kStages == 1 && j == 1) load_w1(ws, n, next);
+      f32x4_t gm[MT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) gm[m] = mfma16x16x32(xa[m][0], b0, zero);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) gm[m] = mfma16x16x32(xa[m][1], b1, gm[m]);
 #pragma unroll
       for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) xa[m][h] = __builtin_bit_cast(bf16x8_t, xs[(m * 4 + j * 2 + h) * 64 + lane]);
-#pragma unroll
-      for (int m = 0; m < MT; ++m) xsum[m] = mfma16x16x32(xa[m][0], ones, zero);
-#pragma unroll
-      for (int m = 0; m < MT; ++m) xsum[m] = mfma16x16x32(xa[m][1], ones, xsum[m]);
-#pragma unroll
-      for (int n = 0; n < NT; ++n) {
-        const bf16x8_t b0 = unpack_nibbles(j ? ws.w[n].z : ws.w[n].x), b1 = unpack_nibbles(j ? ws.w[n].w : ws.w[n].y);
-        const float s = __uint_as_float(j ? (ws.sb[n].x & 0xffff0000u) : (ws.sb[n].x << 16));
-        const float b = __uint_as_float(j ? (ws.sb[n].y & 0xffff0000u) : (ws.sb[n].y << 16));
-        const float bp = fmaf(-128.0f, s, b);
-        f32x4_t gm[MT];
-#pragma unroll
-        for (int m = 0; m < MT; ++m) gm[m] = mfma16x16x32(xa[m][0], b0, zero);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) gm[m] = mfma16x16x32(xa[m][1], b1, gm[m]);
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            acc[m][n][i] = fmaf(s, gm[m][i], acc[m][n][i]);
-            acc[m][n][i] = fmaf(bp, xsum[m][i], acc[m][n][i]);
-          }
-      }
+        for (int i = 0; i < 4; ++i) {
+          acc[m][n][i] = fmaf(s, gm[m][i], acc[m][n][i]);
+          acc[m][n][i] = fmaf(bp, xsum[m][i], acc[m][n][i]);
+        }
     }
   };
 
-  // Pair q of the part (counted from `first`): its X is in LDS buffer q % 2 (stored during pair q - 1, from
-  // registers loaded during q - 2), its weights in ring stage q % 2. One barrier per pair; every part runs
-  // the longest part's count of rounds.
+  // Pair q of the part (counted from `first`): its X is in LDS buffer q % 2, stored while pair q - 1's first
+  // group runs, from registers loaded a pair before. One barrier per pair, between its groups: then pair q + 1
+  // is staged and this pair's operands are read, and each group's operands are fetched while the other group
+  // runs. Every part runs the longest part's count of rounds.
   int rounds = stop - first;
   if constexpr (KS > 1) {
 #pragma unroll
@@ -215,35 +260,55 @@ __global__ __launch_bounds__(256 * KS) void qmm_rows_kernel(const RowsArgs ra) {
       rounds = max(rounds, n);
     }
   }
-  WStage<NT> ws[2];
+  WStage<NT> ws[kStages];
   XPart<MT> xp;
   const int last = stop - 1;
   auto store_x = [&](int buf) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) xl[buf * kXWords + (wave * MT + i) * 64 + lane] = xp.v[i];
+    for (int i = 0; i < MT; ++i) {
+      const int f = wave * MT + i, h = (lane >> 2) & 1;
+      xl[buf * kXWords + ((f & ~1) + h) * 64 + slot_of((f & 1) * 2 + srow, lane & 3, h)] = xp.v[i];
+    }
+  };
+  XOps xo[2];
+  // u: the parity of q. The loads stand in this order on every path into and round the loop (see above): no
+  // branch skips them (past the end they repeat the last pair), and the scheduler keeps the prologue's order.
+  auto step = [&](auto uc, int q) {
+    constexpr int u = decltype(uc)::value;
+    const bool mine = KS == 1 || q <= last;
+    if (mine) {
+      fetch(xo[1], u, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      store_x(u ^ 1);
+      load_xpart<MT>(xp, rx, xoff, min(q + 2, last));
+      compute(xo[0], ws[u & (kStages - 1)], 0, 0);
+    }
+    lds_barrier();
+    if (mine) {
+      fetch(xo[0], u ^ 1, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      compute(xo[1], ws[u & (kStages - 1)], 1, min(q + 1, last));
+      if constexpr (kStages == 2) load_w<NT>(ws[u], rw, woff, sboff, min(q + 2, last), GP);
+      close(q);
+    }
   };
   load_xpart<MT>(xp, rx, xoff, first);
+  __builtin_amdgcn_sched_barrier(0);
   load_w<NT>(ws[0], rw, woff, sboff, first, GP);
-  load_w<NT>(ws[1], rw, woff, sboff, min(first + 1, last), GP);
+  __builtin_amdgcn_sched_barrier(0);
   store_x(0);
   load_xpart<MT>(xp, rx, xoff, min(first + 1, last));
-  for (int p = 0; p < rounds; p += 2) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (p + u >= rounds) break;
-      const int q = first + p + u;
-      lds_barrier();  // pair q is staged; every wave is done with the other buffer
-      if (q < last) {
-        store_x((u + 1) & 1);
-        load_xpart<MT>(xp, rx, xoff, min(q + 2, last));
-      }
-      if (KS == 1 || q <= last) {
-        compute(xl + u * kXWords, ws[u]);
-        load_w<NT>(ws[u], rw, woff, sboff, min(q + 2, last), GP);
-        close(q);
-      }
-    }
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (kStages == 2) load_w<NT>(ws[1], rw, woff, sboff, min(first + 1, last), GP);
+  __builtin_amdgcn_sched_barrier(0);
+  lds_barrier();
+  fetch(xo[0], 0, 0);
+  int q = first;
+  for (const int even = first + (rounds & ~1); q < even; q += 2) {
+    step(IntTag<0>{}, q);
+    step(IntTag<1>{}, q + 1);
   }
+  if (rounds & 1) step(IntTag<0>{}, q);
   if constexpr (KS > 1) {
     if (S > 1 && part > 0) dump(grp);
     __syncthreads();
@@ -270,8 +335,8 @@ __global__ __launch_bounds__(256 * KS) void qmm_rows_kernel(const RowsArgs ra) {
   for (int m = 0; m < MT; ++m) {
     if (m * 16 >= rows) break;
     auto val = [&](int n, int i) {
-      if constexpr (NACC == 1) return acc[m][n][i];
-      if constexpr (NACC == 2) return grp[m][n][i];
+      if constexpr (NACC == 1 || kGrpLds) return acc[m][n][i];
+      if constexpr (NACC == 2 && kGrp) return grp[m][n][i];
       if constexpr (NACC == 3) return spl[m][n][i] + grp[m][n][i];
     };
 #pragma unroll
@@ -321,21 +386,23 @@ struct RowsForm {
 constexpr size_t kRowsMaxLds = 160 * 1024;
 constexpr int kCus = 256;
 
-// LDS slots of the parts' sums (16 MT rows x 64 NT weight rows of fp32 each).
-int rows_slots(int S, int G, int ks) { return ks == 1 ? 0 : S > 1 ? S - 1 : G - G / ks; }
+// LDS slots of the parts' sums, or of the wide wave's group sums (16 MT rows x 64 NT weight rows of fp32 each).
+int rows_slots(int S, int G, const RowsForm& f) {
+  if (f.ks == 1) return f.nt == 4 && G > 1 ? 1 : 0;
+  return S > 1 ? S - 1 : G - G / f.ks;
+}
 
 size_t rows_lds(const RowsForm& f, int S, int G) {
-  return (size_t)f.ks * 2 * f.mt * 4096 + (size_t)rows_slots(S, G, f.ks) * 4 * f.mt * f.nt * 1024;
+  return (size_t)f.ks * 2 * f.mt * 4096 + (size_t)rows_slots(S, G, f) * 4 * f.mt * f.nt * 1024;
 }
 
 int rows_blocks(int M, int N, int mt, int nt) { return ((M + 16 * mt - 1) / (16 * mt)) * ((N / 16 + 4 * nt - 1) / (4 * nt)); }
 
 template <int NT, int EPI>
 RowsForm rows_one_part(int S, int G) {
-  return {S > 1   ? qmm_rows_kernel<2, NT, 3, 1, EPI>
-          : G > 1 ? qmm_rows_kernel<2, NT, 2, 1, EPI>
-                  : qmm_rows_kernel<2, NT, 1, 1, EPI>,
-          2, NT, 1};
+  if constexpr (NT < 4)
+    if (S > 1) return {qmm_rows_kernel<2, NT, 3, 1, EPI>, 2, NT, 1};
+  return {G > 1 ? qmm_rows_kernel<2, NT, 2, 1, EPI> : qmm_rows_kernel<2, NT, 1, 1, EPI>, 2, NT, 1};
 }
 
 template <int NT, int EPI>
@@ -345,14 +412,17 @@ RowsForm rows_parts(int S, int G) {
   return {};
 }
 
-// Which form: a grid of at most one workgroup per CU leaves its 4 waves alone on their CUs, where a pair
+// Which form. A grid of at most one workgroup per CU leaves its 4 waves alone on their CUs, where a pair
 // takes about 0.7 us however few rows there are, so K is cut over the parts of a workgroup (3 for a cut of
-// 3 splits, else 4), with the narrower block while that grid still fits the CUs; from four rounds of one
-// wave per SIMD on, the 64-wide wave amortises its X reads over twice the weights. Measured on MI355X in us
-// (K x N, M: one part / parts / chosen width): 4096x2560, 64: 23.4 / 16.0 (16 NT = 16); 128: 24.4 / 16.8
-// (16); 256: 24.8 / 20.3 (32); 512: 34.6 / 39.2. 9728x2560, 130: 60.1 / 37.9 (16); 260: 63.1 / 45.3 (32);
-// 512: 78.9 / 86.2; 1024: 114 / 132. 2560x6144, 64: 16.2 / 12.4 (16); 160: 16.9 / 15.5 (32). Wide wave against
-// narrow, one part: 2560x19456 gate|up, 501: 87-97 / 96-100; 2560x151936, 64: 81-94 / 100-107.
+// 3 splits, else 4), with the narrower block while that grid still fits the CUs. Larger grids take one part; the
+// busiest CU holds ceil(blocks / CUs) of them, and a wide block (64 weight rows a wave instead of 32) costs
+// 1.72 times a narrow one: it amortises its X reads over twice the weights, and is taken where that count comes
+// out lower (from two wide blocks per CU on: alone on its CU a wide block is slower than two narrow ones).
+// Measured on MI355X in us (K x N, M: one part / parts, chosen width): 4096x2560, 64: 21.7 / 13.3 (16 NT =
+// 16); 256: 22.6 / 18.9 (32). 9728x2560, 96: 50.9 / 25.3 (16); 300: 52.8 / 37.6 (32); 400: 67.4 / 69.7. 2560x6144, 64:
+// 14.8 / 10.7 (16); 160: 15.2 / 14.0 (32). Wide block against narrow, one part: 2560x19456 gate|up, 96: 26.2 /
+// 22.0; 256: 46.9 / 46.3; 320: 50.3 / 55.8; 501: 83.8 / 96.5; 2560x8224, 509: 46.0 / 44.2; 2560x12352, 256: 33.1 /
+// 36.7; 509: 61.2 / 60.7; 2560x151936, 20: 46.4 / 43.3; 64: 84.9 / 90.5.
 template <int EPI>
 RowsForm pick_rows(int M, int N, int S, int G) {
   if constexpr (EPI != kRowsGluSplit) {
@@ -362,7 +432,8 @@ RowsForm pick_rows(int M, int N, int S, int G) {
     }
     const RowsForm f = rows_parts<2, EPI>(S, G);
     if (f.kern && rows_blocks(M, N, f.mt, f.nt) <= kCus && rows_lds(f, S, G) <= kRowsMaxLds) return f;
-    if (rows_blocks(M, N, 2, 4) >= 4 * kCus && S == 1) return rows_one_part<4, EPI>(S, G);
+    const int wide = (rows_blocks(M, N, 2, 4) + kCus - 1) / kCus, narrow = (rows_blocks(M, N, 2, 2) + kCus - 1) / kCus;
+    if (S == 1 && wide > 1 && (long long)wide * 172 < (long long)narrow * 100) return rows_one_part<4, EPI>(S, G);
   }
   return rows_one_part<2, EPI>(S, G);
 }

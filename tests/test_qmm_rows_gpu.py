@@ -54,10 +54,10 @@ def test_rows_gate_up_equal_pieces(dev, m, k, f):
 
 
 @pytest.mark.parametrize("splits,waves", [(1, 1), (1, 2), (1, 16), (2, 4), (3, 4), (4, 4)])
-@pytest.mark.parametrize("m", [40, 600])
-def test_rows_follow_the_cut(dev, splits, waves, m, monkeypatch):
+@pytest.mark.parametrize("m,n", [(40, 1040), (600, 1040), (600, 6416)])  # parts, one part, the wide wave
+def test_rows_follow_the_cut(dev, splits, waves, m, n, monkeypatch):
     """Any cut of K, also one that no table holds (19 pairs: uneven groups and splits)."""
-    k, n = 19 * 128, 1040
+    k = 19 * 128
     w, g = _weights(n, k, splits * 100 + waves, dev)
     x = torch.randn((m, k), generator=g, device=dev).to(torch.bfloat16)
     monkeypatch.setattr(Q, "SPLITK_OVERRIDE", (splits, 1, 1, waves, 2))
