@@ -30,9 +30,12 @@ from .cache import ArraysCache, KVCache, PromptCache
 from .qmm import GROUP, random_w4g64
 
 MAX_STEP = 16  # tokens per step (longer inputs: pieces of this size, or Model._prompt)
-# Inputs of at least PROMPT_MIN tokens run through the many-row kernels in blocks of up to PROMPT_BLOCK
-# tokens (Model._prompt; five 16-token passes and a capture cost about 14 ms on the 36-layer decoders, one
-# block of 80 tokens 4-5 ms).
+# Inputs of more than MAX_STEP tokens run through the many-row kernels in blocks of up to PROMPT_BLOCK
+# tokens (Model._prompt), except from PIECES_MIN to PROMPT_MIN tokens: those leave a captured 16-token pass on
+# the cache (Model._pieces), which callers may hold and replay. Measured on the 36-layer dense decoder in ms,
+# pieces / one block: 17 tokens 6.2 / 3.7, 33: 9.8 / 4.2, 48: 10.2 / 4.3, 79 (with the capture): 13.1 / 4.5; hybrid
+# and qwen35-4b alike.
+PIECES_MIN = 4 * MAX_STEP
 PROMPT_MIN = 80
 PROMPT_BLOCK = 1024
 # Forwards of at most this many tokens form each RMSNorm inside the fused projection after it (its
@@ -456,8 +459,8 @@ class Model(nn.Module):
 
     def hidden(self, ids, cache: PromptCache, tree=None) -> torch.Tensor:
         """Final normed hidden states of the tokens `ids`, appended to `cache`. Inputs longer
-        than MAX_STEP tokens run as consecutive pieces (each a full pass over the layers), or, of
-        PROMPT_MIN tokens and more on a patched model, through the many-row kernels with the same bits.
+        than MAX_STEP tokens run through the many-row kernels on a patched model (see PROMPT_MIN), else as
+        consecutive pieces (each a full pass over the layers), with the same bits.
         `tree` (skinny_mlx.tree.DraftTree) makes the tokens a draft tree instead of a chain."""
         ids = self._ids(ids)
         T = ids.shape[0]
@@ -466,7 +469,8 @@ class Model(nn.Module):
         if T > MAX_STEP:
             if self.recorder.recording or tree is not None:
                 raise ValueError("a recording or draft-tree forward takes at most MAX_STEP tokens")
-            return self._prompt(ids, cache) if T >= PROMPT_MIN and self._prompt_ok(ids) else self._pieces(ids, cache)
+            many = not PIECES_MIN <= T < PROMPT_MIN and self._prompt_ok(ids)
+            return self._prompt(ids, cache) if many else self._pieces(ids, cache)
         a = self.args
         eps = a.rms_norm_eps
         cache.begin_step(T)
@@ -545,7 +549,7 @@ class Model(nn.Module):
         time, and a capture about two passes. The remainder runs eagerly."""
         T = ids.shape[0]
         full = T // MAX_STEP if ids.is_cuda and not torch.cuda.is_current_stream_capturing() else 0
-        if full < 4:
+        if T < PIECES_MIN:
             full = 0
         outs = []
         if full:

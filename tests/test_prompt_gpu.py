@@ -9,7 +9,7 @@ import torch
 from skinny_mlx import kernels as K
 from skinny_mlx import patch as P
 from skinny_mlx.cache import make_prompt_cache
-from skinny_mlx.model import PROMPT_MIN, build_model
+from skinny_mlx.model import PIECES_MIN, PROMPT_MIN, build_model
 from skinny_mlx.spec import forward
 
 pytestmark = pytest.mark.gpu
@@ -35,10 +35,10 @@ def _state(cache, t):
 
 
 @pytest.mark.parametrize("preset", list(SMALL))
-@pytest.mark.parametrize("t,before", [(80, 0), (129, 0), (143, 17), (333, 100)])
+@pytest.mark.parametrize("t,before", [(17, 0), (33, 40), (63, 0), (80, 0), (129, 0), (143, 17), (333, 100)])
 def test_prompt_equals_pieces(preset, t, before):
     model = _model(preset)
-    assert t >= PROMPT_MIN and model._prompt_ok(model._ids([0]))
+    assert not PIECES_MIN <= t < PROMPT_MIN and model._prompt_ok(model._ids([0]))
     ids = torch.randint(0, model.args.vocab_size, (before + t,), generator=torch.Generator().manual_seed(t)).tolist()
     c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
     for c in (c1, c2):
