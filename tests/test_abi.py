@@ -367,3 +367,35 @@ def test_qmm_rows_argument_validation_on_host():
     _expect_einval(call(splits=3, groups=8), "a pair of 128 each")
     _expect_einval(call(x=ctypes.c_void_p(4104)), "misaligned")
     _expect_einval(call(m=1 << 24, n=1 << 20, ldy=1 << 20), "too large")
+
+
+def test_prompt_attention_argument_validation_on_host():
+    L = _lib.lib()
+    d, big = ctypes.c_void_p(4096), 1 << 40
+
+    def dense(qkv=d, ldq=6144, m=64, hq=32, hkv=8, dim=128, pos=d, keys=100, maxlen=1024, rope=1024, ws=d, nbytes=big):
+        return L.skinny_attention_prompt_bf16(qkv, ldq, m, hq, hkv, dim, None, None, 1e-6, d, rope, pos, keys, d, d, maxlen,
+                                              1.0, ws, nbytes, d, None)
+
+    def general(qkv=d, ldq=10240, m=64, hq=16, hkv=4, dim=256, rd=64, pos=d, keys=100, maxlen=1024, rope=1024, ws=d,
+                nbytes=big, v_offset=9216):
+        return L.skinny_attention_general_prompt_bf16(qkv, ldq, m, hq, hkv, dim, 512, 8192, v_offset, 256, None, None, 1e-6, rd,
+                                                      d, rope, pos, keys, d, d, maxlen, 1.0, ws, nbytes, d, None)
+
+    for call in (dense, general):
+        _expect_einval(call(qkv=None), "null")
+        _expect_einval(call(pos=None), "null")
+        _expect_einval(call(dim=96), "head dim 96")
+        _expect_einval(call(hq=20, hkv=8), "multiple of Hkv")
+        _expect_einval(call(hq=5, hkv=1), "query heads each")
+        _expect_einval(call(m=0), "M=0")
+        _expect_einval(call(m=65536, keys=65536, maxlen=65536, rope=65536), "at most 65535")
+        _expect_einval(call(keys=63), "keys=63")
+        _expect_einval(call(keys=1025), "keys=1025")
+        _expect_einval(call(maxlen=1000), "maxlen=1000")
+        _expect_einval(call(rope=512), "RoPE table")
+        _expect_einval(call(ws=ctypes.c_void_p(4104)), "aligned")
+        _expect_einval(call(nbytes=4096), "workspace")
+    _expect_einval(dense(ldq=6136), "ldq")
+    _expect_einval(general(rd=63), "rotary_dim")
+    _expect_einval(general(v_offset=9472), "do not fit")
