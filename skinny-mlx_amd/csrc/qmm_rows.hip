@@ -21,14 +21,15 @@
 // per SIMD for the wide wave, that took 2560x19456 at 501 rows from 81 to 77 us, 9728x2560 at 1024 rows from 106
 // to 95 and at 96 rows from 33 to 25 (VALU active 67% of the CUs' busy time before, 86% after). MT = 4 saves a fifth
 // of the instructions but leaves two waves per SIMD, and was slower everywhere (2560x19456, 501 rows: 95 us).
+// MT = 3 serves grids that fit the CUs with blocks of 48 rows and not with 32 (pick_rows).
 #include "qmm_frag.h"
 
 namespace {
 
 enum RowsEpi { kRowsPlain = 0, kRowsGluSplit = 1, kRowsSwiGlu = 2 };
 
-// X of one pair for this wave's share of the 16 MT rows: fragment f = 4 mt + 2 j + h of the pair (lane
-// 16 quad + tok: row 16 mt + tok, columns 64 j + 32 h + 8 quad ..), MT fragments per wave.
+// X of one pair for this wave's share of the 16 MT rows: MT loads of 16 bytes per lane. Staged, fragment
+// 4 mt + 2 j + h of the pair holds rows 16 mt + tok and columns 64 j + 32 h + 8 quad ... for lane 16 quad + tok.
 template <int MT>
 struct XPart {
   u32x4_t v[MT];
@@ -105,11 +106,11 @@ __global__ __launch_bounds__(256 * KS, NT == 4 ? 3 : 1) void qmm_rows_kernel(con
   const bf16x8_t ones = ones_operand();
   u32x4_t* const xl = reinterpret_cast<u32x4_t*>(lds) + part * 2 * kXWords;
   float* const sums = reinterpret_cast<float*>(lds + (size_t)KS * 2 * kXWords * 16);
-  // This wave stages fragments wave MT .. + MT - 1 of its part's pairs, two (the 64 columns of a scale group)
-  // at a time as 8 rows of 128 bytes per load. Rows past M carry an out-of-range offset and read as zeros.
+  // A load takes 8 rows of a scale group's 64 columns, 128 bytes each: half the rows of two fragments (load f: row tile
+  // f / 4, group f / 2 % 2). This wave does loads wave MT .. + MT - 1. Rows past M carry an out-of-range offset and
+  // read as zeros.
   // Lane group g = lane / 8 takes rows 4 (g % 4) + g / 4 and two below, and a fragment's quad holds its rows in
   // the order t ^ quad ^ 12 h: so both the 16 lanes of a read and any 16 of a write fall on different banks.
-  static_assert(MT % 2 == 0, "a wave stages pairs of fragments");
   auto slot_of = [](int t, int qd, int h) { return qd * 16 + (t ^ qd ^ (12 * h)); };
   const int srow = ((lane >> 3) & 3) * 4 + (lane >> 5);
   uint32_t xoff[MT];
@@ -412,14 +413,25 @@ RowsForm rows_parts(int S, int G) {
   return {};
 }
 
+// As rows_parts with 48 rows a block; one split's groups in two parts, whose eight waves have the registers of two
+// per SIMD.
+template <int EPI>
+RowsForm rows_parts48(int S, int G) {
+  if (S == 3) return {qmm_rows_kernel<3, 2, 2, 3, EPI>, 3, 2, 3};
+  if (S == 1 && G >= 2) return {qmm_rows_kernel<3, 2, 2, 2, EPI>, 3, 2, 2};
+  return {};
+}
+
 // Which form. A grid of at most one workgroup per CU leaves its 4 waves alone on their CUs, where a pair
 // takes about 0.7 us however few rows there are, so K is cut over the parts of a workgroup (3 for a cut of
-// 3 splits, else 4), with the narrower block while that grid still fits the CUs. Larger grids take one part; the
+// 3 splits, else 4), with the narrowest block whose grid still fits the CUs: 16 NT = 16 and 32, then 48 rows of 32
+// (a second workgroup on some CUs would double the time). Larger grids take one part; the
 // busiest CU holds ceil(blocks / CUs) of them, and a wide block (64 weight rows a wave instead of 32) costs
 // 1.72 times a narrow one: it amortises its X reads over twice the weights, and is taken where that count comes
 // out lower (from two wide blocks per CU on: alone on its CU a wide block is slower than two narrow ones).
 // Measured on MI355X in us (K x N, M: one part / parts, chosen width): 4096x2560, 64: 21.7 / 13.3 (16 NT =
-// 16); 256: 22.6 / 18.9 (32). 9728x2560, 96: 50.9 / 25.3 (16); 300: 52.8 / 37.6 (32); 400: 67.4 / 69.7. 2560x6144, 64:
+// 16); 256: 22.6 / 18.9 (32). 9728x2560, 96: 50.9 / 25.3 (16); 300: 52.8 / 37.6 (32); 400: 67.6 / 45.2 (48 rows); 509: 65.0 / 45.8 (48
+// rows). 4096x2560, 509: 29.1 / 23.6 (48 rows); 2048x2560, 509: 17.2 / 15.1 (48 rows). 2560x6144, 64:
 // 14.8 / 10.7 (16); 160: 15.2 / 14.0 (32). Wide block against narrow, one part: 2560x19456 gate|up, 96: 26.2 /
 // 22.0; 256: 46.9 / 46.3; 320: 50.3 / 55.8; 501: 83.8 / 96.5; 2560x8224, 509: 46.0 / 44.2; 2560x12352, 256: 33.1 /
 // 36.7; 509: 61.2 / 60.7; 2560x151936, 20: 46.4 / 43.3; 64: 84.9 / 90.5.
@@ -432,6 +444,8 @@ RowsForm pick_rows(int M, int N, int S, int G) {
     }
     const RowsForm f = rows_parts<2, EPI>(S, G);
     if (f.kern && rows_blocks(M, N, f.mt, f.nt) <= kCus && rows_lds(f, S, G) <= kRowsMaxLds) return f;
+    const RowsForm f48 = rows_parts48<EPI>(S, G);
+    if (f48.kern && rows_blocks(M, N, f48.mt, f48.nt) <= kCus && rows_lds(f48, S, G) <= kRowsMaxLds) return f48;
     const int wide = (rows_blocks(M, N, 2, 4) + kCus - 1) / kCus, narrow = (rows_blocks(M, N, 2, 2) + kCus - 1) / kCus;
     if (S == 1 && wide > 1 && (long long)wide * 172 < (long long)narrow * 100) return rows_one_part<4, EPI>(S, G);
   }
@@ -453,7 +467,7 @@ extern "C" int skinny_qmm_w4g64_rows_bf16(const uint16_t* x, int M, int K, int l
   SKINNY_CHECK_ARG(splits >= 1 && groups >= 1 && (K / 128) / splits >= groups,
                    "qmm rows: %d splits of %d groups need a pair of 128 each (K=%d)", splits, groups, K);
   SKINNY_CHECK_ARG(skinny_aligned(x, 16) && skinny_aligned(w_frag, 16) && skinny_aligned(y, 2), "qmm rows: misaligned buffer");
-  SKINNY_CHECK_ARG((size_t)32 * ldx * 2 < 0x7ff00000u && (size_t)4 * (K / 128) * kBlockBytes < 0x40000000u,
+  SKINNY_CHECK_ARG((size_t)48 * ldx * 2 < 0x7ff00000u && (size_t)4 * (K / 128) * kBlockBytes < 0x40000000u,
                    "qmm rows: rows too long for a buffer descriptor");
   // 32-row x 128-weight blocks of 256 threads: the grid stays below 2^32 threads
   SKINNY_CHECK_ARG(((size_t)M / 32 + 1) * ((size_t)N / 128 + 1) < (1u << 23), "qmm rows: M=%d x N=%d is too large for one launch",

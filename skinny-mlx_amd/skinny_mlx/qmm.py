@@ -288,7 +288,7 @@ def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = N
     L = _lib.lib()
     stream = _lib.stream_of(x2)
     splits, tile = _plain_config(k, n)
-    if m >= rows_from(n, splits) and not CONFIG_OVERRIDE and not SPLITK_OVERRIDE:
+    if m >= rows_from(n, splits) and x2.stride(0) <= _ROWS_MAX_LD and not CONFIG_OVERRIDE and not SPLITK_OVERRIDE:
         _rows(x2, w, y, splits, tile, EPI_PLAIN, "skinny_qmm")
         return _like_rows(y, x, n)
     if splits > 1:
@@ -309,7 +309,8 @@ def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = N
 EPI_PLAIN, EPI_GLU_SPLIT, EPI_SWIGLU = 0, 1, 2
 _ROWS_MAX = 16384
 _ROWS_WIDE_N = 8192
-_ROWS_MAX_N = 1 << 20  # one launch's grid
+_ROWS_MAX_N = 1 << 20   # one launch's grid
+_ROWS_MAX_LD = 1 << 24  # 48 rows of x in one buffer descriptor
 
 
 def rows_from(n: int, splits: int) -> int:
@@ -742,7 +743,7 @@ def skinny_glu(x: torch.Tensor, w: torch.Tensor, swiglu: bool, out: torch.Tensor
             raise ValueError(f"out must be bf16 [M, {width}] with unit inner stride")
         y = out
     tile = glu_tile(k, f)
-    if m >= rows_from(2 * f, 1):
+    if m >= rows_from(2 * f, 1) and x2.stride(0) <= _ROWS_MAX_LD:
         _rows(x2, w, y, 1, tile, EPI_SWIGLU if swiglu else EPI_GLU_SPLIT, "skinny_glu")
         return _like_rows(y, x, width)
     L = _lib.lib()

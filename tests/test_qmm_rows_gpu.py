@@ -23,10 +23,10 @@ def _same(a, b):
 
 
 # (rows, K, N): the least K and N; weight tiles that do not fill a block; the decoders' shapes at each
-# form's row counts (o_proj: 4 parts narrow, 4 parts wide, one part; down: 3 parts narrow, wide, one part
-# with three sums; q|k|v; gate|up-wide and the head: the 64-wide wave)
+# form's row counts (o_proj: 4 parts narrow, 4 parts wide, 2 parts of 48 rows, one part; down: 3 parts narrow, wide, 3
+# parts of 48 rows, one part with three sums; q|k|v; gate|up-wide and the head: the 64-wide wave)
 SHAPES = [(17, 128, 16), (33, 256, 48), (47, 384, 80), (64, 256, 512), (65, 640, 272), (33, 4096, 2560), (200, 4096, 2560),
-          (450, 4096, 2560), (65, 9728, 2560), (250, 9728, 2560), (401, 9728, 2560), (77, 2560, 6144), (450, 2560, 19456),
+          (450, 4096, 2560), (700, 4096, 2560), (65, 9728, 2560), (250, 9728, 2560), (401, 9728, 2560), (700, 9728, 2560), (77, 2560, 6144), (450, 2560, 19456),
           (33, 2560, 151936)]
 
 
@@ -54,7 +54,7 @@ def test_rows_gate_up_equal_pieces(dev, m, k, f):
 
 
 @pytest.mark.parametrize("splits,waves", [(1, 1), (1, 2), (1, 16), (2, 4), (3, 4), (4, 4)])
-@pytest.mark.parametrize("m,n", [(40, 1040), (600, 1040), (600, 6416)])  # parts, one part, the wide wave
+@pytest.mark.parametrize("m,n", [(40, 1040), (600, 1040), (600, 2064), (600, 6416)])  # parts, of 48 rows, the wide wave
 def test_rows_follow_the_cut(dev, splits, waves, m, n, monkeypatch):
     """Any cut of K, also one that no table holds (19 pairs: uneven groups and splits)."""
     k = 19 * 128
