@@ -90,9 +90,11 @@ __global__ __launch_bounds__(64 * kWaves) void attn_chunk_kernel(const int32_t* 
 // on CUs of their own). What bounds it at a long context is the read of K and V^T; at a short one the chain
 // position, chunk, partial, merge. Measured on MI355X, one token, chunk stage and merge of a layer: 32768 keys
 // 41.6 -> 36.7 us (3.66 TB/s of KV; with it, partials of the live rows only and eight merge waves); 2048 keys
-// level (9.8 us); 256-dim heads (general_few_kernel) 512 / 2000 / 5003 keys 10.6 / 11.9 / 16.6 -> 10.5 / 11.5 /
+// level (9.8 us); caches of 256 / 512 / 1280 slots 9.58 / 9.75 / 9.95 -> 9.73 / 9.93 / 10.05, so up to kFewChunks
+// chunks stay staged; 256-dim heads (general_few_kernel) 512 / 2000 / 5003 keys 10.6 / 11.9 / 16.6 -> 10.5 / 11.5 /
 // 15.2 us. With more rows per kv head several waves of a staged chunk have work, and staging serves them all.
 constexpr int kFewRows = 16;
+constexpr int kFewChunks = 12;        // caches of up to this many chunks stay staged
 constexpr int kFewMaxlen = 1 << 22;  // V^T of a head within a buffer descriptor
 
 __device__ __forceinline__ void attn_direct_chunk(int c, int h, int p0, const uint16_t* __restrict__ q, const FusedArgs& fa,
@@ -595,7 +597,7 @@ static int attention_fused(const uint16_t* qkv, int ldq, int M, int Hq, int Hkv,
   float* part_o = workspace;
   float* part_ml = workspace + (size_t)Hkv * nch * kRowsMax * kD;
   const FusedArgs fa{ldq, q_norm, k_norm, eps, rope_table};
-  if ((Hq / Hkv) * M <= kFewRows && maxlen <= kFewMaxlen) {
+  if ((Hq / Hkv) * M <= kFewRows && nch > kFewChunks && maxlen <= kFewMaxlen) {
     const int per = nch * Hkv <= 512 ? 1 : nch * Hkv <= 1024 ? 2 : kWaves;
     hipLaunchKernelGGL(attn_few_kernel, dim3(2 + (nch + per - 1) / per, Hkv), dim3(64 * kWaves), 0, (hipStream_t)stream, pos0,
                        qkv, fa, M, Hq, Hkv, k_cache, vt_cache, maxlen, scale, tree, part_o, part_ml, nch, per);

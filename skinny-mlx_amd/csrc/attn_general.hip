@@ -74,8 +74,6 @@ __global__ __launch_bounds__(64) void general_qk_store_kernel(const int32_t* __r
   uint16_t raw[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) raw[e] = src[lane + 64 * e];
-  const int half = R >> 1;
-  const uint16_t* nw = head < Hq ? qn : kn;
   if (head >= Hq + Hkv) {  // value: into the transposed cache as it is
     const int h = head - Hq - Hkv;
 #pragma unroll
@@ -89,14 +87,17 @@ __global__ __launch_bounds__(64) void general_qk_store_kernel(const int32_t* __r
     x[e] = bf16_bits_to_f32(raw[e]);
     ss = fmaf(x[e], x[e], ss);
   }
+  const uint16_t* nw = head < Hq ? qn : kn;
   if (nw) {
     const float inv = rsqrtf(wave_sum(ss) / (float)D + eps);
 #pragma unroll
-    for (int e = 0; e < E; ++e) x[e] = bf16_bits_to_f32(f32_to_bf16_bits(x[e] * inv * bf16_bits_to_f32(nw[lane + 64 * e])));
+    for (int e = 0; e < E; ++e)
+      x[e] = bf16_bits_to_f32(f32_to_bf16_bits(x[e] * inv * bf16_bits_to_f32(nw[lane + 64 * e])));
   }
 #pragma unroll
   for (int e = 0; e < E; ++e) row[lane + 64 * e] = x[e];
   __syncthreads();
+  const int half = R >> 1;
   uint16_t outv[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) {

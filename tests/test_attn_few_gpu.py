@@ -11,8 +11,8 @@ from skinny_mlx.tree import DraftTree
 
 pytestmark = pytest.mark.gpu
 
-# (kv heads, cache slots, cached tokens): chunks x heads <= 512, <= 1024, past it
-CASES = [(2, 1024, 0), (2, 1024, 100), (2, 1024, 250), (8, 8192, 5000), (8, 12288, 12200), (8, 33024, 32765)]
+# (kv heads, cache slots, cached tokens): the dense layout staged; chunks x heads <= 512, <= 1024, past it
+CASES = [(2, 1024, 100), (2, 2048, 0), (2, 2048, 100), (2, 2048, 250), (8, 8192, 5000), (8, 12288, 12200), (8, 33024, 32765)]
 
 
 def _call(layout, rnd, dev, hkv, maxlen):
