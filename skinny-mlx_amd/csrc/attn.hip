@@ -185,11 +185,12 @@ __global__ __launch_bounds__(64 * kWaves) void attn_few_kernel(const int32_t* __
   const int p0 = pos0[0];
   const int fresh = p0 / kChunk;  // the first chunk with new slots
   if (b < 2) {
+    if ((unsigned)(fresh + b) >= (unsigned)nchunk_max) return;  // slots past the cache are dropped, as the staged grid has none
     attn_chunk_body<true>(fresh + b, h, pos0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
     return;
   }
   const int c = (b - 2) * per + wave;
-  if (c >= fresh) return;
+  if (c >= min(fresh, nchunk_max)) return;
   attn_direct_chunk(c, h, p0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
 }
 
@@ -236,8 +237,8 @@ __device__ __forceinline__ bool combine_row(const float* __restrict__ part_o, co
     }
   }
   const int total = pos0[0] + tokens;
-  // (a prompt's workspace holds the chunks its caller named; no read past them whatever *pos0 says)
-  const int nch = kPrompt ? min((total + kChunk - 1) / kChunk, nchunk_max) : (total + kChunk - 1) / kChunk;
+  // (the workspace holds nchunk_max chunks; no read past them whatever *pos0 says)
+  const int nch = min((total + kChunk - 1) / kChunk, nchunk_max);
   float run_m = -INFINITY, run_l = 0.f, a0 = 0.f, a1 = 0.f;
   for (int c0 = first; c0 < nch; c0 += W * kCombineBlock) {
     const int nb = min(kCombineBlock, nch - c0);

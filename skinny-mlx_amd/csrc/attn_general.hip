@@ -240,7 +240,7 @@ __global__ __launch_bounds__(64 * kGWaves, 2) void general_few_kernel(const int3
   const int c = (int)blockIdx.x * per + wave;
   const int p0 = pos0[0];
   const int key0 = c * CH;
-  if (key0 >= p0 + M) return;
+  if (c >= nchunk_max || key0 >= p0 + M) return;  // the last workgroup's waves may lie past the cache
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
   const int G = Hq / Hkv;
   const bool live = col < G * M;

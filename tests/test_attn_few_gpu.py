@@ -66,3 +66,32 @@ def test_few_rows_of_a_tree(dev, layout, past):
     a = call(qkv, pos, k0.clone(), v0.clone(), DraftTree(parents, dev).desc)
     b = call(qkv[:4], pos, k0.clone(), v0.clone(), DraftTree(parents[:4], dev).desc)
     assert torch.equal(a[:4], b)
+
+
+def test_few_rows_past_the_cache_are_dropped(dev):
+    """A step that begins at the cache's last two slots with four tokens (no caller of the package lets it):
+    the tokens without a slot are dropped, as in a step over staged chunks. Nothing lands in the next head's
+    rows (slot 2048 of a head is slot 0 of the next) or after the last head's, and the rows are the staged
+    step's. The RoPE table covers the positions; caches and workspace have guards behind them."""
+    hkv, maxlen, past, d = 2, 2048, 2046, 128
+    hq, m, guard = 4 * hkv, 4, 1 << 16
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev).to(torch.bfloat16)
+    qkv, table = rnd(16, (hq + 2 * hkv) * d), K.rope_table(1e6, maxlen + 128, dev)
+    k0, v0 = rnd(hkv * maxlen * d + guard), rnd(hkv * maxlen * d + guard)
+    pos = torch.tensor([past], dtype=torch.int32, device=dev)
+    words = K.attn_workspace(hkv, maxlen, dev).numel()
+    got = []
+    for rows in (m, 16):  # few rows; staged chunks
+        k, vt = k0.clone(), v0.clone()
+        ws = torch.full((words + guard,), -7.0, device=dev)
+        kc, vc = k[:-guard].view(hkv, maxlen, d), vt[:-guard].view(hkv, d, maxlen)
+        out = K.attention_fused(qkv[:rows], hq, hkv, d, None, None, 1e-6, table, pos, kc, vc, d ** -0.5, ws[:words], None)
+        assert (ws[words:] == -7).all() and torch.equal(k[-guard:], k0[-guard:]) and torch.equal(vt[-guard:], v0[-guard:])
+        got.append((out[:m], k, vt))
+    (a, k, vt), (b, k2, vt2) = got
+    assert torch.equal(a, b) and torch.equal(k, k2) and torch.equal(vt, vt2)
+    want_k, want_v = k0[:-guard].view(hkv, maxlen, d).clone(), v0[:-guard].view(hkv, d, maxlen).clone()
+    want_v[:, :, past:] = qkv[:2, (hq + hkv) * d:].view(2, hkv, d).permute(1, 2, 0)
+    assert torch.equal(vt[:-guard].view(hkv, d, maxlen), want_v)
+    assert torch.equal(k[:-guard].view(hkv, maxlen, d)[:, :past], want_k[:, :past])
