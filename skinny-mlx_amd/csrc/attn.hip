@@ -85,14 +85,16 @@ __global__ __launch_bounds__(64 * kWaves) void attn_chunk_kernel(const int32_t* 
 // each wave takes a chunk of its own, its K and V^T fragments straight from memory into registers (the
 // same fragments, MFMAs and softmax, so the partials are bitwise attn_chunk_body's). Nothing waits at a
 // barrier, and a CU holds 8 chunks' loads in flight instead of 2. Only chunks without new tokens are taken
-// this way: workgroups 0 and 1 of a head run attn_chunk_body over the chunks that hold the new slots,
-// workgroup 2 + g the chunks g * per .. below them, one per wave (per = 1 keeps a short context's chunks
-// on CUs of their own). What bounds it at a long context is the read of K and V^T; at a short one the chain
-// position, chunk, partial, merge. Measured on MI355X, one token, chunk stage and merge of a layer: 32768 keys
-// 41.6 -> 36.7 us (3.66 TB/s of KV; with it, partials of the live rows only and eight merge waves); 2048 keys
-// level (9.8 us); caches of 256 / 512 / 1280 slots 9.58 / 9.75 / 9.95 -> 9.73 / 9.93 / 10.05, so up to kFewChunks
-// chunks stay staged; 256-dim heads (general_few_kernel) 512 / 2000 / 5003 keys 10.6 / 11.9 / 16.6 -> 10.5 / 11.5 /
-// 15.2 us. With more rows per kv head several waves of a staged chunk have work, and staging serves them all.
+// this way: workgroups 0 and 1 of a head run attn_chunk_body over the chunks that hold the new slots, the n
+// others the chunks below them, 1, 2 or 4 each. The grid is sized for a full cache; how many of its waves a
+// workgroup uses goes by the context, so that a short context's chunks in a long cache are on CUs of their own
+// (4 in every workgroup: 4000 keys in a cache of 32896 slots 14.7 us a layer, spread 12.9; 13.6 staged). What bounds
+// it at a long context is the read of K and V^T; at a short one the chain position, chunk, partial, merge.
+// Measured on MI355X, one token, chunk stage and merge of a layer, staged against this: 32768 keys 41.2 / 36.7 us
+// (3.66 TB/s of KV; with it, partials of the live rows only and eight merge waves); 8000 keys of 8192 slots 14.0 /
+// 13.3; 2000 of 4096 9.6 / 9.4; but 4000 of 4096 10.9 / 11.3, 60 in 2048 or 4224 slots 8.8 / 8.9 and 9.1 / 9.2, and
+// caches of 256 / 512 / 1280 slots 9.58 / 9.75 / 9.95 against 9.73 / 9.93 / 10.05: up to kFewChunks chunks stay
+// staged. With more rows per kv head several waves of a staged chunk have work, and staging serves them all.
 constexpr int kFewRows = 16;
 constexpr int kFewChunks = 12;        // caches of up to this many chunks stay staged
 constexpr int kFewMaxlen = 1 << 22;  // V^T of a head within a buffer descriptor
@@ -179,18 +181,18 @@ __global__ __launch_bounds__(64 * kWaves) void attn_few_kernel(const int32_t* __
                                                                int Hkv, uint16_t* __restrict__ kc, uint16_t* __restrict__ vt,
                                                                int maxlen, float scale, const int32_t* __restrict__ tree,
                                                                float* __restrict__ part_o, float* __restrict__ part_ml,
-                                                               int nchunk_max, int per) {
+                                                               int nchunk_max, int n) {
   const int b = blockIdx.x, h = blockIdx.y, wave = wave_id();
-  if (b >= 2 && wave >= per) return;
   const int p0 = pos0[0];
   const int fresh = p0 / kChunk;  // the first chunk with new slots
+  const int sh = fresh > 2 * n ? 2 : fresh > n ? 1 : 0;
+  const int c = ((b - 2) << sh) + wave;
+  if (b >= 2 && ((wave >> sh) || c >= min(fresh, nchunk_max))) return;
   if (b < 2) {
     if ((unsigned)(fresh + b) >= (unsigned)nchunk_max) return;  // slots past the cache are dropped, as the staged grid has none
     attn_chunk_body<true>(fresh + b, h, pos0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
     return;
   }
-  const int c = (b - 2) * per + wave;
-  if (c >= min(fresh, nchunk_max)) return;
   attn_direct_chunk(c, h, p0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
 }
 
@@ -599,9 +601,9 @@ static int attention_fused(const uint16_t* qkv, int ldq, int M, int Hq, int Hkv,
   float* part_ml = workspace + (size_t)Hkv * nch * kRowsMax * kD;
   const FusedArgs fa{ldq, q_norm, k_norm, eps, rope_table};
   if ((Hq / Hkv) * M <= kFewRows && nch > kFewChunks && maxlen <= kFewMaxlen) {
-    const int per = nch * Hkv <= 512 ? 1 : nch * Hkv <= 1024 ? 2 : kWaves;
-    hipLaunchKernelGGL(attn_few_kernel, dim3(2 + (nch + per - 1) / per, Hkv), dim3(64 * kWaves), 0, (hipStream_t)stream, pos0,
-                       qkv, fa, M, Hq, Hkv, k_cache, vt_cache, maxlen, scale, tree, part_o, part_ml, nch, per);
+    const int per = nch * Hkv <= 512 ? 1 : nch * Hkv <= 1024 ? 2 : kWaves, n = (nch + per - 1) / per;
+    hipLaunchKernelGGL(attn_few_kernel, dim3(2 + n, Hkv), dim3(64 * kWaves), 0, (hipStream_t)stream, pos0, qkv, fa, M, Hq, Hkv,
+                       k_cache, vt_cache, maxlen, scale, tree, part_o, part_ml, nch, n);
   } else {
     hipLaunchKernelGGL(attn_chunk_kernel<true>, dim3(nch, Hkv), dim3(64 * kWaves), 0, (hipStream_t)stream, pos0, qkv, fa, M,
                        Hq, Hkv, k_cache, vt_cache, maxlen, scale, tree, part_o, part_ml, nch);

@@ -219,28 +219,130 @@ __device__ __forceinline__ void general_rows(const uint16_t* ks_lds, const uint1
   general_store_rows<D>(o, mx, sum, rows, rows_o, rows_ml);
 }
 
-// (2, few rows) A step of at most 16 query rows per kv head: as attn.hip's attn_few_kernel, each wave takes
-// a chunk of its own with its K and V^T fragments straight from memory (the new rows are in the caches
-// already), `per` chunks per workgroup; partials bitwise general_chunk_kernel's.
-constexpr int kGFewRows = 16;
-constexpr int kGFewMaxlen = 1 << 21;  // V^T of a head within a buffer descriptor
+// (2) Workgroup (chunk c, kv head h), keys [CH c, CH c + CH); wave w takes the query rows
+// 16w .. 16w + 15 of the (token, group head) rows. attn.hip's chunk kernel over D dims: every thread
+// issues its 16-byte pieces of the chunk's K rows and V^T rows at once (PIECES of each), they go to
+// LDS (pitches D + 8 and CH + 8: the 16 rows one 16-byte read spans fall on distinct banks), and the
+// busy waves compute S^T = K Q^T with the K rows of tile kt taken in the order row r -> key
+// 32(kt/2) + 8(r/4) + 4(kt%2) + r%4, so that lane (col, quad) holds the keys 32s + 8quad + 0..7 of
+// its query row and its bf16 P is the A operand of P.V; base-2 exponents with log2(e) in the scale.
+template <int D>
+__device__ __forceinline__ void general_chunk_body(int c, int h, const int32_t* __restrict__ pos0,
+                                                   const uint16_t* __restrict__ q, int M, int Hq, int Hkv,
+                                                   const uint16_t* __restrict__ kc, const uint16_t* __restrict__ vt, int maxlen,
+                                                   float scale, const int32_t* __restrict__ tree, float* __restrict__ part_o,
+                                                   float* __restrict__ part_ml, int nchunk_max) {
+  constexpr int CH = general_chunk(D);
+  constexpr int KS = D / 32;  // 32-dim steps of a score
+  constexpr int KP = D + 8, VP = CH + 8;
+  constexpr int PIECES = CH * D / 8 / (64 * kGWaves);  // 16-byte pieces per thread of K, and of V^T
+  static_assert(PIECES * 8 * 64 * kGWaves == CH * D, "the chunk splits evenly over the threads");
+  __shared__ __attribute__((aligned(16))) uint16_t ks_lds[CH * KP];  // K rows: [key][dim]
+  __shared__ __attribute__((aligned(16))) uint16_t vs_lds[D * VP];   // V^T rows: [dim][key]
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int p0 = pos0[0];
+  const int total = p0 + M;
+  const int key0 = c * CH;
+  if (key0 >= total) return;
+  const int G = Hq / Hkv;
+  const int rows = G * M;
+  const bool busy = wave * 16 < rows;
+  const int col = lane & 15, quad = lane >> 4;
+  const int qrow = wave * 16 + col;
+  const bool live = busy && qrow < rows;
+  const int t = live ? qrow / G : 0;
+  // Loads in the order their data is needed: the query row (B operand), the tree words, the chunk.
+  bf16x8_t qf[KS];
+  if (live) {
+    const uint16_t* qr = q + ((size_t)t * Hq + h * G + qrow % G) * D;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8_t*>(qr + ks * 32 + quad * 8);
+  } else {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = bf16x8_t{};
+  }
+  int tree0 = 0, tree_mask = 0;
+  if (tree) {
+    tree0 = tree[0];
+    tree_mask = tree[1 + t];
+  }
+  const u32x4_t* kh = reinterpret_cast<const u32x4_t*>(kc + ((size_t)h * maxlen + key0) * D);
+  const uint16_t* vh = vt + (size_t)h * D * maxlen + key0;
+  u32x4_t kr[PIECES], vr[PIECES];
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int e = threadIdx.x + i * 64 * kGWaves;  // K piece e: row e / (D/8); V^T piece e: row e / (CH/8)
+    kr[i] = kh[e];
+    vr[i] = *reinterpret_cast<const u32x4_t*>(vh + (size_t)(e / (CH / 8)) * maxlen + (e % (CH / 8)) * 8);
+  }
+  // Visibility of key kp for this lane's row: with j = kp - tbase, visible iff j < 0, or j < 32
+  // and bit j of tmask. Causal: tbase = p0 + t + 1, tmask = 0; a draft tree: the tree's first slot
+  // and the token's ancestor mask; a padding row sees nothing.
+  int tbase = key0;
+  uint32_t tmask = 0;
+  if (live) {
+    tbase = tree ? p0 - tree0 : p0 + t + 1;
+    tmask = tree ? (uint32_t)tree_mask : 0u;
+  }
+#pragma unroll
+  for (int i = 0; i < PIECES; ++i) {
+    const int e = threadIdx.x + i * 64 * kGWaves;
+    *reinterpret_cast<u32x4_t*>(&ks_lds[(e / (D / 8)) * KP + (e % (D / 8)) * 8]) = kr[i];
+    *reinterpret_cast<u32x4_t*>(&vs_lds[(e / (CH / 8)) * VP + (e % (CH / 8)) * 8]) = vr[i];
+  }
+  __syncthreads();
+  if (!busy) return;
+
+  const size_t base = ((size_t)h * nchunk_max + c) * kGRowsMax + wave * 16;
+  general_rows<D>(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, rows - wave * 16, part_o + base * D, part_ml + base * 2);
+}
 
 template <int D>
+__global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32_t* __restrict__ pos0,
+                                                                     const uint16_t* __restrict__ q, int M, int Hq,
+                                                                     int Hkv, const uint16_t* __restrict__ kc,
+                                                                     const uint16_t* __restrict__ vt, int maxlen,
+                                                                     float scale, const int32_t* __restrict__ tree,
+                                                                     float* __restrict__ part_o,
+                                                                     float* __restrict__ part_ml, int nchunk_max) {
+  general_chunk_body<D>((int)blockIdx.x, (int)blockIdx.y, pos0, q, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml,
+                        nchunk_max);
+}
+
+// (2, few rows) A step of at most 16 query rows per kv head: as attn.hip's attn_few_kernel, each wave takes
+// a chunk of its own with its K and V^T fragments straight from memory (the new rows are in the caches
+// already), 1, 2 or 4 chunks in each of n workgroups by the context; partials bitwise general_chunk_kernel's. In a
+// long cache (kStage) up to kGFewStaged chunks in all, one per CU, are staged by all waves of a workgroup instead:
+// rows of V^T many KB apart come slowly to one wave. 256-dim heads, one token, us a layer, every chunk staged / a chunk per
+// wave / as here: 1000 keys in 8192 slots 11.3 / 12.3 / 11.6, in 32896 10.7 / 11.9 / 11.1, 4000 in 32896 14.7 / 14.2 /
+// 14.2; 8000 in 8192 19.5 / 16.5 / 16.6; 32768 in 33024 62 / 48.6 / 48.7. Smaller caches take a chunk per wave
+// throughout: 1000 / 2000 / 4000 keys in 4096 slots 10.5 / 11.5 / 13.8 staged, 10.4 / 11.1 / 12.7.
+constexpr int kGFewRows = 16;
+constexpr int kGFewStaged = 256;      // a long cache's chunks x kv heads up to which they are staged
+constexpr int kGFewMaxlen = 1 << 21;  // V^T of a head within a buffer descriptor
+
+template <int D, bool kStage>
 __global__ __launch_bounds__(64 * kGWaves, 2) void general_few_kernel(const int32_t* __restrict__ pos0,
                                                                       const uint16_t* __restrict__ q, int M, int Hq,
                                                                       int Hkv, const uint16_t* __restrict__ kc,
                                                                       const uint16_t* __restrict__ vt, int maxlen,
                                                                       float scale, const int32_t* __restrict__ tree,
                                                                       float* __restrict__ part_o,
-                                                                      float* __restrict__ part_ml, int nchunk_max, int per) {
+                                                                      float* __restrict__ part_ml, int nchunk_max, int n) {
   constexpr int CH = general_chunk(D);
   constexpr int KS = D / 32, DT = D / 16, KT = CH / 16, PS = CH / 32;
   constexpr int VPT = DT * PS / KT;  // V^T fragments issued per K tile
   const int h = blockIdx.y, wave = wave_id();
-  const int c = (int)blockIdx.x * per + wave;
   const int p0 = pos0[0];
+  const int nch = min((p0 + M + CH - 1) / CH, nchunk_max), sh = nch > 2 * n ? 2 : nch > n ? 1 : 0;
+  if (kStage && nch * Hkv <= kGFewStaged) {
+    if ((int)blockIdx.x < nch)
+      general_chunk_body<D>((int)blockIdx.x, h, pos0, q, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
+    return;
+  }
+  const int c = ((int)blockIdx.x << sh) + wave;
+  if ((wave >> sh) || c >= nch) return;
   const int key0 = c * CH;
-  if (c >= nchunk_max || key0 >= p0 + M) return;  // the last workgroup's waves may lie past the cache
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
   const int G = Hq / Hkv;
   const bool live = col < G * M;
@@ -301,87 +403,6 @@ __global__ __launch_bounds__(64 * kGWaves, 2) void general_few_kernel(const int3
   }
   const size_t base = ((size_t)h * nchunk_max + c) * kGRowsMax;
   general_store_rows<D>(o, mx, sum, G * M, part_o + base * D, part_ml + base * 2);
-}
-
-// (2) Workgroup (chunk c, kv head h), keys [CH c, CH c + CH); wave w takes the query rows
-// 16w .. 16w + 15 of the (token, group head) rows. attn.hip's chunk kernel over D dims: every thread
-// issues its 16-byte pieces of the chunk's K rows and V^T rows at once (PIECES of each), they go to
-// LDS (pitches D + 8 and CH + 8: the 16 rows one 16-byte read spans fall on distinct banks), and the
-// busy waves compute S^T = K Q^T with the K rows of tile kt taken in the order row r -> key
-// 32(kt/2) + 8(r/4) + 4(kt%2) + r%4, so that lane (col, quad) holds the keys 32s + 8quad + 0..7 of
-// its query row and its bf16 P is the A operand of P.V; base-2 exponents with log2(e) in the scale.
-template <int D>
-__global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32_t* __restrict__ pos0,
-                                                                     const uint16_t* __restrict__ q, int M, int Hq,
-                                                                     int Hkv, const uint16_t* __restrict__ kc,
-                                                                     const uint16_t* __restrict__ vt, int maxlen,
-                                                                     float scale, const int32_t* __restrict__ tree,
-                                                                     float* __restrict__ part_o,
-                                                                     float* __restrict__ part_ml, int nchunk_max) {
-  constexpr int CH = general_chunk(D);
-  constexpr int KS = D / 32;  // 32-dim steps of a score
-  constexpr int KP = D + 8, VP = CH + 8;
-  constexpr int PIECES = CH * D / 8 / (64 * kGWaves);  // 16-byte pieces per thread of K, and of V^T
-  static_assert(PIECES * 8 * 64 * kGWaves == CH * D, "the chunk splits evenly over the threads");
-  __shared__ __attribute__((aligned(16))) uint16_t ks_lds[CH * KP];  // K rows: [key][dim]
-  __shared__ __attribute__((aligned(16))) uint16_t vs_lds[D * VP];   // V^T rows: [dim][key]
-  const int c = blockIdx.x, h = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = wave_id();
-  const int p0 = pos0[0];
-  const int total = p0 + M;
-  const int key0 = c * CH;
-  if (key0 >= total) return;
-  const int G = Hq / Hkv;
-  const int rows = G * M;
-  const bool busy = wave * 16 < rows;
-  const int col = lane & 15, quad = lane >> 4;
-  const int qrow = wave * 16 + col;
-  const bool live = busy && qrow < rows;
-  const int t = live ? qrow / G : 0;
-  // Loads in the order their data is needed: the query row (B operand), the tree words, the chunk.
-  bf16x8_t qf[KS];
-  if (live) {
-    const uint16_t* qr = q + ((size_t)t * Hq + h * G + qrow % G) * D;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8_t*>(qr + ks * 32 + quad * 8);
-  } else {
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = bf16x8_t{};
-  }
-  int tree0 = 0, tree_mask = 0;
-  if (tree) {
-    tree0 = tree[0];
-    tree_mask = tree[1 + t];
-  }
-  const u32x4_t* kh = reinterpret_cast<const u32x4_t*>(kc + ((size_t)h * maxlen + key0) * D);
-  const uint16_t* vh = vt + (size_t)h * D * maxlen + key0;
-  u32x4_t kr[PIECES], vr[PIECES];
-#pragma unroll
-  for (int i = 0; i < PIECES; ++i) {
-    const int e = threadIdx.x + i * 64 * kGWaves;  // K piece e: row e / (D/8); V^T piece e: row e / (CH/8)
-    kr[i] = kh[e];
-    vr[i] = *reinterpret_cast<const u32x4_t*>(vh + (size_t)(e / (CH / 8)) * maxlen + (e % (CH / 8)) * 8);
-  }
-  // Visibility of key kp for this lane's row: with j = kp - tbase, visible iff j < 0, or j < 32
-  // and bit j of tmask. Causal: tbase = p0 + t + 1, tmask = 0; a draft tree: the tree's first slot
-  // and the token's ancestor mask; a padding row sees nothing.
-  int tbase = key0;
-  uint32_t tmask = 0;
-  if (live) {
-    tbase = tree ? p0 - tree0 : p0 + t + 1;
-    tmask = tree ? (uint32_t)tree_mask : 0u;
-  }
-#pragma unroll
-  for (int i = 0; i < PIECES; ++i) {
-    const int e = threadIdx.x + i * 64 * kGWaves;
-    *reinterpret_cast<u32x4_t*>(&ks_lds[(e / (D / 8)) * KP + (e % (D / 8)) * 8]) = kr[i];
-    *reinterpret_cast<u32x4_t*>(&vs_lds[(e / (CH / 8)) * VP + (e % (CH / 8)) * 8]) = vr[i];
-  }
-  __syncthreads();
-  if (!busy) return;
-
-  const size_t base = ((size_t)h * nchunk_max + c) * kGRowsMax + wave * 16;
-  general_rows<D>(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, rows - wave * 16, part_o + base * D, part_ml + base * 2);
 }
 
 // (3) One workgroup per (query head, token), max(1, D / 128) waves, lane l of wave w holding dims
@@ -617,9 +638,11 @@ int launch_general(const int32_t* pos0, const uint16_t* qkv, const HeadLayout& h
                      kn, eps, R, rope, tree, M, q, kc, vt, maxlen);
   if (int rc = skinny_check_launch("attention_general q/k")) return rc;
   if ((Hq / Hkv) * M <= kGFewRows && maxlen <= kGFewMaxlen) {
-    const int per = nch * Hkv <= 512 ? 1 : nch * Hkv <= 1024 ? 2 : kGWaves;
-    hipLaunchKernelGGL(general_few_kernel<D>, dim3((nch + per - 1) / per, Hkv), dim3(64 * per), 0, stream, pos0, q, M, Hq,
-                       Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nch, per);
+    const int per = nch * Hkv <= 512 ? 1 : nch * Hkv <= 1024 ? 2 : kGWaves, n = (nch + per - 1) / per;
+    const bool stage = nch * Hkv >= 2 * kGFewStaged;
+    hipLaunchKernelGGL((stage ? general_few_kernel<D, true> : general_few_kernel<D, false>), dim3(n, Hkv),
+                       dim3(stage ? 64 * kGWaves : 64 * per), 0, stream, pos0, q, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o,
+                       part_ml, nch, n);
   } else {
     hipLaunchKernelGGL(general_chunk_kernel<D>, dim3(nch, Hkv), dim3(64 * kGWaves), 0, stream, pos0, q, M, Hq, Hkv, kc,
                        vt, maxlen, scale, tree, part_o, part_ml, nch);

@@ -11,8 +11,10 @@ from skinny_mlx.tree import DraftTree
 
 pytestmark = pytest.mark.gpu
 
-# (kv heads, cache slots, cached tokens): the dense layout staged; chunks x heads <= 512, <= 1024, past it
-CASES = [(2, 1024, 100), (2, 2048, 0), (2, 2048, 100), (2, 2048, 250), (8, 8192, 5000), (8, 12288, 12200), (8, 33024, 32765)]
+# (kv heads, cache slots, cached tokens): the dense layout staged; chunks x heads <= 512, <= 1024, past it; long caches
+# filled so far that a workgroup takes one chunk (general layouts: staged up to 256 chunks in all), two and four
+CASES = [(2, 1024, 100), (2, 2048, 0), (2, 2048, 100), (2, 2048, 250), (8, 8192, 5000), (8, 12288, 12200), (8, 33024, 32765),
+         (8, 33024, 60), (8, 33024, 2040), (8, 33024, 4090), (8, 33024, 8250), (8, 33024, 16700), (2, 33024, 8180)]
 
 
 def _call(layout, rnd, dev, hkv, maxlen):
