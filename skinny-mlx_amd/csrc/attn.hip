@@ -88,7 +88,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_chunk_kernel(const int32_t* 
 // this way: workgroups 0 and 1 of a head run attn_chunk_body over the chunks that hold the new slots, the n
 // others the chunks below them, 1, 2 or 4 each. The grid is sized for a full cache; how many of its waves a
 // workgroup uses goes by the context, so that a short context's chunks in a long cache are on CUs of their own
-// (4 in every workgroup: 4000 keys in a cache of 32896 slots 14.7 us a layer, spread 12.9; 13.6 staged). What bounds
+// (4 in every workgroup: 4000 keys in a cache of 32896 slots 14.7 us a layer, spread 12.4; 13.6 staged). What bounds
 // it at a long context is the read of K and V^T; at a short one the chain position, chunk, partial, merge.
 // Measured on MI355X, one token, chunk stage and merge of a layer, staged against this: 32768 keys 41.2 / 36.7 us
 // (3.66 TB/s of KV; with it, partials of the live rows only and eight merge waves); 8000 keys of 8192 slots 14.0 /
@@ -221,8 +221,12 @@ __device__ __forceinline__ bool combine_row(const float* __restrict__ part_o, co
   const int first = v * kCombineBlock;                                // this wave's first block
   // The first block's partials are loaded before the chunk count is known (it needs *pos0):
   // every chunk the workspace holds up to kCombineBlock, the ones past the context discarded below
-  // by selection (their stale values never enter an arithmetic operation).
-  const int pre = kPrompt ? 0 : max(0, min(kCombineBlock, nchunk_max - first));
+  // by selection (their stale values never enter an arithmetic operation). Waves past the fourth (of a long cache,
+  // which the context seldom fills) take the count first: 16 tokens over 60 / 4000 keys in 32896 slots 20.3 / 25.4 us a
+  // layer when all eight load ahead, 14.5 / 21.2 so, 14.0 / 20.9 with four waves in all; 32768 keys the same.
+  int pre = kPrompt ? 0 : max(0, min(kCombineBlock, nchunk_max - first));
+  if constexpr (!kPrompt && W > kCombineWaves)
+    if (v >= kCombineWaves) pre = max(0, min(pre, (pos0[0] + tokens + kChunk - 1) / kChunk - first));
   float mc_pre = -INFINITY, lc_pre = 0.f;
   float o0[kCombineBlock], o1[kCombineBlock];
   if (lane < pre) {
