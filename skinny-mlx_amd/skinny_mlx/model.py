@@ -208,16 +208,21 @@ class Attention(nn.Module):
         # rows, counting on the GPU to themselves: not for a model run beside other streams' work.
         self.fuse_qkv = False
 
-    def forward(self, x, cache: KVCache, tree=None):
-        a = self.a
-        sh = cache.shared
-        desc = None if tree is None else tree.desc
+    def _shared(self, cache: KVCache):
+        """The cache's shared state, its RoPE table being this layer's."""
+        a, sh = self.a, cache.shared
         if sh.rope_theta != a.rope_theta:
             raise ValueError(f"cache RoPE table for theta={sh.rope_theta}, layer uses {a.rope_theta}")
+        if a.general_attention and sh.rope_dim != a.rotary_dim:
+            raise ValueError(f"cache RoPE table over {sh.rope_dim} dims, layer rotates {a.rotary_dim}")
+        return sh
+
+    def forward(self, x, cache: KVCache, tree=None):
+        a = self.a
+        sh = self._shared(cache)
+        desc = None if tree is None else tree.desc
         if a.general_attention:
             # Qwen3.5 layouts (another head size, a partial RoPE, the output gate): the general kernels
-            if sh.rope_dim != a.rotary_dim:
-                raise ValueError(f"cache RoPE table over {sh.rope_dim} dims, layer rotates {a.rotary_dim}")
             Hq, Hkv, D = a.num_attention_heads, a.num_key_value_heads, a.head_dim
             qs = 2 * D if a.attn_output_gate else D
             qkv = joined([self.q_proj(x), self.k_proj(x), self.v_proj(x)])
@@ -250,7 +255,7 @@ class Attention(nn.Module):
     def prompt(self, x: torch.Tensor, cache: KVCache, keys: int) -> torch.Tensor:
         """forward over a prompt's rows (more than MAX_STEP tokens), bitwise 16-token steps of it; the
         residual comes summed. `keys` = cached tokens after the call."""
-        a, sh = self.a, cache.shared
+        a, sh = self.a, self._shared(cache)
         Hq, Hkv, D = a.num_attention_heads, a.num_key_value_heads, a.head_dim
         qkv = joined([self.q_proj(x), self.k_proj(x), self.v_proj(x)])
         if a.general_attention:

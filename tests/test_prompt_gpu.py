@@ -79,6 +79,18 @@ def test_unpatched_and_captured_inputs_keep_the_pieces():
     assert not hybrid._prompt_ok(ids)
 
 
+@pytest.mark.parametrize("preset,field,value", [("tiny-dense", "rope_theta", 5e5), ("tiny-qwen35", "rope_theta", 5e5),
+                                                ("tiny-qwen35", "rope_dim", 32)])
+def test_a_cache_of_another_rope_is_refused(preset, field, value):
+    """A long input is refused as its 16-token steps are."""
+    model = _model(preset)
+    for t in (16, 100):
+        cache = make_prompt_cache(model)
+        setattr(cache.shared, field, value)
+        with pytest.raises(ValueError, match="cache RoPE table"):
+            forward(model, list(range(t)), cache)
+
+
 @pytest.mark.parametrize("maxlen,past", [(1024, 0), (1024, 250), (8192, 4300), (17408, 16500)])  # one-, four- and eight-wave merges
 @pytest.mark.parametrize("layout", ["dense", "general"])
 def test_prompt_attention_equals_steps(dev, layout, maxlen, past):
