@@ -559,6 +559,11 @@ class Model(nn.Module):
         outs = []
         if full:
             piece = getattr(cache, "_piece_step", None)
+            first = 0
+            if piece is None and any(isinstance(m, QuantizedLinear) for m in self.layers.modules()):
+                # an unpatched linear's GEMM sets its library up on its first call, which no capture permits
+                outs.append(self.hidden(ids[:MAX_STEP], cache))
+                first = 1
             if piece is None:
                 import weakref
 
@@ -571,7 +576,7 @@ class Model(nn.Module):
                 piece = cache._piece_step = (buf, CapturedStep(lambda: self.hidden(buf, wc()), cache, MAX_STEP,
                                                                weak_cache=True))
             buf, step = piece
-            for i in range(full):
+            for i in range(first, full):
                 buf.copy_(ids[i * MAX_STEP:(i + 1) * MAX_STEP])
                 outs.append(step().clone())
         for i in range(full * MAX_STEP, T, MAX_STEP):

@@ -68,6 +68,19 @@ def test_prompt_blocks_and_short_tail(monkeypatch):
         assert torch.equal(a, b)
 
 
+def test_unpatched_linears_run_once_before_the_pieces_are_captured(monkeypatch):
+    import skinny_mlx.graphs as G
+
+    cached = []
+    step = G.CapturedStep
+    monkeypatch.setattr(G, "CapturedStep", lambda fn, cache, *a, **k: cached.append(cache.attention_offset()) or step(fn, cache, *a, **k))
+    model = build_model("tiny-dense")
+    ids = list(range(70))
+    c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
+    h = model.hidden(ids, c1)
+    assert cached == [16] and torch.equal(h, torch.cat([model.hidden(ids[i:i + 16], c2) for i in range(0, 70, 16)]))
+
+
 def test_unpatched_and_captured_inputs_keep_the_pieces():
     model = build_model("tiny-dense")
     ids = model._ids(list(range(100)))
