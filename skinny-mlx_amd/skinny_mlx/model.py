@@ -156,6 +156,13 @@ def residual_out(proj, x: torch.Tensor):
     return partial(x) if partial is not None else proj(x)
 
 
+def prompt_residual(proj, x: torch.Tensor) -> torch.Tensor:
+    """residual_out for a prompt's rows (more than MAX_STEP tokens): the slices of a patched projection come
+    summed (bitwise what the norm makes of them)."""
+    summed = getattr(proj, "prompt_residual", None)
+    return summed(x) if summed is not None else proj(x)
+
+
 def norm_input(h: torch.Tensor, residual, weight: torch.Tensor, eps: float, spare: torch.Tensor):
     """The input rmsnorm(h + residual) * weight of the next projections, and the tensor that holds
     the residual stream h + residual once they have run. A split-K residual (kernels.PartialSum)
@@ -266,7 +273,7 @@ class Attention(nn.Module):
         else:
             o = K.attention_prompt(qkv, Hq, Hkv, D, self.q_norm, self.k_norm, a.rms_norm_eps, sh.rope, sh.pos, keys,
                                    cache.k, cache.vt, D ** -0.5)
-        return self.o_proj.prompt_residual(o)
+        return prompt_residual(self.o_proj, o)
 
 
 class GatedDeltaNet(nn.Module):
@@ -362,7 +369,7 @@ class GatedDeltaNet(nn.Module):
         xc = K.gdn_conv_silu(qkv, cache.conv_state, self.conv1d_weight, None)
         r = K.gdn_recurrence(xc, b, ag, self.A_log, self.dt_bias, cache.state, None, a.linear_num_heads,
                              a.linear_key_head_dim, a.linear_value_head_dim, None, None, a.gdn_key_heads)
-        return self.out_proj.prompt_residual(K.gated_rmsnorm(r, z, self.norm_weight, a.rms_norm_eps))
+        return prompt_residual(self.out_proj, K.gated_rmsnorm(r, z, self.norm_weight, a.rms_norm_eps))
 
 
 def swiglu(gate: nn.Module, up: nn.Module, x: torch.Tensor) -> torch.Tensor:
@@ -399,7 +406,7 @@ class MLP(nn.Module):
 
     def prompt(self, x: torch.Tensor) -> torch.Tensor:
         """forward over a prompt's rows (more than MAX_STEP tokens), the residual summed."""
-        return self.down_proj.prompt_residual(swiglu(self.gate_proj, self.up_proj, x))
+        return prompt_residual(self.down_proj, swiglu(self.gate_proj, self.up_proj, x))
 
 
 class DecoderLayer(nn.Module):
@@ -418,6 +425,11 @@ class DecoderLayer(nn.Module):
         if self.is_linear:
             return self.linear_attn(x, cache, tree)
         return self.self_attn(x, cache, tree)
+
+
+# The modules that Model._prompt knows how to run in blocks (skinny_mlx.patch adds its linears). A model with any
+# other in its layers (an unpatched linear, a replaced one, a subclass) takes its long inputs in steps.
+PROMPT_MODULES = {nn.ModuleList, DecoderLayer, Attention, GatedDeltaNet, MLP}
 
 
 @dataclass
@@ -511,12 +523,22 @@ class Model(nn.Module):
 
     def _prompt_ok(self, ids: torch.Tensor) -> bool:
         """Whether long inputs take the many-row kernels: on the GPU, outside a capture (the attention's grid
-        follows the host's cache length), every linear of the layers patched, at most 4 query heads per
+        follows the host's cache length), nothing but PROMPT_MODULES in the layers, at most 4 query heads per
         kv head (16 tokens x 4 heads fill a chunk's 64 query rows)."""
         a = self.args
         return (ids.is_cuda and a.num_attention_heads <= 4 * a.num_key_value_heads
-                and not torch.cuda.is_current_stream_capturing()
-                and not any(isinstance(m, QuantizedLinear) for m in self.layers.modules()))
+                and not torch.cuda.is_current_stream_capturing() and self._prompt_modules())
+
+    def _prompt_modules(self) -> bool:
+        """Whether every module of the layers is one of PROMPT_MODULES (asked anew for each input: modules may be
+        replaced at any time)."""
+        left = [self.layers]
+        while left:
+            m = left.pop()
+            if type(m) not in PROMPT_MODULES:
+                return False
+            left.extend(m._modules.values())
+        return True
 
     def _prompt(self, ids: torch.Tensor, cache: PromptCache) -> torch.Tensor:
         """A long input in blocks of up to PROMPT_BLOCK tokens, each weight read once per block of rows:
@@ -560,8 +582,8 @@ class Model(nn.Module):
         if full:
             piece = getattr(cache, "_piece_step", None)
             first = 0
-            if piece is None and any(isinstance(m, QuantizedLinear) for m in self.layers.modules()):
-                # an unpatched linear's GEMM sets its library up on its first call, which no capture permits
+            if piece is None and not self._prompt_modules():
+                # an unpatched or replaced linear's GEMM sets its library up on its first call, which no capture permits
                 outs.append(self.hidden(ids[:MAX_STEP], cache))
                 first = 1
             if piece is None:

@@ -33,7 +33,7 @@ import torch
 from torch import nn
 
 from . import kernels as K
-from .model import QuantizedLinear
+from .model import PROMPT_MODULES, QuantizedLinear
 from .qmm import (GROUP, MAX_M, NORMIN_CONV, NORMIN_PLAIN, NORMIN_SWIGLU, gated_partial_supported, mlp_fused_buffers,
                   mlp_fused_supported, normin_supported, packed_k, repack_for_skinny, repack_gate_up, skinny_glu,
                   skinny_glu_normin, skinny_mlp_fused_partial, skinny_qmm, skinny_qmm_conv, skinny_qmm_conv_normin,
@@ -235,6 +235,9 @@ class FusedSliceLinear(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.projection.output(x)[..., self.columns]
+
+
+PROMPT_MODULES.update((SkinnyQuantizedLinear, FusedSliceLinear))
 
 
 def patch_model(model: nn.Module, fuse: bool = True) -> dict:

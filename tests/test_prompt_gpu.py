@@ -92,6 +92,48 @@ def test_unpatched_and_captured_inputs_keep_the_pieces():
     assert not hybrid._prompt_ok(ids)
 
 
+class _Wrapped(torch.nn.Module):
+    """Any other module in the place of one of the model's: here it only hands through."""
+
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, *args):
+        return self.inner(*args)
+
+
+def _replace(model, where):
+    layer = model.layers[-1]
+    parent = {"o_proj": "self_attn", "q_proj": "self_attn", "down_proj": "mlp", "gate_proj": "mlp"}.get(where)
+    owner = getattr(layer, parent) if parent else layer
+    setattr(owner, where, _Wrapped(getattr(owner, where)))
+
+
+@pytest.mark.parametrize("t", [20, 90])
+@pytest.mark.parametrize("where", ["o_proj", "q_proj", "down_proj", "gate_proj", "mlp", "self_attn"])
+def test_a_replaced_module_keeps_the_pieces(where, t):
+    model = _model("tiny-dense")
+    _replace(model, where)
+    ids = torch.randint(0, model.args.vocab_size, (t,), generator=torch.Generator().manual_seed(t)).tolist()
+    c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
+    assert not model._prompt_ok(model._ids(ids))
+    h, _ = forward(model, ids, c1)
+    assert torch.equal(h, torch.cat([model.hidden(ids[i:i + 16], c2) for i in range(0, t, 16)]))
+
+
+@pytest.mark.parametrize("t", [20, 90])
+def test_a_replaced_linear_of_another_library(t):
+    model = _model("tiny-dense")
+    down = torch.nn.Linear(512, 256, bias=False, device=model.device, dtype=torch.bfloat16)
+    model.layers[0].mlp.down_proj = down
+    ids = list(range(t))
+    c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
+    with torch.no_grad():
+        h = model.hidden(ids, c1)
+        assert torch.equal(h, torch.cat([model.hidden(ids[i:i + 16], c2) for i in range(0, t, 16)]))
+
+
 @pytest.mark.parametrize("preset,field,value", [("tiny-dense", "rope_theta", 5e5), ("tiny-qwen35", "rope_theta", 5e5),
                                                 ("tiny-qwen35", "rope_dim", 32)])
 def test_a_cache_of_another_rope_is_refused(preset, field, value):
