@@ -427,9 +427,13 @@ class DecoderLayer(nn.Module):
         return self.self_attn(x, cache, tree)
 
 
-# The modules that Model._prompt knows how to run in blocks (skinny_mlx.patch adds its linears). A model with any
-# other in its layers (an unpatched linear, a replaced one, a subclass) takes its long inputs in steps.
-PROMPT_MODULES = {nn.ModuleList, DecoderLayer, Attention, GatedDeltaNet, MLP}
+# The modules that Model._prompt knows how to run in blocks (skinny_mlx.patch adds its linears), each with the method
+# through which a step runs it and which a block passes by. A model with any other module in its layers (an unpatched
+# linear, a replaced one, a subclass), with another method in that one's place or with forward hooks takes its long
+# inputs in steps.
+PROMPT_MODULES = {nn.ModuleList: ("forward", nn.ModuleList.forward), DecoderLayer: ("mixer", DecoderLayer.mixer),
+                  **{m: ("forward", m.forward) for m in (Attention, GatedDeltaNet, MLP)}}
+_ANY_HOOKS = [getattr(nn.modules.module, f"_global_forward_{kind}hooks") for kind in ("", "pre_")]  # of every module
 
 
 @dataclass
@@ -530,12 +534,17 @@ class Model(nn.Module):
                 and not torch.cuda.is_current_stream_capturing() and self._prompt_modules())
 
     def _prompt_modules(self) -> bool:
-        """Whether every module of the layers is one of PROMPT_MODULES (asked anew for each input: modules may be
-        replaced at any time)."""
+        """Whether every module of the layers is one of PROMPT_MODULES, run as a step expects and without forward
+        hooks (asked anew for each input: all of that may change at any time)."""
+        if any(_ANY_HOOKS):
+            return False
         left = [self.layers]
         while left:
             m = left.pop()
-            if type(m) not in PROMPT_MODULES:
+            cls = type(m)
+            name, method = PROMPT_MODULES.get(cls, (None, None))
+            if (name is None or getattr(cls, name) is not method or name in m.__dict__ or m._forward_hooks
+                    or m._forward_pre_hooks):
                 return False
             left.extend(m._modules.values())
         return True

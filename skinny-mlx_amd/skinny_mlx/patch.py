@@ -237,7 +237,7 @@ class FusedSliceLinear(nn.Module):
         return self.projection.output(x)[..., self.columns]
 
 
-PROMPT_MODULES.update((SkinnyQuantizedLinear, FusedSliceLinear))
+PROMPT_MODULES.update({m: ("forward", m.forward) for m in (SkinnyQuantizedLinear, FusedSliceLinear)})
 
 
 def patch_model(model: nn.Module, fuse: bool = True) -> dict:

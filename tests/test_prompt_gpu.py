@@ -134,6 +134,38 @@ def test_a_replaced_linear_of_another_library(t):
         assert torch.equal(h, torch.cat([model.hidden(ids[i:i + 16], c2) for i in range(0, t, 16)]))
 
 
+@pytest.mark.parametrize("how", ["hook", "pre-hook", "any module's hook", "forward", "class forward", "mixer"])
+def test_hooks_and_replaced_methods_see_every_step(how, monkeypatch):
+    """33 tokens: three passes, each through the hook or method of a layer's MLP (the mixer's for "mixer")."""
+    from skinny_mlx.model import MLP
+
+    model = _model("tiny-dense")
+    layer, seen = model.layers[0], []
+    mlp, handle = layer.mlp, None
+    note = lambda *a: seen.append(1) if a[0] is mlp else None
+    if how == "hook":
+        mlp.register_forward_hook(note)
+    elif how == "pre-hook":
+        mlp.register_forward_pre_hook(note)
+    elif how == "any module's hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(note)
+    elif how == "forward":
+        old = mlp.forward
+        mlp.forward = lambda x: (seen.append(1), old(x))[1]
+    elif how == "class forward":
+        plain = MLP.forward
+        monkeypatch.setattr(MLP, "forward", lambda self, x: (note(self), plain(self, x))[1])
+    else:
+        old = layer.mixer
+        layer.mixer = lambda *a: (seen.append(1), old(*a))[1]
+    try:
+        model.hidden(list(range(33)), make_prompt_cache(model))
+    finally:
+        if handle is not None:
+            handle.remove()
+    assert len(seen) == 3
+
+
 @pytest.mark.parametrize("preset,field,value", [("tiny-dense", "rope_theta", 5e5), ("tiny-qwen35", "rope_theta", 5e5),
                                                 ("tiny-qwen35", "rope_dim", 32)])
 def test_a_cache_of_another_rope_is_refused(preset, field, value):
