@@ -527,10 +527,15 @@ class Model(nn.Module):
 
     def _prompt_ok(self, ids: torch.Tensor) -> bool:
         """Whether long inputs take the many-row kernels: on the GPU, outside a capture (the attention's grid
-        follows the host's cache length), nothing but PROMPT_MODULES in the layers, at most 4 query heads per
-        kv head (16 tokens x 4 heads fill a chunk's 64 query rows)."""
+        follows the host's cache length), every piece in the skinny range (patch.SKINNY_RANGE), nothing but
+        PROMPT_MODULES in the layers, at most 4 query heads per kv head (16 tokens x 4 heads fill a chunk's 64
+        query rows)."""
+        from .patch import _skinny_ok
+
         a = self.args
+        T = ids.shape[0]
         return (ids.is_cuda and a.num_attention_heads <= 4 * a.num_key_value_heads
+                and _skinny_ok(MAX_STEP) and _skinny_ok(T % MAX_STEP or MAX_STEP)
                 and not torch.cuda.is_current_stream_capturing() and self._prompt_modules())
 
     def _prompt_modules(self) -> bool:
@@ -583,6 +588,8 @@ class Model(nn.Module):
         GPU, the full pieces replay one captured pass (graphs.CapturedStep, kept on the cache for
         its later prompts): issued kernel by kernel from Python, a pass costs about twice its GPU
         time, and a capture about two passes. The remainder runs eagerly."""
+        from .patch import _skinny_ok
+
         T = ids.shape[0]
         full = T // MAX_STEP if ids.is_cuda and not torch.cuda.is_current_stream_capturing() else 0
         if T < PIECES_MIN:
@@ -591,8 +598,9 @@ class Model(nn.Module):
         if full:
             piece = getattr(cache, "_piece_step", None)
             first = 0
-            if piece is None and not self._prompt_modules():
-                # an unpatched or replaced linear's GEMM sets its library up on its first call, which no capture permits
+            if piece is None and not (_skinny_ok(MAX_STEP) and self._prompt_modules()):
+                # another library's GEMM (an unpatched or replaced linear, a piece outside the skinny range) sets
+                # itself up on its first call, which no capture permits
                 outs.append(self.hidden(ids[:MAX_STEP], cache))
                 first = 1
             if piece is None:

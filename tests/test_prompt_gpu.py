@@ -68,13 +68,17 @@ def test_prompt_blocks_and_short_tail(monkeypatch):
         assert torch.equal(a, b)
 
 
-def test_unpatched_linears_run_once_before_the_pieces_are_captured(monkeypatch):
+@pytest.mark.parametrize("skinny_range", [None, (99, 99)])  # unpatched; patched with the kernels switched off
+def test_unpatched_linears_run_once_before_the_pieces_are_captured(skinny_range, monkeypatch):
     import skinny_mlx.graphs as G
 
     cached = []
     step = G.CapturedStep
     monkeypatch.setattr(G, "CapturedStep", lambda fn, cache, *a, **k: cached.append(cache.attention_offset()) or step(fn, cache, *a, **k))
     model = build_model("tiny-dense")
+    if skinny_range:
+        P.patch_model(model)
+        monkeypatch.setattr(P, "SKINNY_RANGE", skinny_range)
     ids = list(range(70))
     c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
     h = model.hidden(ids, c1)
@@ -164,6 +168,19 @@ def test_hooks_and_replaced_methods_see_every_step(how, monkeypatch):
         if handle is not None:
             handle.remove()
     assert len(seen) == 3
+
+
+@pytest.mark.parametrize("t,block", [(18, False), (22, True), (32, True)])
+def test_pieces_outside_the_skinny_range_keep_their_route(t, block, monkeypatch):
+    """With the reference's range of 6 to 16 rows (its patch.py:22) a last piece of two tokens is multiplied
+    unpatched, as a step of two is; whole pieces go through the kernels either way."""
+    monkeypatch.setattr(P, "SKINNY_RANGE", (6, 16))
+    model = _model("tiny-dense")
+    ids = torch.randint(0, model.args.vocab_size, (t,), generator=torch.Generator().manual_seed(t)).tolist()
+    assert model._prompt_ok(model._ids(ids)) == block
+    c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
+    h = model.hidden(ids, c1)
+    assert torch.equal(h, torch.cat([model.hidden(ids[i:i + 16], c2) for i in range(0, t, 16)]))
 
 
 @pytest.mark.parametrize("preset,field,value", [("tiny-dense", "rope_theta", 5e5), ("tiny-qwen35", "rope_theta", 5e5),
