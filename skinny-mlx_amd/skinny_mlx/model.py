@@ -265,6 +265,9 @@ class Attention(nn.Module):
         a, sh = self.a, self._shared(cache)
         Hq, Hkv, D = a.num_attention_heads, a.num_key_value_heads, a.head_dim
         qkv = joined([self.q_proj(x), self.k_proj(x), self.v_proj(x)])
+        proj = getattr(self.q_proj, "projection", None)
+        if proj is not None:
+            proj.forget()  # a fused projection keeps its last rows and result: 17 MB a layer of 1024 tokens
         if a.general_attention:
             qs = 2 * D if a.attn_output_gate else D
             o = K.attention_general_prompt(qkv, Hq, Hkv, D, qs, Hq * qs, Hq * qs + Hkv * D,

@@ -174,6 +174,10 @@ class _Projection:
             self._key, self._out = (x, version), self._compute(x)
         return self._out
 
+    def forget(self) -> None:
+        """Drop the cached result (Attention.prompt: rows by the hundred, which no other member asks for again)."""
+        self._key = self._out = None
+
     def conv_output(self, x, c: int, conv_state: torch.Tensor, conv_w: torch.Tensor, window=None, parent=None):
         """The output with a Gated-DeltaNet mixer's conv + SiLU applied to its first `c` columns in
         the same launch (qmm.skinny_qmm_conv), or None where that form does not apply (a token count

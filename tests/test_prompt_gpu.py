@@ -3,6 +3,8 @@ hidden states, logits, keys, values and Gated-DeltaNet states, at lengths that e
 64-token group and a 128-key chunk, from an empty cache and after cached tokens; and the prompt kernels
 alone, with workspaces that take several launches."""
 
+import gc
+
 import pytest
 import torch
 
@@ -181,6 +183,19 @@ def test_pieces_outside_the_skinny_range_keep_their_route(t, block, monkeypatch)
     c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
     h = model.hidden(ids, c1)
     assert torch.equal(h, torch.cat([model.hidden(ids[i:i + 16], c2) for i in range(0, t, 16)]))
+
+
+@pytest.mark.parametrize("preset", list(SMALL))
+def test_a_prompt_leaves_nothing_behind(preset):
+    """What is allocated after a prompt is what was before it (a fused projection's cached result would be 500 rows
+    of q, k and v a layer)."""
+    model = _model(preset)
+    cache = make_prompt_cache(model)
+    model.hidden(list(range(20)), cache)
+    gc.collect()
+    before = torch.cuda.memory_allocated()
+    model.hidden([i % 999 for i in range(480)], cache)
+    assert torch.cuda.memory_allocated() <= before
 
 
 @pytest.mark.parametrize("preset,field,value", [("tiny-dense", "rope_theta", 5e5), ("tiny-qwen35", "rope_theta", 5e5),
