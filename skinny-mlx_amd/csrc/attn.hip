@@ -173,7 +173,7 @@ __device__ __forceinline__ void attn_direct_chunk(int c, int h, int p0, const ui
     for (int ks = 0; ks < 4; ++ks) o[dt] = mfma16x16x32(__builtin_bit_cast(bf16x8_t, pa[ks]), vf[dt][ks], o[dt]);
   }
   const size_t base = ((size_t)h * nchunk_max + c) * kRowsMax;
-  attn_store_rows(o, mx, sum, rows, part_o + base * kD, part_ml + base * 2);
+  attn_store_rows<true>(o, mx, sum, rows, part_o + base * kD, part_ml + base * 2);
 }
 
 __global__ __launch_bounds__(64 * kWaves) void attn_few_kernel(const int32_t* __restrict__ pos0,
@@ -480,7 +480,7 @@ __global__ __launch_bounds__(64 * kWaves) void prompt_chunk_kernel(const int32_t
     if (key0 >= p0 + t0 + mb || wave * 16 >= G * mb) continue;
     const int tbase = qrow < G * mb ? p0 + t0 + qrow / G + 1 : key0;
     const size_t base = (((size_t)(z - z0) * Hkv + h) * nch + c) * kRowsMax + wave * 16;
-    attn_rows(ks_lds, vs_lds, qf[i], key0, tbase, 0u, scale, G * mb - wave * 16, part_o + base * kD, part_ml + base * 2);
+    attn_rows(ks_lds, vs_lds, qf[i], key0, tbase, 0u, scale, part_o + base * kD, part_ml + base * 2);
   }
 }
 
