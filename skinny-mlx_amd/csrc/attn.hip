@@ -85,16 +85,17 @@ __global__ __launch_bounds__(64 * kWaves) void attn_chunk_kernel(const int32_t* 
 // each wave takes a chunk of its own, its K and V^T fragments straight from memory into registers (the
 // same fragments, MFMAs and softmax, so the partials are bitwise attn_chunk_body's). Nothing waits at a
 // barrier, and a CU holds 8 chunks' loads in flight instead of 2. Only chunks without new tokens are taken
-// this way: workgroups 0 and 1 of a head run attn_chunk_body over the chunks that hold the new slots, the n
-// others the chunks below them, 1, 2 or 4 each. The grid is sized for a full cache; how many of its waves a
-// workgroup uses goes by the context, so that a short context's chunks in a long cache are on CUs of their own
-// (4 in every workgroup: 4000 keys in a cache of 32896 slots 14.7 us a layer, spread 12.4; 13.6 staged). What bounds
-// it at a long context is the read of K and V^T; at a short one the chain position, chunk, partial, merge.
-// Measured on MI355X, one token, chunk stage and merge of a layer, staged against this: 32768 keys 41.2 / 36.7 us
-// (3.66 TB/s of KV; with it, partials of the live rows only and eight merge waves); 8000 keys of 8192 slots 14.0 /
-// 13.3; 2000 of 4096 9.6 / 9.4; but 4000 of 4096 10.9 / 11.3, 60 in 2048 or 4224 slots 8.8 / 8.9 and 9.1 / 9.2, and
-// caches of 256 / 512 / 1280 slots 9.58 / 9.75 / 9.95 against 9.73 / 9.93 / 10.05: up to kFewChunks chunks stay
-// staged. With more rows per kv head several waves of a staged chunk have work, and staging serves them all.
+// this way: the first workgroups of a head run attn_chunk_body over the one or two chunks that hold the new slots, the
+// others the chunks below them, 1, 2 or 4 each. The grid is sized for a full cache; how many of its waves a workgroup
+// uses goes by the context, so that a short context's chunks in a long cache are on CUs of their own, and the grid's
+// workgroups are dealt to the heads anew, the idle ones last: workgroups that end at once between the busy ones left some
+// CUs two chunks and others none (4000 keys of 4096 slots, 256 busy of 272: 11.5 us a layer, dealt 10.1). What bounds it at
+// a long context is the read of K and V^T; at a short one the chain position, chunk, partial, merge.
+// Measured on MI355X, one token, chunk stage and merge of a layer, staged against this: 32768 keys 41.5 / 36.4 us
+// (3.69 TB/s of KV; with it, partials of the live rows only and eight merge waves); 8000 keys of 8192 slots 14.0 / 13.1; 1000
+// of 8192 10.7 / 9.2; 4000 of 32896 13.6 / 10.4; 4000 of 4096 10.9 / 10.1; 2000 of 2048 9.3 / 9.2; 60 in 2048 or 4096 8.9 / 8.9
+// and 9.2 / 9.0. Caches of 256 / 512 / 1280 slots were 1% slower so: up to kFewChunks chunks stay staged. With more rows per
+// kv head several waves of a staged chunk have work, and staging serves them all.
 constexpr int kFewRows = 16;
 constexpr int kFewChunks = 12;        // caches of up to this many chunks stay staged
 constexpr int kFewMaxlen = 1 << 22;  // V^T of a head within a buffer descriptor
@@ -182,17 +183,27 @@ __global__ __launch_bounds__(64 * kWaves) void attn_few_kernel(const int32_t* __
                                                                int maxlen, float scale, const int32_t* __restrict__ tree,
                                                                float* __restrict__ part_o, float* __restrict__ part_ml,
                                                                int nchunk_max, int n) {
-  const int b = blockIdx.x, h = blockIdx.y, wave = wave_id();
-  const int p0 = pos0[0];
-  const int fresh = p0 / kChunk;  // the first chunk with new slots
-  const int sh = fresh > 2 * n ? 2 : fresh > n ? 1 : 0;
-  const int c = ((b - 2) << sh) + wave;
-  if (b >= 2 && ((wave >> sh) || c >= min(fresh, nchunk_max))) return;
-  if (b < 2) {
-    if ((unsigned)(fresh + b) >= (unsigned)nchunk_max) return;  // slots past the cache are dropped, as the staged grid has none
-    attn_chunk_body<true>(fresh + b, h, pos0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
+  const int wave = wave_id(), p0 = pos0[0];
+  const int fresh = max(p0, 0) / kChunk;  // the first chunk with new slots
+  const int last = min((p0 + M - 1) / kChunk, nchunk_max - 1);  // and the last (slots past the cache are dropped)
+  const int old = min(fresh, nchunk_max);
+  const int sh = old > 2 * n ? 2 : old > n ? 1 : 0;
+  const int staged = max(0, last - fresh + 1), used = max(1, staged + ((old + (1 << sh) - 1) >> sh));  // of each head
+  int h = blockIdx.y, b = blockIdx.x, first = 2;  // workgroup of the head, and the first with a chunk per wave
+  if (sh < 2) {  // (with four chunks each the grid is at least half used, and as it stands no slower)
+    const auto [quot, rem] = work_index(h * (2 + n) + b, used);
+    if (quot >= Hkv) return;
+    h = quot;
+    b = rem;
+    first = staged;
+  }
+  if (b < first) {
+    if (b < staged)
+      attn_chunk_body<true>(fresh + b, h, pos0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
     return;
   }
+  const int c = ((b - first) << sh) + wave;
+  if ((wave >> sh) || c >= old) return;
   attn_direct_chunk(c, h, p0, q, fa, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
 }
 

@@ -313,10 +313,12 @@ __global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32
 // a chunk of its own with its K and V^T fragments straight from memory (the new rows are in the caches
 // already), 1, 2 or 4 chunks in each of n workgroups by the context; partials bitwise general_chunk_kernel's. In a
 // long cache (kStage) up to kGFewStaged chunks in all, one per CU, are staged by all waves of a workgroup instead:
-// rows of V^T many KB apart come slowly to one wave. 256-dim heads, one token, us a layer, every chunk staged / a chunk per
-// wave / as here: 1000 keys in 8192 slots 11.3 / 12.3 / 11.6, in 32896 10.7 / 11.9 / 11.1, 4000 in 32896 14.7 / 14.2 /
-// 14.2; 8000 in 8192 19.5 / 16.5 / 16.6; 32768 in 33024 62 / 48.6 / 48.7. Smaller caches take a chunk per wave
-// throughout: 1000 / 2000 / 4000 keys in 4096 slots 10.5 / 11.5 / 13.8 staged, 10.4 / 11.1 / 12.7.
+// rows of V^T many KB apart come slowly to one wave. The staged chunks are dealt to the grid's first workgroups, the idle
+// ones last (see attn_few_kernel); a chunk per wave keeps its place, where dealing took 1% more. 256-dim heads, one token, us
+// a layer, every chunk staged / a chunk per wave / as here: 1000 keys in 8192 slots 11.1 / 12.3 / 10.5, in 32896 10.6 / 11.9 /
+// 10.1, 4000 in 32896 14.6 / 14.2 / 14.2; 8000 in 8192 19.5 / 16.5 / 16.8; 32768 in 33024 62 / 48.6 / 48.7. Smaller caches take
+// a chunk per wave throughout: 1000 / 2000 / 4000 keys in 4096 slots 10.5 / 11.5 / 13.8 staged, 10.4 / 11.1 / 12.7. Up to
+// 192 chunks staged instead of 256: 4000 keys of 8192 slots, four tokens, 15.8 against 15.3.
 constexpr int kGFewRows = 16;
 constexpr int kGFewStaged = 256;      // a long cache's chunks x kv heads up to which they are staged
 constexpr int kGFewMaxlen = 1 << 21;  // V^T of a head within a buffer descriptor
@@ -332,15 +334,15 @@ __global__ __launch_bounds__(64 * kGWaves, 2) void general_few_kernel(const int3
   constexpr int CH = general_chunk(D);
   constexpr int KS = D / 32, DT = D / 16, KT = CH / 16, PS = CH / 32;
   constexpr int VPT = DT * PS / KT;  // V^T fragments issued per K tile
-  const int h = blockIdx.y, wave = wave_id();
-  const int p0 = pos0[0];
+  const int wave = wave_id(), p0 = pos0[0];
   const int nch = min((p0 + M + CH - 1) / CH, nchunk_max), sh = nch > 2 * n ? 2 : nch > n ? 1 : 0;
   if (kStage && nch * Hkv <= kGFewStaged) {
-    if ((int)blockIdx.x < nch)
-      general_chunk_body<D>((int)blockIdx.x, h, pos0, q, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
+    const auto [h, c] = work_index(blockIdx.y * n + blockIdx.x, max(1, nch));
+    if (h < Hkv)
+      general_chunk_body<D>(c, h, pos0, q, M, Hq, Hkv, kc, vt, maxlen, scale, tree, part_o, part_ml, nchunk_max);
     return;
   }
-  const int c = ((int)blockIdx.x << sh) + wave;
+  const int h = blockIdx.y, c = ((int)blockIdx.x << sh) + wave;
   if ((wave >> sh) || c >= nch) return;
   const int key0 = c * CH;
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;

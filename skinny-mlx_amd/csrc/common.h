@@ -38,6 +38,24 @@ __device__ __forceinline__ f32x4_t mfma16x16x32(bf16x8_t a, bf16x8_t b, f32x4_t 
 // it can live in SGPRs, e.g. buffer-load soffsets, which otherwise become per-load waterfall loops.
 __device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
 
+// i / n and i % n of workgroup numbers (0 <= i < 2^23, n >= 1) in scalars, by the reciprocal: a third of the integer
+// division's chain, in a kernel's first instructions.
+struct WorkIndex {
+  int quot, rem;
+};
+__device__ __forceinline__ WorkIndex work_index(int i, int n) {
+  int q = __builtin_amdgcn_readfirstlane((int)((float)i * __builtin_amdgcn_rcpf((float)n)));  // off by one at most
+  int r = i - q * n;
+  if (r < 0) {
+    --q;
+    r += n;
+  } else if (r >= n) {
+    ++q;
+    r -= n;
+  }
+  return {q, r};
+}
+
 // LDS writes of this wave complete, then every wave of the workgroup meets. Global loads still in
 // flight are not waited for (unlike __syncthreads()).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

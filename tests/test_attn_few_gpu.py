@@ -12,9 +12,11 @@ from skinny_mlx.tree import DraftTree
 pytestmark = pytest.mark.gpu
 
 # (kv heads, cache slots, cached tokens): the dense layout staged; chunks x heads <= 512, <= 1024, past it; long caches
-# filled so far that a workgroup takes one chunk (general layouts: staged up to 256 chunks in all), two and four
+# filled so far that a workgroup takes one chunk (general layouts: staged up to 256 chunks in all), two and four;
+# workgroups dealt to the heads: the last chunk's edge, an odd count of heads, a full cache
 CASES = [(2, 1024, 100), (2, 2048, 0), (2, 2048, 100), (2, 2048, 250), (8, 8192, 5000), (8, 12288, 12200), (8, 33024, 32765),
-         (8, 33024, 60), (8, 33024, 2040), (8, 33024, 4090), (8, 33024, 8250), (8, 33024, 16700), (2, 33024, 8180)]
+         (8, 33024, 60), (8, 33024, 2040), (8, 33024, 4090), (8, 33024, 8250), (8, 33024, 16700), (2, 33024, 8180),
+         (3, 4096, 4070), (8, 4096, 3960), (1, 33024, 8300), (3, 33024, 32990)]
 
 
 def _call(layout, rnd, dev, hkv, maxlen):
