@@ -288,7 +288,8 @@ def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = N
     L = _lib.lib()
     stream = _lib.stream_of(x2)
     splits, tile = _plain_config(k, n)
-    if m >= rows_from(n, splits) and x2.stride(0) <= _ROWS_MAX_LD and not CONFIG_OVERRIDE and not SPLITK_OVERRIDE:
+    if (m > MAX_M and m >= rows_from(n, splits, _groups(tile)) and x2.stride(0) <= _ROWS_MAX_LD and not CONFIG_OVERRIDE
+            and not SPLITK_OVERRIDE):
         _rows(x2, w, y, splits, tile, EPI_PLAIN, "skinny_qmm")
         return _like_rows(y, x, n)
     if splits > 1:
@@ -308,34 +309,44 @@ def skinny_qmm(x: torch.Tensor, w: torch.Tensor, scales: torch.Tensor | None = N
 # The many-row kernel (skinny_qmm_w4g64_rows_bf16): epilogues, and the rows one launch takes.
 EPI_PLAIN, EPI_GLU_SPLIT, EPI_SWIGLU = 0, 1, 2
 _ROWS_MAX = 16384
-_ROWS_WIDE_N = 8192
+_ROWS_WIDE_N, _ROWS_WIDE_FEW = 8192, 16384
+_ROWS_PARTS = 4         # groups that one launch can walk side by side
 _ROWS_MAX_N = 1 << 20   # one launch's grid
 _ROWS_MAX_LD = 1 << 24  # 48 rows of x in one buffer descriptor
 
 
-def rows_from(n: int, splits: int) -> int:
-    """Rows from which one launch of the many-row kernel replaces the 16-row pieces (same bits).
-    Measured on MI355X in us, pieces against one launch: a weight of many row tiles from two pieces
-    on (2560 x 19456 gate|up, 20 rows: 24 / 15), others from three (4096 x 2560, 33 rows: 18 / 16; 32
-    rows: 12 / 15), a split-K shape, whose pieces spread K over the whole GPU, from five (9728 x
-    2560, 64 rows: 33 / 34; 77 rows: 41 / 36)."""
+def rows_from(n: int, splits: int, groups: int) -> int:
+    """Rows from which one launch of the many-row kernel replaces the 16-row pieces (same bits); `groups` = the
+    tile's cut of a split. Measured on MI355X with weights out of the caches, in us, pieces / one launch:
+    * a split-K shape, whose pieces spread K over the whole GPU, from five pieces on (9728 x 2560, 64 rows: 31.4 / 31.3;
+      65: 36.9 / 31.1; 48: 23.6 / 31.2);
+    * a weight of so many row tiles that two pieces' launches leave a last round of workgroups nearly empty, from two:
+      K = 2560, N = 8224, 17 rows: 13.6 / 11.6; 12352: 13.4 / 11.8; gate|up of 19456, 20 rows: 19.6 / 13.5; but 8192 (one
+      workgroup per CU) 10.2 / 11.6. Cut in two or three groups, which the one launch walks in one part, only past 16384:
+      10240, 17 rows: 16.8 / 17.5; 16384: 16.9 / 18.0; 20480: 19.9 / 18.3;
+    * others from three (4096 x 2560, 33 rows: 15.4 / 14.8; 32 rows: 12.0 / 15.0; 2560 x 6144, 33: 14.5 / 11.4; 32: 10.7 /
+      11.5)."""
     if n > _ROWS_MAX_N:
         return 1 << 62
     if splits > 1:
         return 4 * MAX_M + 1
-    return MAX_M + 1 if n >= _ROWS_WIDE_N else 2 * MAX_M + 1
+    return MAX_M + 1 if n > (_ROWS_WIDE_FEW if 2 <= groups < _ROWS_PARTS else _ROWS_WIDE_N) else 2 * MAX_M + 1
+
+
+def _groups(tile) -> int:
+    """Groups that a 16-row tile cuts a split of K into."""
+    return tile.waves if tile.kind == _WAVE_X else 1
 
 
 def _rows(x2: torch.Tensor, w: torch.Tensor, y: torch.Tensor, splits: int, tile, epilogue: int, what: str) -> None:
     """The many-row kernel over the rows of x2 with the cut of K of (splits, tile): bitwise the
     16-row pieces."""
     m, k = x2.shape
-    groups = tile.waves if tile.kind == _WAVE_X else 1
     L = _lib.lib()
     stream = _lib.stream_of(x2)
     for m0 in range(0, m, _ROWS_MAX):
         _lib.check(L.skinny_qmm_w4g64_rows_bf16(_row_ptr(x2, m0), min(_ROWS_MAX, m - m0), k, x2.stride(0), w.data_ptr(),
-                                                w.shape[0], _row_ptr(y, m0), y.stride(0), splits, groups, epilogue,
+                                                w.shape[0], _row_ptr(y, m0), y.stride(0), splits, _groups(tile), epilogue,
                                                 stream), what)
 
 
@@ -743,7 +754,7 @@ def skinny_glu(x: torch.Tensor, w: torch.Tensor, swiglu: bool, out: torch.Tensor
             raise ValueError(f"out must be bf16 [M, {width}] with unit inner stride")
         y = out
     tile = glu_tile(k, f)
-    if m >= rows_from(2 * f, 1) and x2.stride(0) <= _ROWS_MAX_LD:
+    if m > MAX_M and m >= rows_from(2 * f, 1, _groups(tile)) and x2.stride(0) <= _ROWS_MAX_LD:
         _rows(x2, w, y, 1, tile, EPI_SWIGLU if swiglu else EPI_GLU_SPLIT, "skinny_glu")
         return _like_rows(y, x, width)
     L = _lib.lib()

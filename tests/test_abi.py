@@ -348,6 +348,17 @@ def test_fused_mlp_entry_point_validates_on_host():
     _expect_einval(call(sync_bytes=need - 4), "sync of")
 
 
+@pytest.mark.parametrize("k,n,rows", [(2560, 8192, 33), (2560, 8224, 17), (2560, 10240, 33), (2560, 12352, 17), (2560, 16384, 33),
+                                      (2560, 32768, 17), (2560, 151936, 17), (4096, 2560, 33), (9728, 2560, 65)])
+def test_rows_of_one_launch_by_shape(k, n, rows):
+    """Where one many-row launch takes over from the 16-row pieces: not at two pieces for weights whose pieces fill
+    the CUs once (8192 rows) or that the launch would walk in one part (10240 and 16384 rows: two groups)."""
+    from skinny_mlx import qmm as Q
+
+    splits, tile = Q._plain_config(k, n)
+    assert Q.rows_from(n, splits, Q._groups(tile)) == rows
+
+
 def test_qmm_rows_argument_validation_on_host():
     L = _lib.lib()
     d = ctypes.c_void_p(4096)
