@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define SKINNY_ABI_VERSION 20
+#define SKINNY_ABI_VERSION 21
 
 /* Error codes. */
 #define SKINNY_OK 0
@@ -237,6 +237,8 @@ int skinny_qmm_w4g64_conv_normin_bf16(const skinny_norm_in* ni, int M, int K, co
 int skinny_qmm_w4g64_conv_bf16(const uint16_t* x, int M, int K, int ldx, const uint32_t* w_frag, int N, uint16_t* y,
                                int ldy, int C, uint16_t* conv_state, const uint16_t* conv_w, int KW, uint16_t* window,
                                const int32_t* parent, const skinny_qmm_tile* tile, void* stream);
+/* The tile that entry point takes by default for (K, N). */
+int skinny_qmm_conv_pick_tile(int K, int N, skinny_qmm_tile* tile);
 /* ---------------------------------------------------------------------------
  * Decoder glue of the verify forward (the mlx_lm model the reference patches and runs at
  * skinny_mlx/spec.py:24-29). bf16 in/out, fp32 arithmetic; every op is per row, so results

@@ -1660,6 +1660,11 @@ static int conv_default_tile(int K, int N, skinny_qmm_tile* out) {
   return SKINNY_OK;
 }
 
+extern "C" int skinny_qmm_conv_pick_tile(int K, int N, skinny_qmm_tile* tile) {
+  SKINNY_CHECK_ARG(tile && K > 0 && K % 128 == 0 && N > 0 && N % 16 == 0, "conv_pick_tile: bad arguments K=%d N=%d", K, N);
+  return conv_default_tile(K, N, tile);
+}
+
 extern "C" int skinny_qmm_w4g64_conv_bf16(const uint16_t* x, int M, int K, int ldx, const uint32_t* w_frag, int N,
                                           uint16_t* y, int ldy, int C, uint16_t* conv_state, const uint16_t* conv_w,
                                           int KW, uint16_t* window, const int32_t* parent,

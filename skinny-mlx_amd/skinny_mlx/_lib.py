@@ -22,7 +22,7 @@ LIB_NAME = "libskinny_hip.so"
 # SKINNY_HIP_LIB names another build of the same library (the host-only sanitizer build the CPU
 # tests load); unset, the in-tree build next to this file.
 LIB_PATH = os.environ.get("SKINNY_HIP_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 _c_void_p = ctypes.c_void_p
 _c_int = ctypes.c_int
@@ -73,6 +73,7 @@ SIGNATURES: dict[str, tuple] = {
     "skinny_qmm_w4g64_glu_bf16": (
         _c_int, [_c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _tile_p, _c_void_p]),
     "skinny_qmm_glu_pick_tile": (_c_int, [_c_int, _c_int, _tile_p]),
+    "skinny_qmm_conv_pick_tile": (_c_int, [_c_int, _c_int, _tile_p]),
     "skinny_stream_read": (_c_int, [_c_void_p, _c_size_t, _c_void_p, _c_int, _c_void_p]),
     "skinny_stream_read_chunked": (_c_int, [_c_void_p, _c_size_t, _c_void_p, _c_int, _c_int, _c_void_p]),
     "skinny_rmsnorm_bf16": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_void_p, _c_void_p, _c_int, _c_int,

@@ -462,30 +462,31 @@ def skinny_qmm_partial(x: torch.Tensor, w: torch.Tensor):
     return PartialSum(parts)
 
 
-def _any_rows(x: torch.Tensor, k: int) -> torch.Tensor:
-    """x as 2-D bf16 rows the kernels can read (16-byte aligned rows of K = k)."""
-    if x.shape[-1] != k:
-        raise ValueError(f"x has K={x.shape[-1]}, weights have K={k}")
-    x2 = x.reshape(-1, k)
-    if x2.dtype != torch.bfloat16:
-        x2 = x2.to(torch.bfloat16)
-    return x2 if x2.stride(-1) == 1 and x2.stride(0) % 8 == 0 and x2.data_ptr() % 16 == 0 else x2.contiguous()
+_CONV_TILES: dict[tuple[int, int], object] = {}
 
 
-def skinny_qmm_rows(x: torch.Tensor, w: torch.Tensor, form: str = "plain") -> torch.Tensor:
+def conv_tile(k: int, n: int):
+    """Tile skinny_qmm_conv takes for (K, N); cached."""
+    t = _CONV_TILES.get((k, n))
+    if t is None:
+        t = _lib.QmmTile()
+        _lib.check(_lib.lib().skinny_qmm_conv_pick_tile(k, n, ctypes.byref(t)), "skinny_qmm_conv_pick_tile")
+        _CONV_TILES[(k, n)] = t
+    return t
+
+
+def skinny_qmm_rows(x: torch.Tensor, w: torch.Tensor, form: str) -> torch.Tensor:
     """x [M, K] against packed weights for a prompt's rows (any M), in one launch of the many-row kernel
-    with the cut of K, and so the bits, of what 1..16 rows take: form "plain" skinny_qmm's, "partial"
-    the sum of skinny_qmm_partial's slices, "conv" skinny_qmm_conv's product before its conv."""
+    with the cut of K, and so the bits, of what 1..16 rows take: form "partial" the sum of skinny_qmm_partial's
+    slices, "conv" skinny_qmm_conv's product before its conv."""
+    if form not in ("partial", "conv"):
+        raise ValueError(f"unknown form {form!r}")
     k = packed_k(w)
     n = w.shape[0]
-    x2 = _any_rows(x, k)
-    splits, tile = partial_config(k, n) if form == "partial" else _plain_config(k, n)
-    if form == "conv":  # the conv epilogue's tile: a wave-X one of at most 8 waves (conv_default_tile)
-        splits, tile = 1, _table_tile(k, n)
-        waves = min(tile.waves, 8) if tile.kind == _WAVE_X else 8
-        while waves > 1 and waves > k // 128:
-            waves >>= 1
-        tile = _lib.QmmTile(_WAVE_X, tile.rf, waves, 2)
+    if x.shape[-1] != k:
+        raise ValueError(f"x has K={x.shape[-1]}, weights have K={k}")
+    x2 = _rows_of(x, k)
+    splits, tile = partial_config(k, n) if form == "partial" else (1, conv_tile(k, n))
     y = torch.empty((x2.shape[0], n), dtype=torch.bfloat16, device=x2.device)
     _rows(x2, w, y, splits, tile, EPI_PLAIN, "skinny_qmm_rows")
     return y

@@ -154,6 +154,18 @@ def test_host_queries_over_many_shapes():
     assert rc == -1 and len(L.skinny_last_error()) < 512
 
 
+def test_conv_tile_query_on_host():
+    """The tile of the conv epilogue: wave-X, at most 8 waves, no more than K has pairs of 128."""
+    L = _lib.lib()
+    t = _lib.QmmTile()
+    for k, n in ((128, 16), (256, 48), (512, 768), (2560, 8224), (2560, 12352), (2560, 151936)):
+        assert L.skinny_qmm_conv_pick_tile(k, n, ctypes.byref(t)) == 0
+        assert t.kind == 1 and 1 <= t.waves <= min(8, k // 128), (k, n, t.as_tuple())
+    for k, n in ((0, 16), (64, 16), (128, 8), (-128, 16)):
+        _expect_einval(L.skinny_qmm_conv_pick_tile(k, n, ctypes.byref(t)), "conv_pick_tile")
+    _expect_einval(L.skinny_qmm_conv_pick_tile(2560, 8224, None), "conv_pick_tile")
+
+
 def test_check_maps_codes_to_exceptions():
     with pytest.raises(ValueError):
         _lib.check(_lib.lib().skinny_w4g64_pack(None, None, None, None, 16, 128, None), "x")

@@ -6,6 +6,7 @@ pieces themselves are held to the oracle in test_qmm_gpu.py."""
 import pytest
 import torch
 
+from skinny_mlx import kernels as K
 from skinny_mlx import qmm as Q
 
 pytestmark = pytest.mark.gpu
@@ -79,3 +80,36 @@ def test_rows_strided_and_unaligned_output(dev):
         assert Q.skinny_qmm(x, w, out=out).data_ptr() == out.data_ptr()
         assert _same(out, ref)
         assert (buf[:, :off] == 7).all() and (buf[:, off + n:] == 7).all()
+
+
+@pytest.mark.parametrize("m,k,n", [(17, 256, 48), (100, 4096, 2560), (77, 9728, 2560), (65, 9216, 2560), (40, 2048, 2560)])
+def test_rows_of_a_residual_equal_the_summed_slices(dev, m, k, n):
+    w, g = _weights(n, k, m + k, dev)
+    x = torch.randn((m, k), generator=g, device=dev).to(torch.bfloat16)
+    ref = []
+    for i in range(0, m, 16):
+        parts = Q.skinny_qmm_partial(x[i:i + 16], w).parts
+        total = parts[0]
+        for p in parts[1:]:
+            total = total + p
+        ref.append(total.to(torch.bfloat16))
+    assert _same(Q.skinny_qmm_rows(x, w, "partial"), torch.cat(ref))
+
+
+@pytest.mark.parametrize("m,k,n,c", [(17, 256, 48, 16), (33, 512, 256, 64), (50, 2560, 8224, 6144), (33, 2560, 12352, 8192)])
+def test_rows_before_the_conv_equal_its_product(dev, m, k, n, c):
+    """The columns past the conv's are skinny_qmm_conv's own; its first c are the conv of ours."""
+    w, g = _weights(n, k, m + n, dev)
+    x = torch.randn((m, k), generator=g, device=dev).to(torch.bfloat16)
+    cw = torch.randn((c, 4), generator=g, device=dev).to(torch.bfloat16)
+    s1, s2 = (torch.zeros((3, c), dtype=torch.bfloat16, device=dev) for _ in range(2))
+    ref = torch.cat([Q.skinny_qmm_conv(x[i:i + 16], w, c, s1, cw) for i in range(0, m, 16)])
+    y = Q.skinny_qmm_rows(x, w, "conv")
+    assert _same(y[:, c:], ref[:, c:])
+    assert _same(K.gdn_conv_silu(y[:, :c], s2, cw, None), ref[:, :c]) and _same(s1, s2)
+
+
+def test_rows_take_no_other_form(dev):
+    w, _ = _weights(48, 256, 1, dev)
+    with pytest.raises(ValueError, match="form"):
+        Q.skinny_qmm_rows(torch.zeros((20, 256), dtype=torch.bfloat16, device=dev), w, "plain")
