@@ -1,7 +1,7 @@
 """Prompts through the many-row kernels (Model._prompt) are bitwise the 16-token passes they replace:
 hidden states, logits, keys, values and Gated-DeltaNet states, at lengths that end inside a 16-token piece, a
-64-token group and a 128-key chunk, from an empty cache and after cached tokens; and the prompt kernels
-alone, with workspaces that take several launches."""
+64-token group and a 128-key chunk, from an empty cache and after cached tokens, on the small decoders and on
+layers of the real sizes; and the prompt kernels alone, with workspaces that take several launches."""
 
 import gc
 
@@ -55,6 +55,33 @@ def test_prompt_equals_pieces(preset, t, before):
     # both caches go on alike
     assert c1.attention_offset() == c2.attention_offset() == before + t
     assert torch.equal(forward(model, [7], c1)[1], forward(model, [7], c2)[1])
+
+
+@pytest.mark.parametrize("t", [64, 70, 79])
+@pytest.mark.parametrize("preset", list(SMALL))
+def test_a_block_of_four_pieces_equals_them(preset, t):
+    """The lengths that Model.hidden leaves to the pieces, as one block."""
+    model = _model(preset)
+    ids = model._ids(torch.randint(0, model.args.vocab_size, (t,), generator=torch.Generator().manual_seed(t)).tolist())
+    c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
+    assert torch.equal(model._prompt(ids, c1), model._pieces(ids, c2))
+    for a, b in zip(_state(c1, t), _state(c2, t)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("t", [1024 + 9, 1024 + 40])
+@pytest.mark.parametrize("preset", ["dense-36", "hybrid-36", "qwen35-4b"])
+def test_a_whole_block_of_the_decoders_layers_equals_pieces(preset, t):
+    """Four layers of the decoders at their own sizes (so with the tiles of their projections and the MLP's one-launch
+    form), past the end of a 1024-token block: a tail run as a step, and a second block."""
+    model = build_model(preset, num_hidden_layers=4, vocab_size=1024)
+    P.patch_model(model)
+    ids = model._ids(torch.randint(0, 1024, (t,), generator=torch.Generator().manual_seed(t)).tolist())
+    assert model._prompt_ok(ids)
+    c1, c2 = make_prompt_cache(model), make_prompt_cache(model)
+    assert torch.equal(model.hidden(ids, c1), model._pieces(ids, c2))
+    for a, b in zip(_state(c1, t), _state(c2, t)):
+        assert torch.equal(a, b)
 
 
 def test_prompt_blocks_and_short_tail(monkeypatch):
