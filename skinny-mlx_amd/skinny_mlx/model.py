@@ -163,6 +163,15 @@ def prompt_residual(proj, x: torch.Tensor) -> torch.Tensor:
     return summed(x) if summed is not None else proj(x)
 
 
+def drop_rows(members) -> None:
+    """Let fused projections drop the last input and result that they keep for their other members: 17 MB a layer
+    for 1024 tokens of q, k and v."""
+    for m in members:
+        proj = getattr(m, "projection", None)
+        if proj is not None:
+            proj.forget()
+
+
 def norm_input(h: torch.Tensor, residual, weight: torch.Tensor, eps: float, spare: torch.Tensor):
     """The input rmsnorm(h + residual) * weight of the next projections, and the tensor that holds
     the residual stream h + residual once they have run. A split-K residual (kernels.PartialSum)
@@ -265,9 +274,7 @@ class Attention(nn.Module):
         a, sh = self.a, self._shared(cache)
         Hq, Hkv, D = a.num_attention_heads, a.num_key_value_heads, a.head_dim
         qkv = joined([self.q_proj(x), self.k_proj(x), self.v_proj(x)])
-        proj = getattr(self.q_proj, "projection", None)
-        if proj is not None:
-            proj.forget()  # a fused projection keeps its last rows and result: 17 MB a layer of 1024 tokens
+        drop_rows((self.q_proj, self.k_proj, self.v_proj))
         if a.general_attention:
             qs = 2 * D if a.attn_output_gate else D
             o = K.attention_general_prompt(qkv, Hq, Hkv, D, qs, Hq * qs, Hq * qs + Hkv * D,
@@ -367,6 +374,8 @@ class GatedDeltaNet(nn.Module):
                 and self.in_proj_qkv.columns == slice(0, self.conv_dim)):
             y = proj.conv_product(x)
         qkv, z, b, ag = (y[:, m.columns] for m in members) if y is not None else (m(x) for m in members)
+        if y is None:
+            drop_rows(members)
         if b.stride(0) != ag.stride(0):
             b, ag = b.contiguous(), ag.contiguous()
         xc = K.gdn_conv_silu(qkv, cache.conv_state, self.conv1d_weight, None)

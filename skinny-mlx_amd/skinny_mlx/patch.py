@@ -175,7 +175,7 @@ class _Projection:
         return self._out
 
     def forget(self) -> None:
-        """Drop the cached result (Attention.prompt: rows by the hundred, which no other member asks for again)."""
+        """Drop the cached input and result (a prompt's: rows by the hundred, which no member asks for again)."""
         self._key = self._out = None
 
     def conv_output(self, x, c: int, conv_state: torch.Tensor, conv_w: torch.Tensor, window=None, parent=None):

@@ -212,11 +212,14 @@ def test_pieces_outside_the_skinny_range_keep_their_route(t, block, monkeypatch)
     assert torch.equal(h, torch.cat([model.hidden(ids[i:i + 16], c2) for i in range(0, t, 16)]))
 
 
-@pytest.mark.parametrize("preset", list(SMALL))
-def test_a_prompt_leaves_nothing_behind(preset):
+@pytest.mark.parametrize("preset,fuse_conv", [(p, True) for p in SMALL] + [("tiny-hybrid", False)])
+def test_a_prompt_leaves_nothing_behind(preset, fuse_conv):
     """What is allocated after a prompt is what was before it (a fused projection's cached result would be 500 rows
     of q, k and v a layer)."""
     model = _model(preset)
+    for layer in model.layers:
+        if layer.is_linear:
+            layer.linear_attn.fuse_conv = fuse_conv
     cache = make_prompt_cache(model)
     model.hidden(list(range(20)), cache)
     gc.collect()
