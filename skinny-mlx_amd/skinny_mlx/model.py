@@ -31,10 +31,10 @@ from .qmm import GROUP, random_w4g64
 
 MAX_STEP = 16  # tokens per step (longer inputs: pieces of this size, or Model._prompt)
 # Inputs of more than MAX_STEP tokens run through the many-row kernels in blocks of up to PROMPT_BLOCK
-# tokens (Model._prompt), except from PIECES_MIN to PROMPT_MIN tokens: those leave a captured 16-token pass on
-# the cache (Model._pieces), which callers may hold and replay. Measured on the 36-layer dense decoder in ms,
-# pieces / one block: 17 tokens 6.2 / 3.7, 33: 9.8 / 4.2, 48: 10.2 / 4.3, 79 (with the capture): 13.1 / 4.5; hybrid
-# and qwen35-4b alike.
+# tokens (Model._prompt), except from PIECES_MIN to PROMPT_MIN tokens: those keep the captured 16-token pass that an input
+# of four pieces has always left on the cache (Model._pieces), though one block would be faster. Measured on the
+# 36-layer dense decoder in ms, pieces / one block: 17 tokens 6.2 / 3.7, 33: 9.8 / 4.2, 48: 10.2 / 4.3, 79 (with the
+# capture): 13.1 / 4.5; hybrid and qwen35-4b alike.
 PIECES_MIN = 4 * MAX_STEP
 PROMPT_MIN = 80
 PROMPT_BLOCK = 1024
