@@ -93,7 +93,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_chunk_kernel(const int32_t* 
 // a long context is the read of K and V^T; at a short one the chain position, chunk, partial, merge.
 // Measured on MI355X, one token, chunk stage and merge of a layer, staged against this: 32768 keys 41.5 / 36.4 us
 // (3.69 TB/s of KV; with it, partials of the live rows only and eight merge waves); 8000 keys of 8192 slots 14.0 / 13.1; 1000
-// of 8192 10.7 / 9.2; 4000 of 32896 13.6 / 10.4; 4000 of 4096 10.9 / 10.1; 2000 of 2048 9.3 / 9.2; 60 in 2048 or 4096 8.9 / 8.9
+// of 8192 10.6 / 9.0; 4000 of 32896 13.6 / 10.4; 4000 of 4096 10.9 / 10.2; 2000 of 2048 9.4 / 9.3; 60 in 2048 or 4096 8.7 / 8.7
 // and 9.2 / 9.0. Caches of 256 / 512 / 1280 slots were 1% slower so: up to kFewChunks chunks stay staged. With more rows per
 // kv head several waves of a staged chunk have work, and staging serves them all.
 constexpr int kFewRows = 16;
@@ -174,7 +174,7 @@ __device__ __forceinline__ void attn_direct_chunk(int c, int h, int p0, const ui
     for (int ks = 0; ks < 4; ++ks) o[dt] = mfma16x16x32(__builtin_bit_cast(bf16x8_t, pa[ks]), vf[dt][ks], o[dt]);
   }
   const size_t base = ((size_t)h * nchunk_max + c) * kRowsMax;
-  attn_store_rows<true>(o, mx, sum, rows, part_o + base * kD, part_ml + base * 2);
+  attn_store_rows(o, mx, sum, rows, part_o + base * kD, part_ml + base * 2);
 }
 
 __global__ __launch_bounds__(64 * kWaves) void attn_few_kernel(const int32_t* __restrict__ pos0,
@@ -499,7 +499,7 @@ __global__ __launch_bounds__(64 * kWaves) void prompt_chunk_kernel(const int32_t
     if (key0 >= p0 + t0 + mb || wave * 16 >= G * mb) continue;
     const int tbase = qrow < G * mb ? p0 + t0 + qrow / G + 1 : key0;
     const size_t base = (((size_t)(z - z0) * Hkv + h) * nch + c) * kRowsMax + wave * 16;
-    attn_rows(ks_lds, vs_lds, qf[i], key0, tbase, 0u, scale, part_o + base * kD, part_ml + base * 2);
+    attn_rows(ks_lds, vs_lds, qf[i], key0, tbase, 0u, scale, G * mb - wave * 16, part_o + base * kD, part_ml + base * 2);
   }
 }
 

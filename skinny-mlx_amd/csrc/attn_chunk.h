@@ -146,21 +146,20 @@ __device__ __forceinline__ void attn_softmax(float (&s)[8][4], int key0, int tba
   row_sum = sum;
 }
 
-// The chunk partial of the wave's rows: O rows 4quad + i, dim 16dt + col, to rows_o [16][128]; the row maxima and
-// sums to rows_ml [16][2]. kLive: only the first `rows` rows, all that the merge reads (a wave alone with its chunk saves
-// the stores; behind a staged chunk the row tests cost more than they save: 256-dim heads, 16 tokens over 2000 keys,
-// 17.05 us a layer without, 17.43 with them).
-template <bool kLive>
+// The chunk partial of the wave's first `rows` rows (the merge reads no others): O rows 4quad + i, dim 16dt + col, to
+// rows_o [16][128]; the row maxima and sums to rows_ml [16][2]. The rows past the last are dropped by the store's range
+// check: a lane test per row splits the block that the P.V reads are scheduled in, and storing all 16 rows is traffic that a
+// long context feels. 256-dim heads, us a layer, row tests / all rows / so: 16 tokens over 2000 keys 17.3 / 17.2 / 17.0, 60
+// keys 11.6 / 11.45 / 11.1, 5 tokens over 32700 keys 50.4 / 53.3 / 49.5.
 __device__ __forceinline__ void attn_store_rows(const f32x4_t (&o)[8], float row_max, float row_sum, int rows,
                                                 float* __restrict__ rows_o, float* __restrict__ rows_ml) {
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(rows_o, (short)0, min(rows, 16) * kD * 4, 0x00020000);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (kLive && quad * 4 + i >= rows) break;
-    float* dst = rows_o + (quad * 4 + i) * kD;
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int dt = 0; dt < 8; ++dt) dst[dt * 16 + col] = o[dt][i];
-  }
+    for (int dt = 0; dt < 8; ++dt)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[dt][i]), ro, ((quad * 4 + i) * kD + dt * 16 + col) * 4, 0, 0);
   if (quad == 0) {
     rows_ml[col * 2] = row_max;
     rows_ml[col * 2 + 1] = row_sum;
@@ -169,7 +168,7 @@ __device__ __forceinline__ void attn_store_rows(const f32x4_t (&o)[8], float row
 
 // One wave's 16 query rows against the staged chunk (keys key0 ..), visibility as attn_softmax has it.
 __device__ __forceinline__ void attn_rows(const uint16_t* ks_lds, const uint16_t* vs_lds, const bf16x8_t (&qf)[4], int key0,
-                                          int tbase, uint32_t tmask, float scale, float* __restrict__ rows_o,
+                                          int tbase, uint32_t tmask, float scale, int rows, float* __restrict__ rows_o,
                                           float* __restrict__ rows_ml) {
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
   // 2. S^T tiles: element i of tile kt is the score of key 32(kt/2) + 8quad + 4(kt%2) + i.
@@ -200,7 +199,7 @@ __device__ __forceinline__ void attn_rows(const uint16_t* ks_lds, const uint16_t
       o[dt] = mfma16x16x32(pf, *reinterpret_cast<const bf16x8_t*>(&vs_lds[(dt * 16 + col) * kPitch + ks * 32 + quad * 8]),
                            o[dt]);
   }
-  attn_store_rows<false>(o, mx, sum, 16, rows_o, rows_ml);
+  attn_store_rows(o, mx, sum, rows, rows_o, rows_ml);
 }
 
 // The body of the chunk kernel for workgroup (chunk c, kv head h), shared by attn_chunk_kernel and
@@ -434,7 +433,7 @@ __device__ __forceinline__ void attn_chunk_body(int c, int h, const int32_t* __r
   if (!busy) return;
 
   const size_t base = ((size_t)h * nchunk_max + c) * kRowsMax + wave * 16;
-  attn_rows(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, part_o + base * kD, part_ml + base * 2);
+  attn_rows(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, rows - wave * 16, part_o + base * kD, part_ml + base * 2);
 }
 
 }  // namespace

@@ -159,17 +159,16 @@ __device__ __forceinline__ void general_softmax(float (&s)[general_chunk(D) / 16
   row_sum = sum;
 }
 
-template <int D, bool kLive>
+template <int D>
 __device__ __forceinline__ void general_store_rows(const f32x4_t (&o)[D / 16], float row_max, float row_sum, int rows,
                                                    float* __restrict__ rows_o, float* __restrict__ rows_ml) {
   const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(rows_o, (short)0, min(rows, 16) * D * 4, 0x00020000);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (kLive && quad * 4 + i >= rows) break;
-    float* dst = rows_o + (quad * 4 + i) * D;
+  for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) dst[dt * 16 + col] = o[dt][i];
-  }
+    for (int dt = 0; dt < D / 16; ++dt)
+      __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(o[dt][i]), ro, ((quad * 4 + i) * D + dt * 16 + col) * 4, 0, 0);
   if (quad == 0) {
     rows_ml[col * 2] = row_max;
     rows_ml[col * 2 + 1] = row_sum;
@@ -180,7 +179,7 @@ __device__ __forceinline__ void general_store_rows(const f32x4_t (&o)[D / 16], f
 // the partial O rows to rows_o [16][D], the row maxima (log2 units) and sums to rows_ml [16][2].
 template <int D>
 __device__ __forceinline__ void general_rows(const uint16_t* ks_lds, const uint16_t* vs_lds, const bf16x8_t (&qf)[D / 32],
-                                             int key0, int tbase, uint32_t tmask, float scale, float* __restrict__ rows_o,
+                                             int key0, int tbase, uint32_t tmask, float scale, int rows, float* __restrict__ rows_o,
                                              float* __restrict__ rows_ml) {
   constexpr int CH = general_chunk(D);
   constexpr int KS = D / 32;   // 32-dim steps of a score
@@ -216,7 +215,7 @@ __device__ __forceinline__ void general_rows(const uint16_t* ks_lds, const uint1
       o[dt] = mfma16x16x32(pf, *reinterpret_cast<const bf16x8_t*>(&vs_lds[(dt * 16 + col) * VP + ks * 32 + quad * 8]),
                            o[dt]);
   }
-  general_store_rows<D, false>(o, mx, sum, 16, rows_o, rows_ml);
+  general_store_rows<D>(o, mx, sum, rows, rows_o, rows_ml);
 }
 
 // (2) Workgroup (chunk c, kv head h), keys [CH c, CH c + CH); wave w takes the query rows
@@ -294,7 +293,7 @@ __device__ __forceinline__ void general_chunk_body(int c, int h, const int32_t* 
   if (!busy) return;
 
   const size_t base = ((size_t)h * nchunk_max + c) * kGRowsMax + wave * 16;
-  general_rows<D>(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, part_o + base * D, part_ml + base * 2);
+  general_rows<D>(ks_lds, vs_lds, qf, key0, tbase, tmask, scale, rows - wave * 16, part_o + base * D, part_ml + base * 2);
 }
 
 template <int D>
@@ -404,7 +403,7 @@ __global__ __launch_bounds__(64 * kGWaves, 2) void general_few_kernel(const int3
     for (int ks = 0; ks < PS; ++ks) o[dt] = mfma16x16x32(__builtin_bit_cast(bf16x8_t, pa[ks]), vf[dt][ks], o[dt]);
   }
   const size_t base = ((size_t)h * nchunk_max + c) * kGRowsMax;
-  general_store_rows<D, true>(o, mx, sum, G * M, part_o + base * D, part_ml + base * 2);
+  general_store_rows<D>(o, mx, sum, G * M, part_o + base * D, part_ml + base * 2);
 }
 
 // (3) One workgroup per (query head, token), max(1, D / 128) waves, lane l of wave w holding dims
@@ -602,7 +601,7 @@ __global__ __launch_bounds__(64 * kGWaves) void general_prompt_chunk_kernel(
       if (!live) qf[ks] = bf16x8_t{};
     }
     const size_t base = (((size_t)(z - z0) * Hkv + h) * nch + c) * kGRowsMax + wave * 16;
-    general_rows<D>(ks_lds, vs_lds, qf, key0, live ? p0 + t0 + qrow / G + 1 : key0, 0u, scale, part_o + base * D,
+    general_rows<D>(ks_lds, vs_lds, qf, key0, live ? p0 + t0 + qrow / G + 1 : key0, 0u, scale, rows - wave * 16, part_o + base * D,
                     part_ml + base * 2);
   }
 }
