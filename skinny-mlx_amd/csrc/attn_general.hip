@@ -314,9 +314,9 @@ __global__ __launch_bounds__(64 * kGWaves) void general_chunk_kernel(const int32
 // long cache (kStage) up to kGFewStaged chunks in all, one per CU, are staged by all waves of a workgroup instead:
 // rows of V^T many KB apart come slowly to one wave. The staged chunks are dealt to the grid's first workgroups, the idle
 // ones last (see attn_few_kernel); a chunk per wave keeps its place, where dealing took 1% more. 256-dim heads, one token, us
-// a layer, every chunk staged / a chunk per wave / as here: 1000 keys in 8192 slots 11.1 / 12.3 / 10.5, in 32896 10.6 / 11.9 /
-// 10.1, 4000 in 32896 14.6 / 14.2 / 14.2; 8000 in 8192 19.5 / 16.5 / 16.8; 32768 in 33024 62 / 48.6 / 48.7. Smaller caches take
-// a chunk per wave throughout: 1000 / 2000 / 4000 keys in 4096 slots 10.5 / 11.5 / 13.8 staged, 10.4 / 11.1 / 12.7. Up to
+// a layer, every chunk staged / a chunk per wave / as here: 1000 keys in 8192 slots 11.2 / 12.3 / 10.2, in 32896 10.6 / 11.9 /
+// 9.9, 4000 in 32896 14.5 / 14.2 / 13.4; 8000 in 8192 19.4 / 16.3 / 16.0; 32700 in 32896 60.3 / 42.0 / 41.8. Smaller caches take
+// a chunk per wave throughout: 1000 / 2000 / 4000 keys in 4096 slots 10.4 / 11.5 / 13.7 staged, 9.9 / 10.9 / 12.4. Up to
 // 192 chunks staged instead of 256: 4000 keys of 8192 slots, four tokens, 15.8 against 15.3.
 constexpr int kGFewRows = 16;
 constexpr int kGFewStaged = 256;      // a long cache's chunks x kv heads up to which they are staged
@@ -423,8 +423,10 @@ constexpr int kGCombineGroups = 4;
 template <int D>
 constexpr int general_combine_waves() { return D > 128 ? D / 128 : 1; }
 
-// (chunk c's partial row at head_base + c * kGRowsMax; pos0[0] + tokens keys; gate_at(): the row's gate
-// values or NULL, and out_at(): its output, asked for last, since their arguments lie past the preloaded ones)
+// (chunk c's partial row at head_base + c * kGRowsMax; pos0[0] + tokens keys; gate_at(): the row's gate values or NULL,
+// and out_at(): its output, asked for after the blocks' loads, since their arguments lie past the preloaded ones, and before
+// the fold, which the gate's load then runs beside: 4 tokens over 5003 keys 16.95 -> 16.4 us a layer; 64-dim heads, one dim
+// a lane, take it after, 1% faster so)
 template <int D, int W, typename GateAt, typename OutAt>
 __device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ pos0, const float* __restrict__ part_o,
                                                     const float* __restrict__ part_ml, size_t head_base, int tokens,
@@ -439,6 +441,9 @@ __device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ 
   const int td = (int)threadIdx.x - v * 64 * DW;                // thread within the group
   const int d0 = td * CW;                                       // this lane's first dim
   const int nch = min((pos0[0] + tokens + CH - 1) / CH, nchunk_max);
+  // No blocks for the other groups: none of them is waited for (16 tokens over 60 keys in 5120 slots 11.85 -> 11.4 us a
+  // layer, with one group in all 11.5).
+  if (W > 1 && v > 0 && nch <= B) return;
   float run_m = -INFINITY, run_l = 0.f, a[CW];
 #pragma unroll
   for (int k = 0; k < CW; ++k) a[k] = 0.f;
@@ -477,13 +482,15 @@ __device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ 
     }
     run_m = new_m;
   }
-  if constexpr (W > 1) {  // group 0 folds the others' sums in their order
-    if (nch <= B) {  // there are none: 16 tokens over 60 keys of 256-dim heads in 5120 slots 11.9 -> 11.65 us a layer
-      if (v > 0) return;
+  const uint16_t* gate = gate_at();
+  uint16_t* dst = out_at() + d0;
+  uint16_t gv[CW] = {};
+  if (D > 64 && gate)
 #pragma unroll
-      for (int k = 0; k < CW; ++k) a[k] += 0.f;  // as adding them would: no zero keeps a sign
-    } else {
-      __shared__ float sm[W], sl[W], sa[W][64 * DW][CW];
+    for (int k = 0; k < CW; ++k) gv[k] = gate[d0 + k];
+  if constexpr (W > 1) {  // group 0 folds the others' sums in their order
+    __shared__ float sm[W], sl[W], sa[W][64 * DW][CW];
+    if (__builtin_expect(nch > B, 1)) {
       if (td == 0) {
         sm[v] = run_m;
         sl[v] = run_l;
@@ -504,15 +511,15 @@ __device__ __forceinline__ void general_combine_row(const int32_t* __restrict__ 
         run_m = new_m;
       }
     }
+#pragma unroll
+    for (int k = 0; k < CW; ++k) a[k] += 0.f;  // as that leaves them: no zero keeps a sign
   }
   const float inv = run_l > 0.f ? 1.0f / run_l : 0.f;
-  const uint16_t* gate = gate_at();
-  uint16_t* dst = out_at() + d0;
 #pragma unroll
   for (int k = 0; k < CW; ++k) {
     const uint16_t ob = f32_to_bf16_bits(a[k] * inv);
     if (gate) {
-      const float g = bf16_bits_to_f32(gate[d0 + k]);
+      const float g = bf16_bits_to_f32(D > 64 ? gv[k] : gate[d0 + k]);
       const float sg = bf16_bits_to_f32(f32_to_bf16_bits(1.0f / (1.0f + expf(-g))));
       dst[k] = f32_to_bf16_bits(bf16_bits_to_f32(ob) * sg);
     } else {
