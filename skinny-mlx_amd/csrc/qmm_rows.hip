@@ -17,10 +17,10 @@
 // against 8 FMAs (32 cycles; the scale and bias terms in fp32, which the bits fix) and the nibble unpacking
 // (17 instructions per 16 weight rows, shared by MT tiles), so everything else has to be hidden: X's LDS reads
 // run half a pair ahead of their MFMAs, X's rows are loaded in whole 128-byte lines, and the loop's loads stand
-// in the same order on every path, as a wait counts the loads issued after the one it is for. With three waves
-// per SIMD for the wide wave, that took 2560x19456 at 501 rows from 81 to 77 us, 9728x2560 at 1024 rows from 106
-// to 95 and at 96 rows from 33 to 25 (VALU active 67% of the CUs' busy time before, 86% after). MT = 4 saves a fifth
-// of the instructions but leaves two waves per SIMD, and was slower everywhere (2560x19456, 501 rows: 95 us).
+// in the same order on every path, as a wait counts the loads issued after the one it is for. So VALU instructions issue in
+// 86% of the CUs' busy cycles (2560x19456 gate|up, 501 rows: 77.4 us). All figures here and at pick_rows: one launch over
+// weights that are in no cache (400 MB of them in turn). MT = 4 saves a fifth of the instructions but leaves two waves per
+// SIMD (the same case 81.5 us with NT = 2; with NT = 4 it spills).
 // MT = 3 serves grids that fit the CUs with blocks of 48 rows and not with 32 (pick_rows).
 #include "qmm_frag.h"
 
@@ -66,9 +66,9 @@ struct RowsArgs {
 //
 // The wide wave (NT = 4) and several parts keep one pair of weights per wave in flight, loaded again as soon
 // as its second half is unpacked: half a pair of time, which the other waves of the SIMD fill; one part of
-// NT = 2 has registers for two (9728x2560, 1024 rows: 97 against 104 us). The wide wave also keeps its group sums in
-// LDS, each lane its own words: in registers they spilled within the loop at three waves per SIMD (2560x19456,
-// 501 rows: 90 against 86 us).
+// NT = 2 has registers for two (9728x2560, 1024 rows: level with one, 94.7 us). The wide wave also keeps its group sums in
+// LDS, each lane its own words: in registers they spill within the loop at three waves per SIMD (2560x19456,
+// 501 rows: 83.5 against 77.4 us).
 template <int MT, int NT, int NACC, int KS, int EPI>
 __global__ __launch_bounds__(256 * KS, NT == 4 ? 3 : 1) void qmm_rows_kernel(const RowsArgs ra) {
   static_assert(EPI == kRowsPlain || NT % 2 == 0, "gate|up epilogues pair two row tiles per wave");
@@ -429,12 +429,12 @@ RowsForm rows_parts48(int S, int G) {
 // busiest CU holds ceil(blocks / CUs) of them, and a wide block (64 weight rows a wave instead of 32) costs
 // 1.72 times a narrow one: it amortises its X reads over twice the weights, and is taken where that count comes
 // out lower (from two wide blocks per CU on: alone on its CU a wide block is slower than two narrow ones).
-// Measured on MI355X in us (K x N, M: one part / parts, chosen width): 4096x2560, 64: 21.7 / 13.3 (16 NT =
-// 16); 256: 22.6 / 18.9 (32). 9728x2560, 96: 50.9 / 25.3 (16); 300: 52.8 / 37.6 (32); 400: 67.6 / 45.2 (48 rows); 509: 65.0 / 45.8 (48
-// rows). 4096x2560, 509: 29.1 / 23.6 (48 rows); 2048x2560, 509: 17.2 / 15.1 (48 rows). 2560x6144, 64:
-// 14.8 / 10.7 (16); 160: 15.2 / 14.0 (32). Wide block against narrow, one part: 2560x19456 gate|up, 96: 26.2 /
-// 22.0; 256: 46.9 / 46.3; 320: 50.3 / 55.8; 501: 83.8 / 96.5; 2560x8224, 509: 46.0 / 44.2; 2560x12352, 256: 33.1 /
-// 36.7; 509: 61.2 / 60.7; 2560x151936, 20: 46.4 / 43.3; 64: 84.9 / 90.5.
+// Measured on MI355X in us (K x N, M: one part / parts, chosen width; see the top): 4096x2560, 64: 22.3 / 14.9 (16 NT =
+// 16); 256: 22.2 / 18.1 (32); 509: 28.9 / 25.5 (48 rows). 9728x2560, 96: 50.1 / 31.1 (16); 300: 50.5 / 38.8 (32); 400: 63.4 /
+// 44.0 (48 rows); 509: 63.8 / 45.9 (48 rows). 2048x2560, 509: 16.7 / 15.5 (48 rows). 2560x6144, 64: 15.2 / 11.5 (16); 77:
+// 15.1 / 13.5 (32); 160: 15.2 / 13.7 (32). Wide block against narrow, one part: 2560x19456 gate|up, 96: 29.4 / 22.3; 256: 47.5 /
+// 46.2; 320: 50.3 / 54.4; 501: 77.7 / 84.8; 1024: 152 / 174; 2560x8224, 509: 44.1 / 42.7; 2560x12352, 256: 34.6 / 36.4; 509:
+// 61.3 / 58.3; 2560x151936, 20: 50.8 / 51.4; 64: 85.2 / 91.0. A wide block of these takes 1.66 to 1.83 times a narrow one.
 template <int EPI>
 RowsForm pick_rows(int M, int N, int S, int G) {
   if constexpr (EPI != kRowsGluSplit) {
