@@ -574,6 +574,7 @@ __global__ __launch_bounds__(64 * kGWaves) void general_prompt_chunk_kernel(
   constexpr int PIECES = CH * D / 8 / (64 * kGWaves);
   __shared__ __attribute__((aligned(16))) uint16_t ks_lds[CH * KP];
   __shared__ __attribute__((aligned(16))) uint16_t vs_lds[D * VP];
+  __shared__ int odd_lds[kGWaves];
   const int c = blockIdx.x, h = blockIdx.y, p0 = pos0[0], G = Hq / Hkv;
   const int lane = threadIdx.x & 63, wave = wave_id();
   const int za = z0 + (int)blockIdx.z * kGPieceGroup, zb = min(za + kGPieceGroup, z1);
@@ -594,11 +595,27 @@ __global__ __launch_bounds__(64 * kGWaves) void general_prompt_chunk_kernel(
     *reinterpret_cast<u32x4_t*>(&ks_lds[(e / (D / 8)) * KP + (e % (D / 8)) * 8]) = kr[i];
     *reinterpret_cast<u32x4_t*>(&vs_lds[(e / (CH / 8)) * VP + (e % (CH / 8)) * 8]) = vr[i];
   }
+  const bool edge = key0 + CH > p0 + min(M, (za + 1) * kGMaxTokens);  // see prompt_chunk_kernel
+  if (edge) odd_lds[wave] = any_not_finite(vr);
   __syncthreads();
+  bool odd = false;
+  if (edge) {
+#pragma unroll
+    for (int w = 0; w < kGWaves; ++w) odd |= __builtin_amdgcn_readfirstlane(odd_lds[w]) != 0;
+  }
+  int seen = CH;
   const int col = lane & 15, quad = lane >> 4, qrow = wave * 16 + col;
-  for (int z = za; z < zb; ++z) {
+  for (int z = zb - 1; z >= za; --z) {
     const int t0 = z * kGMaxTokens, mb = min(kGMaxTokens, M - t0), rows = G * mb;
-    if (key0 >= p0 + t0 + mb || wave * 16 >= rows) continue;
+    const int end = min(p0 + t0 + mb - key0, CH);
+    if (end <= 0) break;
+    if (odd && end < seen) {
+      __syncthreads();
+      for (int e = threadIdx.x; e < D * (seen - end); e += 64 * kGWaves) vs_lds[e % D * VP + end + e / D] = 0;
+      __syncthreads();
+      seen = end;
+    }
+    if (wave * 16 >= rows) continue;
     const bool live = qrow < rows;
     const uint16_t* qr = q + ((size_t)(live ? t0 + qrow / G : 0) * Hq + h * G + (live ? qrow % G : 0)) * D;
     bf16x8_t qf[KS];

@@ -56,6 +56,18 @@ __device__ __forceinline__ WorkIndex work_index(int i, int n) {
   return {q, r};
 }
 
+// Whether a bf16 among the eight of any v[i] is an infinity or a NaN, in any lane of the wave.
+template <int N>
+__device__ __forceinline__ bool any_not_finite(const u32x4_t (&v)[N]) {
+  typedef __attribute__((ext_vector_type(2))) uint16_t u16x2_t;
+  u16x2_t m = {0, 0};
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) m = __builtin_elementwise_max(m, __builtin_bit_cast(u16x2_t, v[i][w] & 0x7fff7fffu));
+  return __any(m.x >= 0x7f80 || m.y >= 0x7f80);
+}
+
 // LDS writes of this wave complete, then every wave of the workgroup meets. Global loads still in
 // flight are not waited for (unlike __syncthreads()).
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }

@@ -275,6 +275,36 @@ def test_prompt_attention_equals_steps(dev, layout, maxlen, past):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("past,token", [(0, 99), (100, 20), (250, 149), (120, 16)])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("layout", ["dense", "general"])
+def test_an_infinite_value_reaches_no_token_before_its_step(dev, layout, bad, past, token):
+    """A token whose values are no numbers: the rows of the pieces before it are what 16-token steps give."""
+    hq, hkv, d, t, maxlen = (8, 2, 128, 150, 512) if layout == "dense" else (4, 1, 256, 150, 512)
+    g = torch.Generator(device=dev).manual_seed(past)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev).to(torch.bfloat16)
+    if layout == "dense":
+        table, ws = K.rope_table(1e6, maxlen, dev), K.attn_workspace(hkv, maxlen, dev)
+        lay, first, step = (), K.attention_prompt, K.attention_fused
+        qkv = rnd(t, (hq + 2 * hkv) * d)
+    else:
+        table, ws = K.rope_table_dim(1e7, 64, maxlen, dev), K.attn_general_workspace(hq, hkv, d, maxlen, dev)
+        lay, first, step = (d, hq * d, (hq + hkv) * d, None), K.attention_general_prompt, K.attention_general
+        qkv = rnd(t, (hq + 2 * hkv) * d)
+    qkv[token, (hq + hkv) * d:] = bad
+    k0, v0 = rnd(hkv, maxlen, d), rnd(hkv, d, maxlen)
+    pos = torch.tensor([past], dtype=torch.int32, device=dev)
+    tail = () if layout == "dense" else (64,)
+    k, vt = k0.clone(), v0.clone()
+    out = first(qkv, hq, hkv, d, *lay, None, None, 1e-6, *tail, table, pos, past + t, k, vt, d ** -0.5)
+    k2, vt2 = k0.clone(), v0.clone()
+    ref = torch.cat([step(qkv[i:i + 16], hq, hkv, d, *lay, None, None, 1e-6, *tail, table, pos + i, k2, vt2, d ** -0.5, ws)
+                     for i in range(0, t, 16)])
+    piece = token // 16 * 16
+    assert ref[:piece].isfinite().all() and torch.equal(out[:piece], ref[:piece])
+    assert torch.equal(out.isnan(), ref.isnan())
+
+
 def test_prompt_attention_in_several_launches(dev):
     """A workspace of one group of pieces (four) instead of all ten: three launches, the same bits."""
     from skinny_mlx import _lib
