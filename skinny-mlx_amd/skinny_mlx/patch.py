@@ -131,8 +131,7 @@ class _Projection:
         for q in linears:
             edges.append(edges[-1] + q.out_features)
         self.columns = [slice(lo, hi) for lo, hi in zip(edges, edges[1:])]
-        self._key = None
-        self._out = None
+        self._last = None  # (input, its version, result)
         self._mlp_buffers = None  # (act, sync) of the fused MLP launch, made on its first call
 
     def mlp_partial(self, x, down):
@@ -170,13 +169,14 @@ class _Projection:
 
     def output(self, x) -> torch.Tensor:
         version = getattr(x, "_version", 0)
-        if self._key is None or self._key[0] is not x or self._key[1] != version:
-            self._key, self._out = (x, version), self._compute(x)
-        return self._out
+        last = self._last  # read once: a prompt on another thread may drop it (forget)
+        if last is None or last[0] is not x or last[1] != version:
+            last = self._last = (x, version, self._compute(x))
+        return last[2]
 
     def forget(self) -> None:
         """Drop the cached input and result (a prompt's: rows by the hundred, which no member asks for again)."""
-        self._key = self._out = None
+        self._last = None
 
     def conv_output(self, x, c: int, conv_state: torch.Tensor, conv_w: torch.Tensor, window=None, parent=None):
         """The output with a Gated-DeltaNet mixer's conv + SiLU applied to its first `c` columns in

@@ -228,6 +228,22 @@ def test_a_prompt_leaves_nothing_behind(preset, fuse_conv):
     assert torch.cuda.memory_allocated() <= before
 
 
+def test_a_dropped_result_is_still_returned():
+    """Another thread's prompt may drop a projection's kept result between its computation and its return."""
+    class Dropping(P._Projection):
+        def __init__(self):
+            self.forget()
+
+        def __setattr__(self, name, value):
+            object.__setattr__(self, name, None)
+
+        def _compute(self, x):
+            return x + 1
+
+    x = torch.ones(4)
+    assert torch.equal(Dropping().output(x), x + 1)
+
+
 @pytest.mark.parametrize("preset,field,value", [("tiny-dense", "rope_theta", 5e5), ("tiny-qwen35", "rope_theta", 5e5),
                                                 ("tiny-qwen35", "rope_dim", 32)])
 def test_a_cache_of_another_rope_is_refused(preset, field, value):
