@@ -421,6 +421,7 @@ __global__ __launch_bounds__(256) void prompt_qkv_kernel(const int32_t* __restri
     const int r = (b - nq) * 4 + wave;
     if (r >= M * Hkv) return;
     const int t = r / Hkv, h = r % Hkv, slot = p0 + t;
+    if (slot >= pa.maxlen) return;  // tokens past the cache are dropped, as the steps drop them
     const uint16_t* src = qkv + (size_t)t * ldq + (size_t)(Hq + h) * kD;
     float ka = bf16_bits_to_f32(src[lane]), kb = bf16_bits_to_f32(src[lane + 64]);
     const float2 cs = reinterpret_cast<const float2*>(pa.rope)[(size_t)slot * 64 + lane];
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(256) void prompt_qkv_kernel(const int32_t* __restri
       for (int k = 0; k < 4; ++k) *reinterpret_cast<uint32_t*>(&vl[t][piece * 8 + 2 * k]) = v[k];
     }
     __syncthreads();
-    if (t0 + lane < M)
+    if (t0 + lane < M && p0 + t0 + lane < pa.maxlen)
       for (int d = wave; d < kD; d += 4) pa.vt[((size_t)h * kD + d) * pa.maxlen + p0 + t0 + lane] = vl[lane][d];
   }
 }

@@ -291,6 +291,26 @@ def test_prompt_attention_equals_steps(dev, layout, maxlen, past):
         assert torch.equal(a, b)
 
 
+def test_prompt_tokens_past_the_cache_are_dropped(dev):
+    """A device position that leaves slots for 20 of 40 tokens (no caller of the package lets it): the others land
+    nowhere, neither in the next head's rows nor behind the last head's. The RoPE table covers the positions."""
+    hq, hkv, d, t, maxlen, guard = 8, 2, 128, 40, 512, 1 << 14
+    past = maxlen - 20
+    g = torch.Generator(device=dev).manual_seed(8)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev).to(torch.bfloat16)
+    qkv, table = rnd(t, (hq + 2 * hkv) * d), K.rope_table(1e6, maxlen + 128, dev)
+    k0, v0 = rnd(hkv * maxlen * d + guard), rnd(hkv * maxlen * d + guard)
+    k, vt = k0.clone(), v0.clone()
+    kc, vc = k[:-guard].view(hkv, maxlen, d), vt[:-guard].view(hkv, d, maxlen)
+    pos = torch.tensor([past], dtype=torch.int32, device=dev)
+    K.attention_prompt(qkv, hq, hkv, d, None, None, 1e-6, table, pos, maxlen, kc, vc, d ** -0.5)
+    assert torch.equal(k[-guard:], k0[-guard:]) and torch.equal(vt[-guard:], v0[-guard:])
+    assert torch.equal(kc[:, :past], k0[:-guard].view(hkv, maxlen, d)[:, :past])
+    want = v0[:-guard].view(hkv, d, maxlen).clone()
+    want[:, :, past:] = qkv[:20, (hq + hkv) * d:].view(20, hkv, d).permute(1, 2, 0)
+    assert torch.equal(vc, want)
+
+
 @pytest.mark.parametrize("past,token", [(0, 99), (100, 20), (250, 149), (120, 16)])
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 @pytest.mark.parametrize("layout", ["dense", "general"])
